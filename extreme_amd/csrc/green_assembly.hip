@@ -12,7 +12,8 @@
 //         [HankelCoefficients.cs:103-118, ScalarMathUtils.cs:189-241, InnerResultsCombiner.cs:19-62]
 //   K4    piecewise-linear segments I(rho) = A rho + B  [ScalarSegments.cs:86-128]
 //   K5    lateral integration of every cell of the positive quadrant by line integrals along
-//         its four edges, written with the mirror parities straight into the device layout
+//         its four edges, written straight into the device layout (a full tensor with its mirror
+//         images; a folded one gets them from the parities in the FFT's loads)
 //         [GreenTensorCalculator.cs:166-552, IntegralFactors.cs:17-30, QSign.cs:64-67,
 //          GreenTensorFftPopulator.cs:37-148]
 //   FFT   forward 2-D pencil FFT of every column  [AtoAGreenTensorCalculatorComponent.cs:197-279]
@@ -27,6 +28,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstdio>
+#include <cstring>
 #include <vector>
 
 namespace xtr {
@@ -341,6 +343,8 @@ __device__ inline Factors factors(double s, double u, double rs, double ru, doub
 
 struct LatArgs {
     int nx, ny, nz, npairs, asym, nr;
+    int p0;                       // first pair of this chunk
+    int folded;                   // G holds blocks [Nx+1][Ny+1], else [2Nx][2Ny]
     double dx, dy;
     const double2 *segA, *segB;   // [seg][comp][pair]
     const double *radii;
@@ -459,15 +463,18 @@ __global__ __launch_bounds__(256) void lateral_kernel(LatArgs a)
             fill(a, G, integrate(a, p, kz, kr, 0, y2, x, true), sign, 1);
         }
     }
-    // write G(i,j) and its mirror images (GreenTensorFftPopulator.cs:88-148)
+    // write G(i,j) and, into a full tensor, its mirror images (GreenTensorFftPopulator.cs:88-148); of a folded
+    // one the FFT forms the images from the parities as it reads
     const int nq = a.asym ? 2 : 4;
-    const int64_t nx2 = 2LL * a.nx, ny2 = 2LL * a.ny;
+    const int64_t nx2 = 2LL * a.nx, ny2 = a.folded ? a.ny + 1 : 2LL * a.ny;
     // asym pairs are rc-major (p = rc*nz + tr); the device block stores them swizzled
-    const int pd = a.asym ? asym_pos(p / a.nz, p % a.nz, a.nz, asym_swizzle_mask(a.nz)) : p;
+    const int pa = a.p0 + p;
+    const int pd = a.asym ? asym_pos(pa / a.nz, pa % a.nz, a.nz, asym_swizzle_mask(a.nz)) : pa;
     for (int t = 0; t < nq; ++t) {
         const int64_t o = a.off[t] + pd;
         const double2 g = G.q[t];
         a.G[((int64_t)i * ny2 + j) * a.gblk + o] = g;
+        if (a.folded) continue;
         if (i >= 1) a.G[((nx2 - i) * ny2 + j) * a.gblk + o] = (double)a.xs[t] * g;
         if (j >= 1) a.G[((int64_t)i * ny2 + (ny2 - j)) * a.gblk + o] = (double)a.ys[t] * g;
         if (i >= 1 && j >= 1) a.G[((nx2 - i) * ny2 + (ny2 - j)) * a.gblk + o] = (double)(a.xs[t] * a.ys[t]) * g;
@@ -587,31 +594,78 @@ HostPlan make_level_plan(const GreenInput &in, double sx, double sy)
     return make_plan(in.number_of_hankels, rmin, rmax, zero);
 }
 
-template <typename T>
-struct Dev {
-    T *p = nullptr;
-    explicit Dev(size_t n) { XTR_CHECK(hipMalloc((void **)&p, std::max<size_t>(n, 1) * sizeof(T))); }
-    Dev(const std::vector<T> &h) : Dev(h.size())
+// Host arrays that one copy takes to the device: add() returns where an array lies in it.
+struct Pack {
+    std::vector<unsigned char> bytes;
+    template <typename T> size_t add(const std::vector<T> &v)
     {
-        XTR_CHECK(hipMemcpy(p, h.data(), h.size() * sizeof(T), hipMemcpyHostToDevice));
+        const size_t at = bytes.size();
+        bytes.resize(at + GreenScratch::padded(v.size() * sizeof(T)));
+        std::memcpy(bytes.data() + at, v.data(), v.size() * sizeof(T));
+        return at;
     }
-    ~Dev() { (void)hipFree(p); }
-    Dev(const Dev &) = delete;
 };
 
-int layer_at_depth(const Section &s, double depth)   // ScalarMathUtils.cs:15-31
-{
-    const int k = layer_index_at_depth(s, depth);
-    if (k < 0) throw hip_error("anomaly is not within 1D section");
-    return k;
-}
+// The scalar plan and the filter on the device, and the layer recursions of every (item, lambda).
+struct PlanDev {
+    const int *nlam, *mitem, *midx;
+    const double *lam, *radii, *h0, *h1;
+    double2 *eta, *ex, *p1, *q1, *ps, *qs;
+};
+struct PlanHost {
+    int nitems = 0, nlam_max = 0, nmerged = 0;
+    std::vector<int> nlam;
+    Pack pack;
+    size_t at[7];
+    size_t auxn = 0;
+    PlanHost(const HostPlan &hp, const GreenInput &in, int nl)
+    {
+        nitems = (int)hp.rho.size();
+        nmerged = (int)hp.merged.size();
+        for (auto &l : hp.lam) {
+            nlam.push_back((int)l.size());
+            nlam_max = std::max(nlam_max, nlam.back());
+        }
+        std::vector<double> flat((size_t)nitems * nlam_max, 0.0);
+        for (int it = 0; it < nitems; ++it) std::copy(hp.lam[it].begin(), hp.lam[it].end(), flat.begin() + (size_t)it * nlam_max);
+        at[0] = pack.add(nlam);
+        at[1] = pack.add(hp.m_item);
+        at[2] = pack.add(hp.m_idx);
+        at[3] = pack.add(flat);
+        at[4] = pack.add(hp.merged);
+        at[5] = pack.add(in.hank0);
+        at[6] = pack.add(in.hank1);
+        auxn = (size_t)nitems * nlam_max * nl;
+    }
+    size_t device_bytes() const
+    {
+        return GreenScratch::padded(pack.bytes.size()) + 6 * GreenScratch::padded(auxn * sizeof(double2));
+    }
+    // uploads the pack (its device address into base) and runs the recursions; the pack must outlive them
+    PlanDev upload(GreenScratch &work, const LayerModel &lm, unsigned char *&base, hipStream_t s) const
+    {
+        base = work.take<unsigned char>(pack.bytes.size());
+        XTR_CHECK(hipMemcpyAsync(base, pack.bytes.data(), pack.bytes.size(), hipMemcpyHostToDevice, s));
+        PlanDev d;
+        d.nlam = (const int *)(base + at[0]);
+        d.mitem = (const int *)(base + at[1]);
+        d.midx = (const int *)(base + at[2]);
+        d.lam = (const double *)(base + at[3]);
+        d.radii = (const double *)(base + at[4]);
+        d.h0 = (const double *)(base + at[5]);
+        d.h1 = (const double *)(base + at[6]);
+        double2 **aux[6] = {&d.eta, &d.ex, &d.p1, &d.q1, &d.ps, &d.qs};
+        for (auto *a : aux) *a = work.take<double2>(auxn);
+        dim3 grid((unsigned)ceil_div(nlam_max, 128), nitems);
+        hipLaunchKernelGGL(layer_aux_kernel, grid, dim3(128), 0, s, lm, nitems, nlam_max, d.nlam, d.lam, d.eta, d.ex,
+                           d.p1, d.q1, d.ps, d.qs);
+        XTR_LAUNCH_CHECK("layer_aux_kernel");
+        return d;
+    }
+};
 
-}  // namespace
-
-void build_green_atoa(const GreenInput &in, double2 *G, const double2 *tw_x, const double2 *tw_y, hipStream_t s)
+LayerModel layer_model(const GreenInput &in)
 {
-    const Geom &g = in.g;
-    const int nz = g.nz;
     const int nl = (int)in.section.thickness.size();
     if (nl > kMaxLayers) throw hip_error("too many background layers for the device recursion");
     LayerModel lm{};
@@ -626,115 +680,123 @@ void build_green_atoa(const GreenInput &in, double2 *G, const double2 *tw_x, con
         d += in.section.thickness[k];
     }
     lm.depth[nl] = d;
+    return lm;
+}
 
+int layer_at_depth(const Section &s, double depth)   // ScalarMathUtils.cs:15-31
+{
+    const int k = layer_index_at_depth(s, depth);
+    if (k < 0) throw hip_error("anomaly is not within 1D section");
+    return k;
+}
+
+}  // namespace
+
+// The pairs of one set pass through the stages in chunks whose U stays in the 256 MB Infinity Cache between
+// pair_u and hankel, which also bounds the scratch (about 130 MB) whatever nz.
+constexpr size_t kChunkBytes = (size_t)64 << 20;
+
+void build_green_atoa(const GreenInput &in, GreenScratch &work, double2 *G, bool folded, const double2 *tw_x,
+                      const double2 *tw_y, hipStream_t s)
+{
+    const Geom &g = in.g;
+    const int nz = g.nz;
+    const LayerModel lm = layer_model(in);
     const HostPlan hp = make_plan(in);
-    const int nitems = (int)hp.rho.size();
-    int nlam_max = 0;
-    std::vector<int> nlam(nitems);
-    for (int it = 0; it < nitems; ++it) {
-        nlam[it] = (int)hp.lam[it].size();
-        nlam_max = std::max(nlam_max, nlam[it]);
-    }
-    std::vector<double> lam_flat((size_t)nitems * nlam_max, 0.0);
-    for (int it = 0; it < nitems; ++it) std::copy(hp.lam[it].begin(), hp.lam[it].end(), lam_flat.begin() + (size_t)it * nlam_max);
-    const int nmerged = (int)hp.merged.size();
+    PlanHost ph(hp, in, lm.nl);
 
-    Dev<int> d_nlam(nlam);
-    Dev<double> d_lam(lam_flat);
-    Dev<double> d_radii(hp.merged);
-    Dev<int> d_mitem(hp.m_item), d_midx(hp.m_idx);
-    Dev<double> d_h0(in.hank0), d_h1(in.hank1);
-    const size_t auxn = (size_t)nitems * nlam_max * nl;
-    Dev<double2> eta(auxn), ex(auxn), p1(auxn), q1(auxn), ps(auxn), qs(auxn);
-    {
-        dim3 grid((unsigned)ceil_div(nlam_max, 128), nitems);
-        hipLaunchKernelGGL(layer_aux_kernel, grid, dim3(128), 0, s, lm, nitems, nlam_max, d_nlam.p, d_lam.p, eta.p,
-                           ex.p, p1.p, q1.p, ps.p, qs.p);
-        XTR_LAUNCH_CHECK("layer_aux_kernel");
+    // transceiver pairs: Combine (rc-major) for asym, CombineSymm (tr-major, rc <= tr) for symm
+    std::vector<PairInfo> pairs[2];
+    auto add = [&](int asym, int rc, int tr) {
+        PairInfo pi{};
+        pi.r1 = in.depth[rc];
+        pi.r2 = in.depth[rc] + in.thick[rc];
+        pi.s1 = in.depth[tr];
+        pi.s2 = in.depth[tr] + in.thick[tr];
+        pi.r = layer_at_depth(in.section, pi.r1 + (pi.r2 - pi.r1) / 2);
+        pi.s = layer_at_depth(in.section, pi.s1 + (pi.s2 - pi.s1) / 2);
+        pi.t = std::min(pi.r, pi.s);
+        pi.b = std::max(pi.r, pi.s);
+        pi.dt = lm.depth[pi.t];
+        pi.db1 = lm.depth[pi.b + 1];
+        const double zw = pi.r1 + (pi.r2 - pi.r1) / 2;
+        pi.kase = (zw > pi.s1 && zw < pi.s2) ? 0 : (zw >= pi.s2 ? 1 : 2);
+        pairs[asym].push_back(pi);
+    };
+    for (int rc = 0; rc < nz; ++rc)
+        for (int tr = 0; tr < nz; ++tr) add(1, rc, tr);
+    for (int tr = 0; tr < nz; ++tr)
+        for (int rc = 0; rc <= tr; ++rc) add(0, rc, tr);
+    size_t pairs_at[2];
+    int chunk[2];
+    size_t need[4] = {0, 0, 0, 0};
+    for (int asym = 0; asym < 2; ++asym) {
+        pairs_at[asym] = ph.pack.add(pairs[asym]);
+        const int np = (int)pairs[asym].size(), ncomp = asym ? 1 : 3;
+        const size_t u1 = (size_t)ph.nitems * ncomp * ph.nlam_max;     // U of one pair
+        chunk[asym] = (int)std::min<size_t>(np, std::max<size_t>(1, kChunkBytes / (u1 * sizeof(double2)) / 256) * 256);
+        need[0] = std::max(need[0], chunk[asym] * u1);
+        need[1] = std::max(need[1], (size_t)chunk[asym] * ncomp * ph.nmerged);
+        need[2] = need[3] = need[1];
     }
-    XTR_CHECK(hipMemsetAsync(G, 0, (size_t)g.L() * g.gblk() * sizeof(double2), s));
+    size_t bytes = ph.device_bytes();
+    for (size_t n : need) bytes += GreenScratch::padded(n * sizeof(double2));
+    work.reserve(bytes);
+    unsigned char *base;
+    const PlanDev d = ph.upload(work, lm, base, s);
+    double2 *U = work.take<double2>(need[0]), *I = work.take<double2>(need[1]), *segA = work.take<double2>(need[2]),
+            *segB = work.take<double2>(need[3]);
+    if (!folded) XTR_CHECK(hipMemsetAsync(G, 0, (size_t)g.L() * g.gblk() * sizeof(double2), s));
 
+    const int nitems = ph.nitems, nlam_max = ph.nlam_max, nmerged = ph.nmerged, nseg = nmerged - 1;
     for (int asym = 1; asym >= 0; --asym) {
-        // transceiver pairs: Combine (rc-major) for asym, CombineSymm (tr-major, rc <= tr) for symm
-        std::vector<PairInfo> pairs;
-        auto add = [&](int rc, int tr) {
-            PairInfo pi{};
-            pi.r1 = in.depth[rc];
-            pi.r2 = in.depth[rc] + in.thick[rc];
-            pi.s1 = in.depth[tr];
-            pi.s2 = in.depth[tr] + in.thick[tr];
-            pi.r = layer_at_depth(in.section, pi.r1 + (pi.r2 - pi.r1) / 2);
-            pi.s = layer_at_depth(in.section, pi.s1 + (pi.s2 - pi.s1) / 2);
-            pi.t = std::min(pi.r, pi.s);
-            pi.b = std::max(pi.r, pi.s);
-            pi.dt = lm.depth[pi.t];
-            pi.db1 = lm.depth[pi.b + 1];
-            const double zw = pi.r1 + (pi.r2 - pi.r1) / 2;
-            pi.kase = (zw > pi.s1 && zw < pi.s2) ? 0 : (zw >= pi.s2 ? 1 : 2);
-            pairs.push_back(pi);
-        };
-        if (asym) {
-            for (int rc = 0; rc < nz; ++rc)
-                for (int tr = 0; tr < nz; ++tr) add(rc, tr);
-        } else {
-            for (int tr = 0; tr < nz; ++tr)
-                for (int rc = 0; rc <= tr; ++rc) add(rc, tr);
-        }
-        const int npairs = (int)pairs.size();
-        const int ncomp = asym ? 1 : 3;
-        Dev<PairInfo> d_pairs(pairs);
-        Dev<double2> U((size_t)npairs * nitems * ncomp * nlam_max);
-        {
-            dim3 grid((unsigned)ceil_div(nlam_max, 64), nitems, npairs);
-            hipLaunchKernelGGL(pair_u_kernel, grid, dim3(64), 0, s, lm, npairs, d_pairs.p, asym, nitems, nlam_max,
-                               d_nlam.p, d_lam.p, eta.p, ex.p, p1.p, q1.p, ps.p, qs.p, U.p);
+        const int ncomp = asym ? 1 : 3, all = (int)pairs[asym].size();
+        for (int p0 = 0; p0 < all; p0 += chunk[asym]) {
+            const int np = std::min(chunk[asym], all - p0);
+            const PairInfo *dp = (const PairInfo *)(base + pairs_at[asym]) + p0;
+            hipLaunchKernelGGL(pair_u_kernel, dim3((unsigned)ceil_div(nlam_max, 64), nitems, np), dim3(64), 0, s, lm, np,
+                               dp, asym, nitems, nlam_max, d.nlam, d.lam, d.eta, d.ex, d.p1, d.q1, d.ps, d.qs, U);
             XTR_LAUNCH_CHECK("pair_u_kernel");
-        }
-        Dev<double2> I((size_t)ncomp * npairs * nmerged);
-        {
-            dim3 grid((unsigned)ceil_div(nmerged, 128), npairs, ncomp);
-            hipLaunchKernelGGL(hankel_kernel, grid, dim3(128), 0, s, npairs, nitems, ncomp, nlam_max, U.p, nmerged,
-                               d_mitem.p, d_midx.p, d_radii.p, d_h0.p, d_h1.p, asym, I.p);
+            hipLaunchKernelGGL(hankel_kernel, dim3((unsigned)ceil_div(nmerged, 128), np, ncomp), dim3(128), 0, s, np,
+                               nitems, ncomp, nlam_max, U, nmerged, d.mitem, d.midx, d.radii, d.h0, d.h1, asym, I);
             XTR_LAUNCH_CHECK("hankel_kernel");
-        }
-        const int nseg = nmerged - 1;
-        Dev<double2> segA((size_t)nseg * ncomp * npairs), segB((size_t)nseg * ncomp * npairs);
-        {
-            dim3 grid((unsigned)ceil_div(npairs, 128), ncomp, nseg);
-            hipLaunchKernelGGL(segments_kernel, grid, dim3(128), 0, s, npairs, ncomp, nmerged, d_radii.p, I.p, segA.p,
-                               segB.p);
+            hipLaunchKernelGGL(segments_kernel, dim3((unsigned)ceil_div(np, 128), ncomp, nseg), dim3(128), 0, s, np,
+                               ncomp, nmerged, d.radii, I, segA, segB);
             XTR_LAUNCH_CHECK("segments_kernel");
+            LatArgs la{};
+            la.nx = g.nx;
+            la.ny = g.ny;
+            la.nz = nz;
+            la.npairs = np;
+            la.p0 = p0;
+            la.folded = folded ? 1 : 0;
+            la.asym = asym;
+            la.nr = nmerged;
+            la.dx = in.dx;
+            la.dy = in.dy;
+            la.segA = segA;
+            la.segB = segB;
+            la.radii = d.radii;
+            la.G = G;
+            la.gblk = g.gblk();
+            const int64_t S = g.S(), A = (int64_t)nz * nz;
+            if (asym) {   // q-order {xz, yz}; device block [xx|xy|yy|zz|xz|yz]; parities XZ (-,+), YZ (+,-)
+                la.off[0] = 4 * S; la.off[1] = 4 * S + A;
+                la.xs[0] = -1; la.ys[0] = 1;
+                la.xs[1] = 1; la.ys[1] = -1;
+            } else {      // q-order {xx, yy, zz, xy}; parities (+,+) x3, XY (-,-)
+                la.off[0] = 0; la.off[1] = 2 * S; la.off[2] = 3 * S; la.off[3] = S;
+                for (int t = 0; t < 3; ++t) { la.xs[t] = 1; la.ys[t] = 1; }
+                la.xs[3] = -1; la.ys[3] = -1;
+            }
+            dim3 grid((unsigned)((int64_t)g.nx * g.ny), (unsigned)ceil_div(np, 256));
+            hipLaunchKernelGGL(lateral_kernel, grid, dim3(std::min(256, ((np + 63) / 64) * 64)), 0, s, la);
+            XTR_LAUNCH_CHECK("lateral_kernel");
         }
-        LatArgs la{};
-        la.nx = g.nx;
-        la.ny = g.ny;
-        la.nz = nz;
-        la.npairs = npairs;
-        la.asym = asym;
-        la.nr = nmerged;
-        la.dx = in.dx;
-        la.dy = in.dy;
-        la.segA = segA.p;
-        la.segB = segB.p;
-        la.radii = d_radii.p;
-        la.G = G;
-        la.gblk = g.gblk();
-        const int64_t S = g.S(), A = (int64_t)nz * nz;
-        if (asym) {   // q-order {xz, yz}; device block [xx|xy|yy|zz|xz|yz]; parities XZ (-,+), YZ (+,-)
-            la.off[0] = 4 * S; la.off[1] = 4 * S + A;
-            la.xs[0] = -1; la.ys[0] = 1;
-            la.xs[1] = 1; la.ys[1] = -1;
-        } else {      // q-order {xx, yy, zz, xy}; parities (+,+) x3, XY (-,-)
-            la.off[0] = 0; la.off[1] = 2 * S; la.off[2] = 3 * S; la.off[3] = S;
-            for (int t = 0; t < 3; ++t) { la.xs[t] = 1; la.ys[t] = 1; }
-            la.xs[3] = -1; la.ys[3] = -1;
-        }
-        dim3 grid((unsigned)((int64_t)g.nx * g.ny), (unsigned)ceil_div(npairs, 256));
-        hipLaunchKernelGGL(lateral_kernel, grid, dim3(std::min(256, ((npairs + 63) / 64) * 64)), 0, s, la);
-        XTR_LAUNCH_CHECK("lateral_kernel");
-        XTR_CHECK(hipStreamSynchronize(s));   // the temporaries above are freed on scope exit
     }
-    launch_fft2_plain(G, 2 * g.nx, 2 * g.ny, g.gblk(), tw_x, tw_y, -1, s);
+    if (folded) launch_fft2_mirror(G, g, tw_x, tw_y, s);
+    else launch_fft2_plain(G, 2 * g.nx, 2 * g.ny, g.gblk(), tw_x, tw_y, -1, s);
+    XTR_CHECK(hipStreamSynchronize(s));   // the host pack is freed on return
 }
 
 
@@ -1050,51 +1112,17 @@ int atoo_components(int electric, int *slot)
     return electric ? 8 : 7;
 }
 
-void build_green_atoo_level(const GreenInput &in, double level_z, double shift_x, double shift_y, int electric,
-                            double2 *G, const double2 *tw_x, const double2 *tw_y, hipStream_t s)
+void build_green_atoo_level(const GreenInput &in, GreenScratch &work, double level_z, double shift_x, double shift_y,
+                            int electric, double2 *G, const double2 *tw_x, const double2 *tw_y, hipStream_t s)
 {
     const Geom &g = in.g;
     const int nz = g.nz;
-    const int nl = (int)in.section.thickness.size();
-    if (nl > kMaxLayers) throw hip_error("too many background layers for the device recursion");
-    LayerModel lm{};
-    lm.nl = nl;
-    lm.omega = in.omega;
-    const double eps0 = 1.0 / (kMu0 * 299792458.0 * 299792458.0);
-    double d = in.section.zero_level;
-    for (int k = 0; k < nl; ++k) {
-        lm.zeta[k] = make_double2(in.section.sigma[k], -in.omega * eps0);
-        lm.thick[k] = in.section.thickness[k];
-        lm.depth[k] = d;
-        d += in.section.thickness[k];
-    }
-    lm.depth[nl] = d;
+    const LayerModel lm = layer_model(in);
     // the level's own scalar plan (AtoOCalculator.cs:129, 151)
     const HostPlan hp = make_level_plan(in, shift_x, shift_y);
     if (hp.zero_rho && hp.rho[0].size() < 3) throw hip_error("zero-rho plan needs three radii in its first item");
-    const int nitems = (int)hp.rho.size();
-    int nlam_max = 0;
-    std::vector<int> nlam(nitems);
-    for (int it = 0; it < nitems; ++it) {
-        nlam[it] = (int)hp.lam[it].size();
-        nlam_max = std::max(nlam_max, nlam[it]);
-    }
-    std::vector<double> lam_flat((size_t)nitems * nlam_max, 0.0);
-    for (int it = 0; it < nitems; ++it) std::copy(hp.lam[it].begin(), hp.lam[it].end(), lam_flat.begin() + (size_t)it * nlam_max);
-    const int nmerged = (int)hp.merged.size();
-    Dev<int> d_nlam(nlam);
-    Dev<double> d_lam(lam_flat);
-    Dev<double> d_radii(hp.merged);
-    Dev<int> d_mitem(hp.m_item), d_midx(hp.m_idx);
-    Dev<double> d_h0(in.hank0), d_h1(in.hank1);
-    const size_t auxn = (size_t)nitems * nlam_max * nl;
-    Dev<double2> eta(auxn), ex(auxn), p1(auxn), q1(auxn), ps(auxn), qs(auxn);
-    {
-        dim3 grid((unsigned)ceil_div(nlam_max, 128), nitems);
-        hipLaunchKernelGGL(layer_aux_kernel, grid, dim3(128), 0, s, lm, nitems, nlam_max, d_nlam.p, d_lam.p, eta.p,
-                           ex.p, p1.p, q1.p, ps.p, qs.p);
-        XTR_LAUNCH_CHECK("layer_aux_kernel");
-    }
+    PlanHost ph(hp, in, lm.nl);
+    const int nitems = ph.nitems, nlam_max = ph.nlam_max, nmerged = ph.nmerged;
     // transmitters: the anomaly layers; receiver: the level point (AuxContainer.CreateContainer)
     const int r = layer_at_depth(in.section, level_z);
     std::vector<PointInfo> pts(nz);
@@ -1113,30 +1141,29 @@ void build_green_atoo_level(const GreenInput &in, double level_z, double shift_x
         pts[tr] = pi;
     }
     const int ncomp = electric ? 5 : 4;
-    Dev<PointInfo> d_pts(pts);
-    Dev<double2> U((size_t)nz * nitems * ncomp * nlam_max);
-    {
-        dim3 grid((unsigned)ceil_div(nlam_max, 64), nitems, nz);
-        hipLaunchKernelGGL(point_u_kernel, grid, dim3(64), 0, s, lm, nz, d_pts.p, electric, nitems, nlam_max, d_nlam.p,
-                           d_lam.p, eta.p, ex.p, p1.p, q1.p, ps.p, qs.p, U.p);
-        XTR_LAUNCH_CHECK("point_u_kernel");
-    }
-    Dev<double2> I((size_t)ncomp * nz * nmerged);
-    {
-        dim3 grid((unsigned)ceil_div(nmerged, 128), nz, ncomp);
-        hipLaunchKernelGGL(atoo_hankel_kernel, grid, dim3(128), 0, s, nz, nitems, ncomp, nlam_max, U.p, nmerged,
-                           d_mitem.p, d_midx.p, d_radii.p, d_h0.p, d_h1.p, electric,
-                           hp.zero_rho ? hp.rho[0][1] : 0.0, hp.zero_rho ? hp.rho[0][2] : 0.0,
-                           log10_rho_step() * log10_rho_step(), I.p);
-        XTR_LAUNCH_CHECK("atoo_hankel_kernel");
-    }
     const int nseg = nmerged - 1;
-    Dev<double2> segA((size_t)nseg * ncomp * nz), segB((size_t)nseg * ncomp * nz);
-    {
-        dim3 grid((unsigned)ceil_div(nz, 128), ncomp, nseg);
-        hipLaunchKernelGGL(segments_kernel, grid, dim3(128), 0, s, nz, ncomp, nmerged, d_radii.p, I.p, segA.p, segB.p);
-        XTR_LAUNCH_CHECK("segments_kernel");
-    }
+    const size_t pts_at = ph.pack.add(pts);
+    const size_t need[4] = {(size_t)nz * nitems * ncomp * nlam_max, (size_t)ncomp * nz * nmerged,
+                            (size_t)nseg * ncomp * nz, (size_t)nseg * ncomp * nz};
+    size_t bytes = ph.device_bytes();
+    for (size_t n : need) bytes += GreenScratch::padded(n * sizeof(double2));
+    work.reserve(bytes);
+    unsigned char *base;
+    const PlanDev d = ph.upload(work, lm, base, s);
+    double2 *U = work.take<double2>(need[0]), *I = work.take<double2>(need[1]), *segA = work.take<double2>(need[2]),
+            *segB = work.take<double2>(need[3]);
+    hipLaunchKernelGGL(point_u_kernel, dim3((unsigned)ceil_div(nlam_max, 64), nitems, nz), dim3(64), 0, s, lm, nz,
+                       (const PointInfo *)(base + pts_at), electric, nitems, nlam_max, d.nlam, d.lam, d.eta, d.ex, d.p1,
+                       d.q1, d.ps, d.qs, U);
+    XTR_LAUNCH_CHECK("point_u_kernel");
+    hipLaunchKernelGGL(atoo_hankel_kernel, dim3((unsigned)ceil_div(nmerged, 128), nz, ncomp), dim3(128), 0, s, nz,
+                       nitems, ncomp, nlam_max, U, nmerged, d.mitem, d.midx, d.radii, d.h0, d.h1, electric,
+                       hp.zero_rho ? hp.rho[0][1] : 0.0, hp.zero_rho ? hp.rho[0][2] : 0.0,
+                       log10_rho_step() * log10_rho_step(), I);
+    XTR_LAUNCH_CHECK("atoo_hankel_kernel");
+    hipLaunchKernelGGL(segments_kernel, dim3((unsigned)ceil_div(nz, 128), ncomp, nseg), dim3(128), 0, s, nz, ncomp,
+                       nmerged, d.radii, I, segA, segB);
+    XTR_LAUNCH_CHECK("segments_kernel");
     AoArgs a{};
     a.nx = g.nx;
     a.ny = g.ny;
@@ -1149,9 +1176,9 @@ void build_green_atoo_level(const GreenInput &in, double level_z, double shift_x
     a.dy = in.dy;
     a.xs = -shift_x;
     a.ys = -shift_y;
-    a.segA = segA.p;
-    a.segB = segB.p;
-    a.radii = d_radii.p;
+    a.segA = segA;
+    a.segB = segB;
+    a.radii = d.radii;
     a.G = G;
     XTR_CHECK(hipMemsetAsync(G, 0, (size_t)g.L() * a.ntc * nz * sizeof(double2), s));
     {
@@ -1160,7 +1187,7 @@ void build_green_atoo_level(const GreenInput &in, double level_z, double shift_x
         XTR_LAUNCH_CHECK("atoo_lateral_kernel");
     }
     launch_fft2_plain(G, 2 * g.nx, 2 * g.ny, (int64_t)a.ntc * nz, tw_x, tw_y, -1, s);
-    XTR_CHECK(hipStreamSynchronize(s));   // the temporaries above are freed on return
+    XTR_CHECK(hipStreamSynchronize(s));   // the host pack is freed on return
 }
 
 }  // namespace xtr

@@ -203,6 +203,7 @@ struct xtr_op {
     DevBuf<float2> tw32_x, tw32_y;
     DevBuf<unsigned char> buf;    // max_rhs * M spectrum
     DevBuf<double2> stage_x, stage_y;   // host-pointer apply staging
+    xtr::GreenScratch green_work;  // scratch of the tensor assemblies
     DevBuf<double2> Go[2];        // AtoO level tensors [L][ncomp][nz]: [0] magnetic, [1] electric
     bool go_ready[2] = {false, false};
     DevBuf<double2> lvl_spec, lvl_small;   // level-field scratch: L * 3nz and L * 3
@@ -1246,15 +1247,18 @@ int xtr_op_build_green(xtr_op *op)
         require(op, "null argument");
         require(op->hank0.size() == 431 && op->hank1.size() == 431, "the 431-tap Hankel filter is required");
         require(op->number_of_hankels > 0, "NumberOfHankels must be positive");
+        // the assembled tensor has the mirror symmetry by construction (signed mirroring), so it is assembled
+        // folded, straight into the buffer it stays in, which a rebuild uses again
         const xtr::Geom &g = op->g;
-        op->green_ready = false;
-        op->G64.release();
-        op->G32.release();
-        DevBuf<double2> full((size_t)(g.L() * g.gblk()));
-        xtr::build_green_atoa(green_input(op), full.p, op->tw64_x.p, op->tw64_y.p, op->stream);
+        const bool fold = green_fold_allowed();
+        const size_t need = (size_t)((fold ? g.Lq() : g.L()) * g.gblk());
         XTR_CHECK(hipStreamSynchronize(op->stream));
-        // the assembled tensor has the mirror symmetry by construction (signed mirroring)
-        store_green(op, full, green_fold_allowed());
+        op->green_ready = false;
+        op->G32.release();
+        if (op->G64.count != need) op->G64.alloc(need);
+        op->folded = fold;
+        xtr::build_green_atoa(green_input(op), op->green_work, op->G64.p, fold, op->tw64_x.p, op->tw64_y.p, op->stream);
+        finish_green(op);
     });
 }
 
@@ -1731,9 +1735,10 @@ int xtr_op_build_green_atoo(xtr_op *op, double level_z, double x_shift, double y
         int slot[9];
         const int ncomp = xtr::atoo_components(e, slot);
         op->go_ready[e] = false;
-        op->Go[e].alloc((size_t)(op->g.L() * ncomp * op->g.nz));
         require(std::isfinite(x_shift) && std::isfinite(y_shift), "level shift must be finite");
-        xtr::build_green_atoo_level(green_input(op), level_z, x_shift, y_shift, e, op->Go[e].p, op->tw64_x.p,
+        const size_t need = (size_t)(op->g.L() * ncomp * op->g.nz);
+        if (op->Go[e].count != need) op->Go[e].alloc(need);
+        xtr::build_green_atoo_level(green_input(op), op->green_work, level_z, x_shift, y_shift, e, op->Go[e].p, op->tw64_x.p,
                                     op->tw64_y.p, op->stream);
         op->go_ready[e] = true;
     });

@@ -1,6 +1,7 @@
 // Device assembly of the anomaly-to-anomaly Green tensor (FP64).
 #pragma once
 
+#include "xtr_common.h"
 #include "xtr_kernels.h"
 
 #include <cmath>
@@ -58,16 +59,50 @@ struct GreenInput {
     std::vector<double> hank0, hank1;   // 431 taps each
 };
 
-// Writes the FFT'd tensor in the device layout [L][xx S | xy S | yy S | zz S | xz nz^2 | yz nz^2]
-// into G (L * gblk complex128), ordered on stream s.
-void build_green_atoa(const GreenInput &in, double2 *G, const double2 *tw_x, const double2 *tw_y, hipStream_t s);
+// Device scratch of the assemblies, kept on the operator handle: one allocation, grown when a build needs
+// more and handed out piecewise (256-byte aligned). Builds of one handle run one after the other on its
+// stream and have finished when they return, so the next one may take the same bytes.
+class GreenScratch {
+public:
+    GreenScratch() = default;
+    ~GreenScratch() { (void)hipFree(p_); }
+    GreenScratch(const GreenScratch &) = delete;
+    GreenScratch &operator=(const GreenScratch &) = delete;
+    void reserve(size_t bytes)
+    {
+        used_ = 0;
+        if (bytes <= cap_) return;
+        (void)hipFree(p_);
+        p_ = nullptr;
+        cap_ = 0;
+        XTR_CHECK(hipMalloc((void **)&p_, bytes));
+        cap_ = bytes;
+    }
+    static size_t padded(size_t bytes) { return (bytes + 255) / 256 * 256; }
+    template <typename T> T *take(size_t n)
+    {
+        unsigned char *q = p_ + used_;
+        used_ += padded(n * sizeof(T));
+        if (used_ > cap_) throw hip_error("Green assembly scratch too small");
+        return reinterpret_cast<T *>(q);
+    }
+
+private:
+    unsigned char *p_ = nullptr;
+    size_t cap_ = 0, used_ = 0;
+};
+
+// Writes the FFT'd tensor in the device layout [xx S | xy S | yy S | zz S | xz nz^2 | yz nz^2] per block into
+// G, all L wavenumbers or (folded) the (Nx+1)(Ny+1) blocks kx <= Nx, ky <= Ny, on stream s, and waits for it.
+void build_green_atoa(const GreenInput &in, GreenScratch &work, double2 *G, bool folded, const double2 *tw_x,
+                      const double2 *tw_y, hipStream_t s);
 
 // AtoO level tensor for the observation level at depth level_z whose sites are the cell centres
 // shifted by (shift_x, shift_y) metres: device layout [L][component][nz] with components, in order,
 // xx yy zz xy xz yz zx zy (electric = 1) or xx xy yx xz yz zx zy (electric = 0), FFT'd; G holds
 // L * ncomp * nz complex128.
 int atoo_components(int electric, int *slot /* [9]: xx yy zz xy yx xz yz zx zy -> compact or -1 */);
-void build_green_atoo_level(const GreenInput &in, double level_z, double shift_x, double shift_y, int electric,
-                            double2 *G, const double2 *tw_x, const double2 *tw_y, hipStream_t s);
+void build_green_atoo_level(const GreenInput &in, GreenScratch &work, double level_z, double shift_x, double shift_y,
+                            int electric, double2 *G, const double2 *tw_x, const double2 *tw_y, hipStream_t s);
 
 }  // namespace xtr

@@ -136,6 +136,10 @@ void launch_inv_y(const ApplyArgs &a, hipStream_t s);
 // In-place forward 2-D FFT of a [2nx][2ny][ncols] array (Green tensor), FP64.
 void launch_fft2_plain(double2 *data, int n1, int n2, int64_t ncols, const double2 *tw1, const double2 *tw2,
                        int sign, hipStream_t s);
+// The same for a Green tensor held folded, [Nx+1][Ny+1][gblk], in place: points (i, j), i < Nx and j < Ny,
+// hold the tensor at those lateral offsets on entry, and every block the spectrum on return; the negative
+// offsets follow from the mirror parities.
+void launch_fft2_mirror(double2 *folded, const Geom &g, const double2 *tw_x, const double2 *tw_y, hipStream_t s);
 bool fft_length_supported(int p);
 
 // Reorders the Green tensor between the reference layout (six component arrays) and the
