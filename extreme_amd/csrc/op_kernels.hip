@@ -15,6 +15,7 @@
 
 #include "xtr_common.h"
 #include "xtr_kernels.h"
+#include "xtr_mfma.h"
 
 namespace xtr {
 
@@ -162,16 +163,6 @@ static_assert(Cfg<double>::NBUF * Cfg<double>::BUF * 16 + 4 * 2 * C * 16 <= 160 
 static_assert(Cfg<float>::NBUF * Cfg<float>::BUF * 8 + 4 * 2 * C * 8 <= 160 * 1024, "LDS");
 constexpr int kMaxStreamRhs = 4;
 }  // namespace stream
-
-template <int N>
-__device__ __forceinline__ void wait_vm()
-{
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
-}
-
-// LDS writes of this wave (partial sums) must be complete before other waves pass the barrier and
-// read them: s_barrier alone does not wait for them.
-#define XTR_BARRIER() asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory")
 
 #pragma clang diagnostic push
 #pragma clang diagnostic ignored "-Winline-asm"
@@ -551,7 +542,7 @@ static bool contract_force_generic()
     return e && std::strcmp(e, "generic") == 0;
 }
 
-static int device_cus()
+int device_cus()
 {
     static int cus[64] = {0};
     int dev = 0;
@@ -595,327 +586,6 @@ static bool contract_stream(const ApplyArgs &a, hipStream_t s)
                        (cplx<T> *)a.buf, L, a.g.M(), a.nrhs);
     XTR_LAUNCH_CHECK("contract_stream_kernel");
     return true;
-}
-
-// ---- folded contraction on MFMA, nz = 32 -------------------------------------------------------------
-// Folded block b serves up to 4 wavenumbers (its mirror images), so one LDS-resident block meets up to
-// 4 images x 2 right-hand sides = 8 complex columns U (96 x 8), and Y = G U is a small GEMM for the
-// 16x16x4 MFMA: B = [Re U | Im U] (96 x 16 real), A = Re G and Im G (96 x 96 each), D1 = Re G . B,
-// D2 = Im G . B, then Re Y = D1[:, :8] - D2[:, 8:] and Im Y = D1[:, 8:] + D2[:, :8] (a lane and its
-// xor-8 partner). Mirror signs: u_x (u_y) of an image with kx (ky) mirrored is negated on the way
-// into B, and y_x (y_y) on the way out. Persistent: one 256-thread workgroup per CU walks blocks; each
-// block and its spectrum columns are copied HBM -> LDS by global_load_lds_dwordx4 into a ring of NBUF
-// slots (FP64 2 x 77 KB, FP32 4 x 39 KB) exactly as in the streaming kernel. The six 16-row tiles
-// times (Re, Im) make 12 accumulators, three per wave; tiles 1 and 4 have their two parts on two
-// waves and meet through the block's slot once the MFMAs have read it. Two workgroups share a CU,
-// so one workgroup's copy runs under the other's MFMAs (FP64: one slot per workgroup; FP32: two,
-// the next block copied during the current one's MFMA steps).
-namespace fold32 {
-constexpr int NZ = 32, C = 3 * NZ, S = NZ * (NZ + 1) / 2, A = NZ * NZ, GB = 4 * S + 2 * A;
-constexpr int MASK = 15;                  // asym_swizzle_mask(32)
-constexpr int NCOL = 8;                   // complex columns per block (images x right-hand sides)
-constexpr int KSTEPS = C / 4;             // 24
-template <typename T>
-struct Cfg {
-    static constexpr int E = (int)sizeof(cplx<T>);
-    static constexpr int EPL = 16 / E;
-    static constexpr int EPC = 64 * EPL;
-    static constexpr int IMG = GB + NCOL * C;
-    static constexpr int NLOAD = (IMG + EPC - 1) / EPC;     // wave-loads per block
-    static constexpr int SLOT = NLOAD * EPC;
-    // two workgroups per CU: FP64 one slot each (one computes while the other copies), FP32 two
-    static constexpr int NBUF = E == 16 ? 1 : 2;
-    static constexpr int PW_HI = (NLOAD + 3) / 4;           // wave-loads of the waves with the most
-};
-static_assert(2 * 1 * Cfg<double>::SLOT * 16 <= 160 * 1024, "LDS (FP64, two workgroups per CU)");
-static_assert(2 * 2 * Cfg<float>::SLOT * 8 <= 160 * 1024, "LDS (FP32, two workgroups per CU)");
-static_assert(2 * 64 * 4 * 8 <= Cfg<double>::SLOT * 16 && 2 * 64 * 4 * 4 <= Cfg<float>::SLOT * 8, "exchange fits a slot");
-static_assert((Cfg<double>::SLOT * 16) % 32 == 0 && (Cfg<float>::SLOT * 8) % 32 == 0, "slots stay 32-byte aligned");
-static_assert(Cfg<double>::PW_HI < 64 && Cfg<float>::PW_HI < 64, "vmcnt range");
-static_assert(GB % 2 == 0 && C % 2 == 0, "two-element lanes stay inside one column");
-static_assert(2 * KSTEPS >= Cfg<double>::PW_HI && 2 * KSTEPS >= Cfg<float>::PW_HI, "copy spread over the steps");
-}  // namespace fold32
-
-typedef double mfma_d4 __attribute__((ext_vector_type(4)));
-typedef float mfma_f4 __attribute__((ext_vector_type(4)));
-template <typename T> struct MfmaAcc;
-template <> struct MfmaAcc<double> { typedef mfma_d4 type; };
-template <> struct MfmaAcc<float> { typedef mfma_f4 type; };
-__device__ __forceinline__ mfma_d4 mfma16(double a, double b, mfma_d4 c)
-{
-    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
-}
-__device__ __forceinline__ mfma_f4 mfma16(float a, float b, mfma_f4 c)
-{
-    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-}
-// Row of D held in register r of lane l (16x16x4 results; column = l % 16): the FP64 instruction
-// spreads consecutive rows over the lane quarters, the FP32 one over the registers.
-template <typename T>
-__device__ __forceinline__ int mfma_row(int lane, int r)
-{
-    return sizeof(T) == 8 ? 4 * r + (lane >> 4) : 4 * (lane >> 4) + r;
-}
-
-#pragma clang diagnostic push
-#pragma clang diagnostic ignored "-Winline-asm"
-// Copy of the next block, issued one wave-load at a time between the MFMA steps of the current one
-// (all at once, a wave stalls on the full memory queues before it can start its MFMAs).
-template <typename T>
-struct Fold32Copy {
-    const cplx<T> *G;
-    const cplx<T> *buf;
-    int64_t M, b;
-    FoldImages im;
-    int nrhs;
-    unsigned dst;
-    bool active;
-};
-
-template <typename T>
-__device__ __forceinline__ void fold32_issue_one(const Fold32Copy<T> &cp, int t, int wave, int lane)
-{
-    using namespace fold32;
-    using K = Cfg<T>;
-    const int k = __builtin_amdgcn_readfirstlane(wave + 4 * t);   // uniform: the branches below are scalar
-    if (!cp.active || k >= K::NLOAD) return;
-    const int e = k * K::EPC + lane * K::EPL;
-    const cplx<T> *src;
-    if ((k + 1) * K::EPC <= GB || (k * K::EPC < GB && e < GB)) {
-        // Green data (the second test: the one FP32 wave-load that straddles GB, its lower lanes)
-        src = cp.G + cp.b * GB + e;
-    } else {
-        // spectrum column q at LDS position GB + q C, element kk at (kk + 2q) mod C (the rotation
-        // spreads the columns over the LDS banks for the B reads)
-        const int u = e - GB;
-        int q = u / C, j = u - q * C;
-        const int ncol = cp.im.n * cp.nrhs;
-        if (q >= ncol) q = j = 0;                            // unused column / padding: valid data
-        int kk = j - 2 * q;
-        if (kk < 0) kk += C;
-        const int img = q / cp.nrhs, h = q - img * cp.nrhs;
-        src = cp.buf + h * cp.M + cp.im.l(img) * C + kk;
-    }
-    const unsigned m0 = __builtin_amdgcn_readfirstlane(cp.dst + (unsigned)k * 1024u);
-    asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, off nt" ::"s"(m0), "v"(src) : "memory", "m0");
-}
-
-template <typename T>
-__device__ __forceinline__ void fold32_issue(const Fold32Copy<T> &cp, int wave, int lane)
-{
-#pragma unroll
-    for (int t = 0; t < fold32::Cfg<T>::PW_HI; ++t) fold32_issue_one<T>(cp, t, wave, lane);
-}
-#pragma clang diagnostic pop
-
-// A element (row 16 TILE + i, column 4 STEP + kl) of the 96 x 96 block matrix
-// [xx xy xz; xy yy yz; -xz^T -yz^T zz]: its index in the folded block (complex elements), and whether
-// the stored value enters negated (the -xz^T, -yz^T part).
-template <int TILE, int STEP>
-__device__ __forceinline__ int fold32_a_idx(int i, int kl)
-{
-    using namespace fold32;
-    constexpr int o = TILE / 2, ci = STEP / 8;
-    const int r = 16 * (TILE % 2) + i, c = 4 * (STEP % 8) + kl;
-    if constexpr (o == ci || (o < 2 && ci < 2)) {
-        constexpr int base = o != ci ? S : o == 0 ? 0 : o == 1 ? 2 * S : 3 * S;   // xy | xx, yy, zz
-        return base + (c >= r ? r + c * (c + 1) / 2 : c + r * (r + 1) / 2);
-    } else if constexpr (ci == 2) {
-        constexpr int base = o == 0 ? 4 * S : 4 * S + A;                       // xz, yz (r, c)
-        return base + r * NZ + (c ^ (r & MASK));
-    } else {
-        constexpr int base = ci == 0 ? 4 * S : 4 * S + A;                      // -xz^T, -yz^T
-        return base + c * NZ + (r ^ (c & MASK));
-    }
-}
-template <int TILE, int STEP>
-constexpr bool fold32_a_neg = TILE / 2 == 2 && STEP / 8 < 2;
-
-// D += (NEG ? -a : a) b. The FP64 instruction negates its A operand itself (the neg modifier);
-// the FP32 one has no such modifier, the sign goes on the value.
-template <bool NEG>
-__device__ __forceinline__ mfma_d4 mfma16s(double a, double b, mfma_d4 c)
-{
-    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, NEG ? 1 : 0);
-}
-template <bool NEG>
-__device__ __forceinline__ mfma_f4 mfma16s(float a, float b, mfma_f4 c)
-{
-    return __builtin_amdgcn_mfma_f32_16x16x4f32(NEG ? -a : a, b, c, 0, 0, 0);
-}
-
-// Per-lane byte offsets, within a slot, of the A values a wave reads at each k-step: the whole
-// complex element of tile TF and part PH of tile TH. They depend only on the lane, so a wave
-// computes them once and keeps them in registers for all its blocks.
-template <typename T, int TF, int TH, int PH, int... Ss>
-__device__ __forceinline__ void fold32_offsets(std::integer_sequence<int, Ss...>, int i, int kl,
-                                               unsigned (&of)[fold32::KSTEPS], unsigned (&oh)[fold32::KSTEPS])
-{
-    constexpr unsigned E = sizeof(cplx<T>);
-    ((of[Ss] = E * (unsigned)fold32_a_idx<TF, Ss>(i, kl)), ...);
-    ((oh[Ss] = E * (unsigned)fold32_a_idx<TH, Ss>(i, kl) + (unsigned)(PH * sizeof(T))), ...);
-}
-
-template <typename T>
-__device__ __forceinline__ cplx<T> lds_cplx(const cplx<T> *blk, unsigned off)
-{
-    return *reinterpret_cast<const cplx<T> *>(reinterpret_cast<const char *>(blk) + off);
-}
-template <typename T>
-__device__ __forceinline__ T lds_part(const cplx<T> *blk, unsigned off)
-{
-    return *reinterpret_cast<const T *>(reinterpret_cast<const char *>(blk) + off);
-}
-
-// One k-step: the A values of the next step are read before this step's MFMAs, so the LDS latency
-// is covered by three MFMAs; two wave-loads of the next block's copy go out over the first steps.
-template <typename T, int TF, int TH, int PH, int STEP>
-__device__ __forceinline__ void fold32_step(const cplx<T> *__restrict__ blk, const T (&bf)[fold32::KSTEPS],
-                                            const unsigned (&of)[fold32::KSTEPS],
-                                            const unsigned (&oh)[fold32::KSTEPS], typename MfmaAcc<T>::type &f1,
-                                            typename MfmaAcc<T>::type &f2, typename MfmaAcc<T>::type &hh,
-                                            cplx<T> &gf, T &gh, const Fold32Copy<T> &cp, int wave, int lane)
-{
-    cplx<T> nf = gf;
-    T nh = gh;
-    if constexpr (STEP + 1 < fold32::KSTEPS) {
-        nf = lds_cplx<T>(blk, of[STEP + 1]);
-        nh = lds_part<T>(blk, oh[STEP + 1]);
-    }
-    if constexpr (2 * STEP < fold32::Cfg<T>::PW_HI) fold32_issue_one<T>(cp, 2 * STEP, wave, lane);
-    if constexpr (2 * STEP + 1 < fold32::Cfg<T>::PW_HI) fold32_issue_one<T>(cp, 2 * STEP + 1, wave, lane);
-    f1 = mfma16s<fold32_a_neg<TF, STEP>>(gf.x, bf[STEP], f1);
-    f2 = mfma16s<fold32_a_neg<TF, STEP>>(gf.y, bf[STEP], f2);
-    hh = mfma16s<fold32_a_neg<TH, STEP>>(gh, bf[STEP], hh);
-    gf = nf;
-    gh = nh;
-}
-
-// Wave's three accumulators over one block: tile TF (Re G and Im G parts) and part PH of tile TH.
-template <typename T, int TF, int TH, int PH, int... Ss>
-__device__ __forceinline__ void fold32_wave(std::integer_sequence<int, Ss...>, const cplx<T> *__restrict__ blk,
-                                            const T (&bf)[fold32::KSTEPS], const unsigned (&of)[fold32::KSTEPS],
-                                            const unsigned (&oh)[fold32::KSTEPS], typename MfmaAcc<T>::type &f1,
-                                            typename MfmaAcc<T>::type &f2, typename MfmaAcc<T>::type &hh,
-                                            const Fold32Copy<T> &cp, int wave, int lane)
-{
-    cplx<T> gf = lds_cplx<T>(blk, of[0]);
-    T gh = lds_part<T>(blk, oh[0]);
-    (fold32_step<T, TF, TH, PH, Ss>(blk, bf, of, oh, f1, f2, hh, gf, gh, cp, wave, lane), ...);
-}
-
-// Y of tile TILE from D1 (Re G . B) and D2 (Im G . B), stored with the image signs.
-template <typename T, int TILE>
-__device__ __forceinline__ void fold32_store(typename MfmaAcc<T>::type d1, typename MfmaAcc<T>::type d2,
-                                             cplx<T> *buf, int64_t M, const FoldImages &im, int nrhs, int lane)
-{
-    using namespace fold32;
-    constexpr int o = TILE / 2;
-    const int n = lane & 15, q = n & 7, part = n >> 3;
-    const int img = (q / nrhs) & 3, h = q % nrhs;
-    const bool live = q < im.n * nrhs;
-    const bool flip = (o == 0 && im.mx(img)) || (o == 1 && im.my(img));
-    T *dst = reinterpret_cast<T *>(buf + h * M + im.l(img) * C + o * NZ) + part;
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-        const T other = __shfl_xor(d2[r], 8, 64);
-        T v = part ? d1[r] + other : d1[r] - other;
-        if (flip) v = -v;
-        const int rr = 16 * (TILE % 2) + mfma_row<T>(lane, r);
-        if (live) dst[2 * rr] = v;
-    }
-}
-
-// The block loop of wave `wave` (tiles TF, TH): every wave runs the same loop and barriers.
-template <typename T, int TF, int TH, int PH>
-__device__ __forceinline__ void fold32_run(const cplx<T> *__restrict__ G, cplx<T> *buf, int64_t Lq, int64_t M,
-                                           int nrhs, int nx, int ny, cplx<T> *ring, unsigned base, int wave,
-                                           int lane)
-{
-    using namespace fold32;
-    using K = Cfg<T>;
-    using acc_t = typename MfmaAcc<T>::type;
-    const int64_t g = gridDim.x;                                 // the launch keeps gridDim.x <= Lq
-    const int64_t b0 = blockIdx.x;
-    const int64_t cnt = (Lq - 1 - b0) / g + 1;
-    using Seq = std::make_integer_sequence<int, KSTEPS>;
-    unsigned of[KSTEPS], oh[KSTEPS];
-    fold32_offsets<T, TF, TH, PH>(Seq{}, lane & 15, lane >> 4, of, oh);
-    Fold32Copy<T> cp{G, buf, M, 0, FoldImages{}, nrhs, 0u, false};
-    if (K::NBUF == 2) {                                          // block 0 now, block it + 1 during block it
-        cp.b = b0;
-        cp.im = fold_images(b0, nx, ny);
-        cp.dst = base;
-        cp.active = true;
-        fold32_issue<T>(cp, wave, lane);
-    }
-    for (int64_t it = 0; it < cnt; ++it) {
-        const int64_t b = b0 + it * g;
-        if (K::NBUF == 1) {                                      // the whole block now
-            cp.b = b;
-            cp.im = fold_images(b, nx, ny);
-            cp.dst = base;
-            cp.active = true;
-            fold32_issue<T>(cp, wave, lane);
-            cp.active = false;
-        } else {
-            cp.active = it + 1 < cnt;
-            if (cp.active) {
-                cp.b = b + g;
-                cp.im = fold_images(cp.b, nx, ny);
-                cp.dst = base + (unsigned)(((it + 1) % K::NBUF) * K::SLOT * K::E);
-            }
-        }
-        wait_vm<0>();                                            // block it (the only copy in flight)
-        XTR_BARRIER();                                           // block it in LDS for every wave
-        cplx<T> *blk = ring + (it % K::NBUF) * K::SLOT;
-        const FoldImages im = fold_images(b, nx, ny);
-        // B fragments: lane (kl = lane / 16, n = lane % 16) holds B[4s + kl][n] for each k-step s
-        T bf[KSTEPS];
-        {
-            const int n = lane & 15, q = n & 7, part = n >> 3, kl = lane >> 4;
-            const int img = (q / nrhs) & 3;
-            const T *ucol = reinterpret_cast<const T *>(blk + GB + q * C) + part;
-            const bool fx = im.mx(img), fy = im.my(img);
-#pragma unroll
-            for (int st = 0; st < KSTEPS; ++st) {
-                int j = 4 * st + kl + 2 * q;                     // rotated position of element 4 st + kl
-                if (j >= C) j -= C;
-                const T v = ucol[2 * j];
-                const bool flip = (st < 8 && fx) || (st >= 8 && st < 16 && fy);
-                bf[st] = flip ? -v : v;
-            }
-        }
-        acc_t f1 = {0, 0, 0, 0}, f2 = f1, hh = f1;
-        fold32_wave<T, TF, TH, PH>(Seq{}, blk, bf, of, oh, f1, f2, hh, cp, wave, lane);
-        // tiles 1 and 4: the Im G part (waves 1, 3) joins the Re G part (waves 0, 2), through the slot
-        acc_t (*exch)[64] = reinterpret_cast<acc_t (*)[64]>(blk);
-        XTR_BARRIER();                                           // every wave has read the slot
-        if (wave & 1) exch[wave >> 1][lane] = hh;
-        XTR_BARRIER();
-        acc_t h2 = f1;
-        if (!(wave & 1)) h2 = exch[wave >> 1][lane];
-        fold32_store<T, TF>(f1, f2, buf, M, im, nrhs, lane);
-        if constexpr (PH == 0) fold32_store<T, TH>(hh, h2, buf, M, im, nrhs, lane);
-        XTR_BARRIER();                                           // slot free (exchange read)
-    }
-    wait_vm<0>();                                                // no copy may land after exit
-}
-
-template <typename T>
-__global__ __launch_bounds__(256, 2) void contract_fold32_kernel(const cplx<T> *__restrict__ G, cplx<T> *buf,
-                                                                 int64_t Lq, int64_t M, int nrhs, int nx, int ny)
-{
-    using K = fold32::Cfg<T>;
-    __shared__ __attribute__((aligned(32))) cplx<T> ring[K::NBUF * K::SLOT];   // 32: exchange vectors
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const unsigned base = (unsigned)(size_t)(__attribute__((address_space(3))) cplx<T> *)ring;
-    switch (wave) {
-    case 0: fold32_run<T, 0, 1, 0>(G, buf, Lq, M, nrhs, nx, ny, ring, base, wave, lane); break;
-    case 1: fold32_run<T, 2, 1, 1>(G, buf, Lq, M, nrhs, nx, ny, ring, base, wave, lane); break;
-    case 2: fold32_run<T, 3, 4, 0>(G, buf, Lq, M, nrhs, nx, ny, ring, base, wave, lane); break;
-    default: fold32_run<T, 5, 4, 1>(G, buf, Lq, M, nrhs, nx, ny, ring, base, wave, lane); break;
-    }
 }
 
 // ---- folded contraction on MFMA, nz = 64 -------------------------------------------------------------
@@ -1307,455 +977,17 @@ static bool contract_fold64(const ApplyArgs &a, hipStream_t s)
     return true;
 }
 
-// Folded tensor, nz = 32: right-hand sides in launches of up to two.
-static bool contract_fold32(const ApplyArgs &a, hipStream_t s)
+// Folded tensor, a block that fits in LDS (contract_block.h); 1-8 right-hand sides.
+static bool contract_block(const ApplyArgs &a, hipStream_t s)
 {
-    if (!a.folded || a.g.nz != fold32::NZ || contract_force_generic()) return false;
-    const int64_t Lq = a.g.Lq();
-    const unsigned grid = (unsigned)std::min<int64_t>(Lq, 2 * (int64_t)device_cus());   // two per CU
-    for (int h0 = 0; h0 < a.nrhs; h0 += 2) {
-        const int nh = std::min(2, a.nrhs - h0);
-        if (a.precision == 0)
-            hipLaunchKernelGGL((contract_fold32_kernel<double>), dim3(grid), dim3(256), 0, s, (const double2 *)a.G,
-                               (double2 *)a.buf + h0 * a.g.M(), Lq, a.g.M(), nh, a.g.nx, a.g.ny);
-        else
-            hipLaunchKernelGGL((contract_fold32_kernel<float>), dim3(grid), dim3(256), 0, s, (const float2 *)a.G,
-                               (float2 *)a.buf + h0 * a.g.M(), Lq, a.g.M(), nh, a.g.nx, a.g.ny);
-        XTR_LAUNCH_CHECK("contract_fold32_kernel");
-    }
-    return true;
-}
-
-// ---- folded contraction for small nz ---------------------------------------------------------------
-// ApplyGreenTensorAlongZ (ConvolutionOperator.cs:274-327) over a folded tensor for the depths that
-// have no kernel of their own (nz <= 31; from nz = 4 to 24 the operator handle times it against
-// contract_foldm_kernel once per shape and takes the faster). A workgroup takes folded blocks b = blockIdx.x,
-// += gridDim.x; each block is read from HBM once, expanded into six full nz x ld matrices in LDS
-// (xx, xy, yy, zz, xz, yz; ld = nz rounded up to odd, so that rows and columns are both read without
-// bank conflicts), and applied to the spectrum columns of all its images (<= 4) and right-hand sides
-// (<= 8) at once, with the image's mirror signs on the x and y components of u and y. Thread
-// (group cg, row q = (a, i)) forms row q of y for columns cg, cg + ngroups, ...: J accumulators.
-// Each thread holds E elements of the block in registers, and the next block's are loaded while this
-// one is contracted.
-// The mirror signs are formed as integer flags with bitwise operators and applied as a factor of
-// +-1: with hipcc (ROCm 7.2, gfx950) the short-circuit form
-//   if ((a == 0 && mx) || (a == 1 && my)) v = -v;
-// in this divergent code compiled to an empty conditional block for the second term, so lanes where
-// only a == 1 && my held stored v unnegated (the same source run on CPU threads is exact).
-namespace foldn {
-// f(integral_constant<int, t>) for t = 0 .. N-1: array indices known at compile time, so per-thread
-// arrays stay in registers
-template <typename F, int... Ts>
-__device__ __forceinline__ void static_for(std::integer_sequence<int, Ts...>, F &&f)
-{
-    (f(std::integral_constant<int, Ts>{}), ...);
-}
-constexpr int NT = 256;
-constexpr int MAX_NZ = 31;
-static_assert(4 * (MAX_NZ * (MAX_NZ + 1) / 2) + 2 * MAX_NZ * MAX_NZ <= 16 * NT, "a block is at most 16 elements per thread");
-__host__ __device__ inline int ld_of(int nz) { return nz | 1; }
-// row stride of the spectrum columns in LDS: 3nz rounded up to odd, so that the columns of a block's
-// images (3nz complex apart; a multiple of 256 bytes at nz = 16) fall on different LDS banks
-__host__ __device__ inline int ldu_of(int nz) { return (3 * nz) | 1; }
-
-// A thread's share of one folded block's loads: Green elements e = tid + t NT (t < E) and spectrum
-// elements tid + t NT (t < U; a block with more spectrum values loads the rest directly). What does
-// not depend on the block is computed once per kernel: each Green element's LDS destinations (two for
-// an off-diagonal element of a symmetric block), each spectrum element's column (image, right-hand
-// side) and k, and the divisions behind them. The values of the next block are loaded while the
-// current one is contracted.
-template <typename T, int E>
-struct Loads {
-    static constexpr int U = 4;
-    int gd1[E], gd2[E];                  // LDS destinations, -1: none
-    T gre[E], gim[E];
-    int uimg[U], uh[U], uk[U], ucomp[U]; // uimg -1: outside the largest block
-    int us[U];                           // LDS position: column * ldu + k
-    T ure[U], uim[U];
-
-    __device__ void init(int tid, int nz, int nrhs, const uint16_t *__restrict__ packed_rc)
-    {
-        const int ld = ld_of(nz), msz = nz * ld, S = nz * (nz + 1) / 2, A = nz * nz, gblk = 4 * S + 2 * A;
-        const int C = 3 * nz, swz = asym_swizzle_mask(nz);
-        static_for(std::make_integer_sequence<int, E>{}, [&](auto t) {
-            const int e = tid + t * NT;
-            gd1[t] = gd2[t] = -1;
-            if (e < 4 * S) {
-                const int bi = e / S, o = e - bi * S;
-                const int rc = packed_rc[2 * o], tr = packed_rc[2 * o + 1];
-                gd1[t] = bi * msz + rc * ld + tr;
-                if (rc != tr) gd2[t] = bi * msz + tr * ld + rc;
-            } else if (e < gblk) {
-                const int o = e - 4 * S, bi = 4 + o / A, pos = o % A;
-                const int rc = pos / nz, tr = (pos % nz) ^ (rc & swz);
-                gd1[t] = bi * msz + rc * ld + tr;
-            }
-        });
-        static_for(std::make_integer_sequence<int, U>{}, [&](auto t) {
-            const int e = tid + t * NT;
-            uimg[t] = -1;
-            uh[t] = uk[t] = ucomp[t] = us[t] = 0;
-            if (e < 4 * nrhs * C) {
-                const int j = e / C;
-                uk[t] = e - j * C;
-                us[t] = j * ldu_of(nz) + uk[t];
-                uimg[t] = j / nrhs;
-                uh[t] = j - uimg[t] * nrhs;
-                ucomp[t] = uk[t] < nz ? 0 : uk[t] < 2 * nz ? 1 : 2;
-            }
-        });
-    }
-    // block b's values into registers; spectrum values with the image's mirror signs
-    __device__ void load(const cplx<T> *__restrict__ G, int64_t b, int gblk, const cplx<T> *buf, int64_t M, int C,
-                         const FoldImages &im)
-    {
-        const cplx<T> *gb = G + b * (int64_t)gblk;
-        static_for(std::make_integer_sequence<int, E>{}, [&](auto t) {
-            if (gd1[t] >= 0) {
-                const cplx<T> g = gb[threadIdx.x + t * NT];
-                gre[t] = g.x;
-                gim[t] = g.y;
-            }
-        });
-        static_for(std::make_integer_sequence<int, U>{}, [&](auto t) {
-            ure[t] = uim[t] = T(0);
-            if (uimg[t] >= 0 && uimg[t] < im.n) {
-                const cplx<T> v = buf[uh[t] * M + im.l(uimg[t]) * C + uk[t]];
-                const int flip = ((ucomp[t] == 0) & im.mx(uimg[t])) | ((ucomp[t] == 1) & im.my(uimg[t]));
-                const T sg = flip ? T(-1) : T(1);
-                ure[t] = sg * v.x;
-                uim[t] = sg * v.y;
-            }
-        });
-    }
-    // the registers into LDS (gm: six nz x ld matrices, u: [images * nrhs][ldu])
-    __device__ void store(cplx<T> *gm, cplx<T> *u, int ncols) const
-    {
-        static_for(std::make_integer_sequence<int, E>{}, [&](auto t) {
-            const cplx<T> g = mk<T>(gre[t], gim[t]);
-            if (gd1[t] >= 0) gm[gd1[t]] = g;
-            if (gd2[t] >= 0) gm[gd2[t]] = g;
-        });
-        static_for(std::make_integer_sequence<int, U>{}, [&](auto t) {
-            if (uimg[t] >= 0 && threadIdx.x + t * NT < ncols) u[us[t]] = mk<T>(ure[t], uim[t]);
-        });
-    }
-};
-
-// Spectrum values of block im beyond the U NT that Loads carries (more than 1024 values: several
-// right-hand sides at larger nz), loaded directly.
-template <typename T>
-__device__ void load_rest(cplx<T> *u, const cplx<T> *buf, int64_t M, int nz, int nrhs, const FoldImages &im, int from)
-{
-    const int C = 3 * nz, ncols = im.n * nrhs * C;
-    for (int e = from + (int)threadIdx.x; e < ncols; e += NT) {
-        const int j = e / C, k = e - j * C;
-        const int img = j / nrhs, h = j - img * nrhs;
-        const cplx<T> v = buf[h * M + im.l(img) * C + k];
-        const int flip = ((k < nz) & im.mx(img)) | ((k >= nz) & (k < 2 * nz) & im.my(img));
-        const T sg = flip ? T(-1) : T(1);
-        u[j * ldu_of(nz) + k] = mk<T>(sg * v.x, sg * v.y);
-    }
-}
-}  // namespace foldn
-
-template <typename T, int J, int E>
-__global__ __launch_bounds__(foldn::NT) void contract_foldn_kernel(const cplx<T> *__restrict__ G, cplx<T> *buf,
-                                                                  int64_t Lq, int64_t M, int nz, int nrhs, int nx,
-                                                                  int ny, const uint16_t *__restrict__ packed_rc)
-{
-    extern __shared__ unsigned char smem_raw[];
-    const int ld = foldn::ld_of(nz), C = 3 * nz, S = nz * (nz + 1) / 2, A = nz * nz;
-    const int gblk = 4 * S + 2 * A;                        // the launch keeps gblk <= E * NT
-    const int msz = nz * ld;
-    cplx<T> *gm = reinterpret_cast<cplx<T> *>(smem_raw);   // [6][nz][ld]
-    cplx<T> *u = gm + 6 * msz;                             // [images * nrhs][ldu]
-    const int ldu = foldn::ldu_of(nz);
-    const int tid = threadIdx.x;
-    const int ngroups = foldn::NT / C;                     // the launch keeps C <= NT
-    const int q = tid % C, cg = tid / C;
-    const int a = q / nz, i = q % nz;
-    // row q of the 3x3 block operator, one segment per component of u:
-    //   y_x = XX u_x + XY u_y + XZ u_z; y_y = XY u_x + YY u_y + YZ u_z; y_z = -XZ^T u_x - YZ^T u_y + ZZ u_z
-    int mat[3];
-    bool trn[3];
-    mat[0] = a == 0 ? 0 : a == 1 ? 1 : 4;
-    mat[1] = a == 0 ? 1 : a == 1 ? 2 : 5;
-    mat[2] = a == 0 ? 4 : a == 1 ? 5 : 3;
-    trn[0] = a == 2;
-    trn[1] = a == 2;
-    trn[2] = false;
-    using Lo = foldn::Loads<T, E>;
-    Lo lo;
-    lo.init(tid, nz, nrhs, packed_rc);
-    if ((int64_t)blockIdx.x < Lq) lo.load(G, blockIdx.x, gblk, buf, M, C, fold_images(blockIdx.x, nx, ny));
-    for (int64_t b = blockIdx.x; b < Lq; b += gridDim.x) {
-        const FoldImages im = fold_images(b, nx, ny);
-        const int ncol = im.n * nrhs;
-        __syncthreads();                                   // the previous block's LDS reads are done
-        lo.store(gm, u, ncol * C);
-        if (ncol * C > Lo::U * foldn::NT) foldn::load_rest<T>(u, buf, M, nz, nrhs, im, Lo::U * foldn::NT);
-        __syncthreads();
-        if (b + gridDim.x < Lq) lo.load(G, b + gridDim.x, gblk, buf, M, C, fold_images(b + gridDim.x, nx, ny));
-        if (cg >= ngroups) continue;
-        cplx<T> acc[J];
-#pragma unroll
-        for (int jj = 0; jj < J; ++jj) acc[jj] = mk<T>(0, 0);
-#pragma unroll
-        for (int sgm = 0; sgm < 3; ++sgm) {
-            const cplx<T> *m = gm + mat[sgm] * msz;
-            const cplx<T> *row = trn[sgm] ? m + i : m + i * ld;
-            const int step = trn[sgm] ? ld : 1;
-            const cplx<T> *us = u + sgm * nz;
-            for (int c = 0; c < nz; ++c) {
-                cplx<T> g = row[c * step];
-                if (trn[sgm]) g = mk<T>(-g.x, -g.y);
-#pragma unroll
-                for (int jj = 0; jj < J; ++jj) {
-                    const int j = cg + jj * ngroups;
-                    if (j < ncol) acc[jj] = cfma<T>(acc[jj], g, us[j * ldu + c]);
-                }
-            }
-        }
-#pragma unroll
-        for (int jj = 0; jj < J; ++jj) {
-            const int j = cg + jj * ngroups;
-            if (j < ncol) {
-                const int img = j / nrhs, h = j - img * nrhs;
-                const int flip = ((a == 0) & im.mx(img)) | ((a == 1) & im.my(img));
-                const T sg = flip ? T(-1) : T(1);
-                buf[h * M + im.l(img) * C + q] = mk<T>(sg * acc[jj].x, sg * acc[jj].y);
-            }
-        }
-    }
-}
-
-// ---- folded contraction for small nz on MFMA ---------------------------------------------------
-// The same work as contract_foldn_kernel (same LDS layout, same loads) with the products on
-// 16x16x4 MFMAs: per (row tile of 16 rows of the 3nz x 3nz block operator, column tile of 8 complex
-// columns) a wave forms D1 = Re A . B and D2 = Im A . B with B = [Re U | Im U] (the 8 columns' spectrum
-// values, held in registers for all k-steps), and Y = D1 - D2' / D1' + D2 by a lane exchange. Each
-// A operand is read from the six expanded matrices through a per-lane address: row (a, i) of the
-// operator and k = (segment, c) pick matrix, orientation and sign (-XZ^T, -YZ^T in the z rows);
-// (segment, c) advance by 4 per k-step. The operands come from registers, so LDS carries about one
-// Green value per lane and MFMA instead of one spectrum value per complex MAC.
-namespace foldm {
-constexpr int NT = foldn::NT;               // four waves; foldn::Loads assumes this count
-constexpr int MIN_NZ = 4;                   // one k-step of 4 advances c across at most one segment
-constexpr int MAX_NZ = 24;
-constexpr int MAX_KS = (3 * MAX_NZ + 3) / 4;
-static_assert(4 * (MAX_NZ * (MAX_NZ + 1) / 2) + 2 * MAX_NZ * MAX_NZ <= 12 * NT, "a block is at most 12 elements per thread");
-}  // namespace foldm
-
-template <typename T, int E>
-__global__ __launch_bounds__(foldm::NT) void contract_foldm_kernel(const cplx<T> *__restrict__ G, cplx<T> *buf,
-                                                                  int64_t Lq, int64_t M, int nz, int nrhs, int nx,
-                                                                  int ny, const uint16_t *__restrict__ packed_rc)
-{
-    using acc_t = typename MfmaAcc<T>::type;
-    extern __shared__ unsigned char smem_raw[];
-    const int ld = foldn::ld_of(nz), C = 3 * nz, S = nz * (nz + 1) / 2, A = nz * nz;
-    const int gblk = 4 * S + 2 * A;                        // the launch keeps gblk <= E * NT
-    const int msz = nz * ld;
-    const int KS = (C + 3) / 4, RT = (C + 15) / 16;        // k-steps, row tiles
-    cplx<T> *gm = reinterpret_cast<cplx<T> *>(smem_raw);   // [6][nz][ld]: xx, xy, yy, zz, xz, yz
-    cplx<T> *u = gm + 6 * msz;                             // [images * nrhs][ldu]
-    const int ldu = foldn::ldu_of(nz);
-    const int tid = threadIdx.x, lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int n = lane & 15, kk = lane >> 4, part = n >> 3;
-    using Lo = foldn::Loads<T, E>;
-    Lo lo;
-    lo.init(tid, nz, nrhs, packed_rc);
-    if ((int64_t)blockIdx.x < Lq) lo.load(G, blockIdx.x, gblk, buf, M, C, fold_images(blockIdx.x, nx, ny));
-    for (int64_t b = blockIdx.x; b < Lq; b += gridDim.x) {
-        const FoldImages im = fold_images(b, nx, ny);
-        const int ncol = im.n * nrhs;
-        __syncthreads();                                   // the previous block's LDS reads are done
-        lo.store(gm, u, ncol * C);
-        if (ncol * C > Lo::U * foldn::NT) foldn::load_rest<T>(u, buf, M, nz, nrhs, im, Lo::U * foldn::NT);
-        __syncthreads();
-        if (b + gridDim.x < Lq) lo.load(G, b + gridDim.x, gblk, buf, M, C, fold_images(b + gridDim.x, nx, ny));
-        const int nct = (ncol + 7) / 8;
-        for (int it = wave; it < RT * nct; it += 4) {      // (row tile, column tile) items of this wave
-            const int rt = it % RT, ct = it / RT;
-            const int col = 8 * ct + (n & 7);
-            const bool cval = col < ncol;
-            // B[k][n] = Re (n < 8) or Im (n >= 8) of column col's value at k = 4 ks + kk
-            T bfr[foldm::MAX_KS];
-#pragma unroll
-            for (int ks = 0; ks < foldm::MAX_KS; ++ks) {
-                const int k = 4 * ks + kk;
-                T v = T(0);
-                if (ks < KS && cval && k < C) {
-                    const cplx<T> w = u[col * ldu + k];
-                    v = part ? w.y : w.x;
-                }
-                bfr[ks] = v;
-            }
-            // lane's A row: operator row 16 rt + n = (a, i); per segment the matrix base, the step along
-            // c and the sign (row-major XX XY XZ / XY YY YZ / ZZ; the z rows read -XZ, -YZ by columns)
-            const int row = 16 * rt + n;
-            const bool rval = row < C;
-            const int a = rval ? row / nz : 0, i = rval ? row - a * nz : 0;
-            const int m0 = a == 0 ? 0 : a == 1 ? 1 : 4;
-            const int m1 = a == 0 ? 1 : a == 1 ? 2 : 5;
-            const int m2 = a == 0 ? 4 : a == 1 ? 5 : 3;
-            const int zr = a == 2;                          // the z rows: segments 0, 1 transposed and negated
-            const int base0 = m0 * msz + (zr ? i : i * ld), step0 = zr ? ld : 1;
-            const int base1 = m1 * msz + (zr ? i : i * ld), step1 = zr ? ld : 1;
-            const int base2 = m2 * msz + i * ld;
-            const T s01 = zr ? T(-1) : T(1);
-            const T rv = rval ? T(1) : T(0);
-            int seg = 0, c = kk;                            // k = 4 ks + kk = seg nz + c (nz >= 4)
-            if (c >= nz) { c -= nz; seg = 1; }
-            acc_t d1 = {0, 0, 0, 0}, d2 = {0, 0, 0, 0};
-#pragma unroll
-            for (int ks = 0; ks < foldm::MAX_KS; ++ks) {
-                if (ks < KS) {
-                    const int base = seg == 0 ? base0 : seg == 1 ? base1 : base2;
-                    const int step = seg == 0 ? step0 : seg == 1 ? step1 : 1;
-                    const T f = seg < 2 ? s01 * rv : (seg == 2 ? rv : T(0));
-                    const cplx<T> g = gm[seg < 3 ? base + c * step : 0];
-                    d1 = mfma16(f * g.x, bfr[ks], d1);
-                    d2 = mfma16(f * g.y, bfr[ks], d2);
-                    c += 4;
-                    if (c >= nz) { c -= nz; ++seg; }
-                    if (c >= nz) { c -= nz; ++seg; }
-                }
-            }
-            const acc_t y = fold64_combine<T>(d1, d2, lane);
-            if (cval) {
-                const int img = col / nrhs, h = col - img * nrhs;
-                const int fx = im.mx(img), fy = im.my(img);
-                T *dst = reinterpret_cast<T *>(buf + h * M + im.l(img) * C) + part;
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const int rr = 16 * rt + mfma_row<T>(lane, r);
-                    if (rr < C) {
-                        const int ar = rr / nz;
-                        const int flip = ((ar == 0) & fx) | ((ar == 1) & fy);
-                        dst[2 * rr] = flip ? -y[r] : y[r];
-                    }
-                }
-            }
-        }
-    }
-}
-
-// Workgroups of `kernel` (NT threads, lds bytes of dynamic LDS) resident per CU, from the compiled
-// kernel's registers and LDS; cached per kernel and LDS size. A persistent grid larger than
-// CUs x this would run in rounds, each workgroup paying its prologue and first loads again.
-static int resident_per_cu(const void *kernel, int nt, size_t lds)
-{
-    static std::mutex mu;
-    static std::map<std::pair<const void *, size_t>, int> cache;
-    std::lock_guard<std::mutex> lk(mu);
-    auto it = cache.find({kernel, lds});
-    if (it != cache.end()) return it->second;
-    int nb = 0;
-    XTR_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, kernel, nt, lds));
-    nb = std::max(1, nb);
-    cache[{kernel, lds}] = nb;
-    return nb;
-}
-
-static int device_max_lds()
-{
-    static int lds[64] = {0};
-    int dev = 0;
-    XTR_CHECK(hipGetDevice(&dev));
-    if (dev < 0 || dev >= 64) throw hip_error("device index out of range");
-    if (!lds[dev]) XTR_CHECK(hipDeviceGetAttribute(&lds[dev], hipDeviceAttributeMaxSharedMemoryPerBlock, dev));
-    return lds[dev];
-}
-
-template <typename T, int J, int E>
-static void launch_foldn(const ApplyArgs &a, unsigned grid, size_t lds, hipStream_t s)
-{
-    const void *k = (const void *)contract_foldn_kernel<T, J, E>;
-    grid = (unsigned)std::min<int64_t>(grid, (int64_t)resident_per_cu(k, foldn::NT, lds) * device_cus());
-    hipLaunchKernelGGL((contract_foldn_kernel<T, J, E>), dim3(grid), dim3(foldn::NT), lds, s, (const cplx<T> *)a.G,
-                       (cplx<T> *)a.buf, a.g.Lq(), a.g.M(), a.g.nz, a.nrhs, a.g.nx, a.g.ny, a.packed_rc);
-}
-
-template <typename T, int J>
-static void launch_foldn_e(const ApplyArgs &a, unsigned grid, size_t lds, hipStream_t s)
-{
-    const int64_t per_thread = ceil_div(a.g.gblk(), foldn::NT);   // <= 16 for nz <= 31
-    if (per_thread <= 4) launch_foldn<T, J, 4>(a, grid, lds, s);
-    else if (per_thread <= 8) launch_foldn<T, J, 8>(a, grid, lds, s);
-    else if (per_thread <= 12) launch_foldn<T, J, 12>(a, grid, lds, s);
-    else launch_foldn<T, J, 16>(a, grid, lds, s);
-}
-
-// Folded tensor, nz <= 31, 1-8 right-hand sides in one launch (one Green-tensor read).
-template <typename T>
-static bool contract_foldn(const ApplyArgs &a, hipStream_t s)
-{
-    const int nz = a.g.nz;
-    if (!a.folded || nz < 1 || nz > foldn::MAX_NZ || a.nrhs < 1 || a.nrhs > kMaxRhs || contract_force_generic())
-        return false;
-    const int C = 3 * nz;
-    const size_t lds = sizeof(cplx<T>) * ((size_t)6 * nz * foldn::ld_of(nz) + (size_t)4 * a.nrhs * foldn::ldu_of(nz));
-    if (lds > (size_t)device_max_lds()) return false;
-    const int ngroups = foldn::NT / C;
-    const int need = (4 * a.nrhs + ngroups - 1) / ngroups;    // columns per thread
-    const int per_cu = std::max(1, std::min(8, (int)(device_max_lds() / lds)));
-    const unsigned grid = (unsigned)std::min<int64_t>(a.g.Lq(), (int64_t)per_cu * device_cus());
-    if (need <= 2) launch_foldn_e<T, 2>(a, grid, lds, s);
-    else if (need <= 4) launch_foldn_e<T, 4>(a, grid, lds, s);
-    else if (need <= 8) launch_foldn_e<T, 8>(a, grid, lds, s);
-    else launch_foldn_e<T, 16>(a, grid, lds, s);
-    XTR_LAUNCH_CHECK("contract_foldn_kernel");
-    return true;
-}
-
-// XTR_CONTRACT_KERNEL=vector keeps small-nz folded tensors on contract_foldn_kernel, =mfma puts every
-// depth contract_foldm_kernel supports on it (to compare the two).
-static bool contract_kernel_is(const char *name)
-{
-    const char *e = std::getenv("XTR_CONTRACT_KERNEL");
-    return e && std::strcmp(e, name) == 0;
-}
-
-template <typename T, int E>
-static void launch_foldm(const ApplyArgs &a, unsigned grid, size_t lds, hipStream_t s)
-{
-    const void *k = (const void *)contract_foldm_kernel<T, E>;
-    grid = (unsigned)std::min<int64_t>(grid, (int64_t)resident_per_cu(k, foldm::NT, lds) * device_cus());
-    hipLaunchKernelGGL((contract_foldm_kernel<T, E>), dim3(grid), dim3(foldm::NT), lds, s, (const cplx<T> *)a.G,
-                       (cplx<T> *)a.buf, a.g.Lq(), a.g.M(), a.g.nz, a.nrhs, a.g.nx, a.g.ny, a.packed_rc);
-}
-
-// Folded tensor, 1-8 right-hand sides in one launch, on MFMA: by the fixed rule from nz = 17 to 24.
-// Measured against contract_foldn_kernel (two right-hand sides, FP64): 163 against 186 us per launch
-// at nz = 24, but 63 against 48 us at nz = 16 and 38 against 30 us at nz = 8 and 12. The operator
-// handle measures the two once per process and shape and sets a.contract_variant.
-template <typename T>
-static bool contract_foldm(const ApplyArgs &a, hipStream_t s)
-{
-    const int nz = a.g.nz;
-    const int lowest = contract_kernel_is("mfma") || a.contract_variant == CONTRACT_MFMA ? foldm::MIN_NZ : 17;
-    if (!a.folded || nz < lowest || nz > foldm::MAX_NZ || a.nrhs < 1 || a.nrhs > kMaxRhs ||
-        contract_force_generic() || contract_kernel_is("vector") || a.contract_variant == CONTRACT_VECTOR)
-        return false;
-    const size_t lds = sizeof(cplx<T>) * ((size_t)6 * nz * foldn::ld_of(nz) + (size_t)4 * a.nrhs * foldn::ldu_of(nz));
-    if (lds > (size_t)device_max_lds()) return false;
-    const int per_cu = std::max(1, std::min(8, (int)(device_max_lds() / lds)));
-    const unsigned grid = (unsigned)std::min<int64_t>(a.g.Lq(), (int64_t)per_cu * device_cus());
-    const int64_t per_thread = ceil_div(a.g.gblk(), foldm::NT);
-    if (per_thread <= 4) launch_foldm<T, 4>(a, grid, lds, s);
-    else if (per_thread <= 8) launch_foldm<T, 8>(a, grid, lds, s);
-    else launch_foldm<T, 12>(a, grid, lds, s);
-    XTR_LAUNCH_CHECK("contract_foldm_kernel");
-    return true;
-}
-
-bool contract_variants_apply(const ApplyArgs &a)
-{
-    return a.folded && a.g.nz >= foldm::MIN_NZ && a.g.nz <= foldm::MAX_NZ && a.nrhs >= 1 && a.nrhs <= kMaxRhs &&
-           !std::getenv("XTR_CONTRACT_KERNEL");
+    // byte offsets within one right-hand side's spectrum are 32-bit
+    if (!a.folded || a.nrhs < 1 || a.nrhs > kMaxRhs || contract_force_generic() || a.g.M() * 16 > 0xffffffffLL) return false;
+    using Range = bool (*)(const ApplyArgs &, hipStream_t);
+    static const Range c128[] = {contract_block_c128_a, contract_block_c128_b, contract_block_c128_c, contract_block_c128_d};
+    static const Range c64[] = {contract_block_c64_a, contract_block_c64_b, contract_block_c64_c, contract_block_c64_d};
+    for (Range r : a.precision ? c64 : c128)
+        if (r(a, s)) return true;
+    return false;
 }
 
 template <typename T>
@@ -1763,10 +995,8 @@ static void contract(const ApplyArgs &a, hipStream_t s)
 {
     if (!a.folded && contract_stream<T>(a, s)) return;
     if (!a.folded && contract_stream64(a, s)) return;
-    if (contract_fold32(a, s)) return;
     if (contract_fold64(a, s)) return;
-    if (contract_foldm<T>(a, s)) return;
-    if (contract_foldn<T>(a, s)) return;
+    if (contract_block(a, s)) return;
     const int nz = a.g.nz, C = 3 * nz;
     const int per_w = a.nrhs * C;
     int W = per_w >= 256 ? 1 : 256 / per_w;

@@ -106,14 +106,8 @@ struct ApplyArgs {
     const void *tw_y;         // twiddles for P = 2 ny
     int fft_tile[4];          // column tile of fwd_y, fwd_x, inv_x, inv_y (FFT_TILE_*)
     int vec32;                // v.x and v.y point to complex64 vectors (float2; precision FP32 only)
-    int contract_variant;     // folded nz <= 31: CONTRACT_* (CONTRACT_RULE: MFMA from nz = 17)
     RhsPtrs v;
 };
-
-enum { CONTRACT_RULE = 0, CONTRACT_VECTOR = 1, CONTRACT_MFMA = 2 };
-// true when the apply can take either small-nz contraction (folded, 4 <= nz <= 24) and no
-// XTR_CONTRACT_KERNEL override fixes the kernel
-bool contract_variants_apply(const ApplyArgs &a);
 
 enum {
     FFT_TILE_DEFAULT = 0,
@@ -130,6 +124,17 @@ int fft_tile_options(int p, int precision, int *tiles);
 void launch_fwd_y(const ApplyArgs &a, hipStream_t s);
 void launch_fwd_x(const ApplyArgs &a, hipStream_t s);
 void launch_contract(const ApplyArgs &a, hipStream_t s);
+// the contraction of a folded tensor whose block fits in LDS (contract_block.h), by ranges of depths; false:
+// not a depth of the range, or one that does not fit
+bool contract_block_c128_a(const ApplyArgs &a, hipStream_t s);
+bool contract_block_c128_b(const ApplyArgs &a, hipStream_t s);
+bool contract_block_c128_c(const ApplyArgs &a, hipStream_t s);
+bool contract_block_c128_d(const ApplyArgs &a, hipStream_t s);
+bool contract_block_c64_a(const ApplyArgs &a, hipStream_t s);
+bool contract_block_c64_b(const ApplyArgs &a, hipStream_t s);
+bool contract_block_c64_c(const ApplyArgs &a, hipStream_t s);
+bool contract_block_c64_d(const ApplyArgs &a, hipStream_t s);
+int device_cus();            // compute units of the current device
 void launch_inv_x(const ApplyArgs &a, hipStream_t s);
 void launch_inv_y(const ApplyArgs &a, hipStream_t s);
 
