@@ -24,6 +24,7 @@
 #include "xtr_common.h"
 #include "xtr_green.h"
 #include "xtr_kernels.h"
+#include "xtr_mfma.h"
 
 #include <algorithm>
 #include <cmath>
@@ -92,12 +93,13 @@ struct LayerModel {
     double omega;
 };
 
-__global__ void layer_aux_kernel(LayerModel lm, int nitems, int nlam_max, const int *nlam, const double *lam,
+__global__ __launch_bounds__(128) void layer_aux_kernel(const LayerModel *lmp, int nitems, int nlam_max, const int *nlam, const double *lam,
                                  double2 *eta, double2 *ex, double2 *p1, double2 *q1, double2 *ps, double2 *qs)
 {
     const int m = blockIdx.x * blockDim.x + threadIdx.x;
     const int it = blockIdx.y;
     if (it >= nitems || m >= nlam[it]) return;
+    const LayerModel &lm = *lmp;
     const int nl = lm.nl;
     const double l = lam[(int64_t)it * nlam_max + m];
     const int64_t base = ((int64_t)it * nlam_max + m) * nl;
@@ -151,11 +153,6 @@ struct PairInfo {
     double r1, r2, s1, s2, dt, db1;
 };
 
-__device__ inline double2 e4(double2 a, double2 b, double2 c, double2 d)
-{
-    return cexp_d(a) - cexp_d(b) - cexp_d(c) + cexp_d(d);
-}
-
 // A[rc][tr] (CalculateA :160-200; CalculateASigma :138-158 for sigma = 1)
 __device__ inline double2 ann_at(const LayerModel &lm, const double2 *E, const double2 *X, const double2 *P,
                                  const double2 *Q, int rc, int tr, int sigma)
@@ -170,7 +167,8 @@ __device__ inline double2 ann_at(const LayerModel &lm, const double2 *E, const d
     return prev;
 }
 
-__global__ void pair_u_kernel(LayerModel lm, int npairs, const PairInfo *pairs, int asym, int nitems,
+// The layer model lies in memory: indexed by a pair's layer, an argument would go through scratch.
+__global__ __launch_bounds__(64) void pair_u_kernel(const LayerModel *lmp, int npairs, const PairInfo *pairs, int asym, int nitems,
                               int nlam_max, const int *nlam, const double *lam, const double2 *eta,
                               const double2 *ex, const double2 *p1, const double2 *q1, const double2 *ps,
                               const double2 *qs, double2 *U)
@@ -180,26 +178,32 @@ __global__ void pair_u_kernel(LayerModel lm, int npairs, const PairInfo *pairs, 
     const int p = blockIdx.z;
     if (it >= nitems || m >= nlam[it] || p >= npairs) return;
     const PairInfo pi = pairs[p];
+    const LayerModel &lm = *lmp;
     const int nl = lm.nl;
     const int64_t base = ((int64_t)it * nlam_max + m) * nl;
     const double2 *E = eta + base, *X = ex + base;
     const double l = lam[(int64_t)it * nlam_max + m];
     const double2 er = E[pi.r], es = E[pi.s], et = E[pi.t], eb = E[pi.b];
-    // PreCalculate (VolumeToVolumeCalculatorUFast.cs:34-46)
-    const double2 T = e4(-pi.r1 * er - pi.s1 * es + 2 * pi.dt * et, -pi.r1 * er - pi.s2 * es + 2 * pi.dt * et,
-                         -pi.r2 * er - pi.s1 * es + 2 * pi.dt * et, -pi.r2 * er - pi.s2 * es + 2 * pi.dt * et);
-    const double2 Rv = e4(-2 * pi.db1 * eb + pi.s2 * es + pi.r2 * er, -2 * pi.db1 * eb + pi.s1 * es + pi.r2 * er,
-                          -2 * pi.db1 * eb + pi.s2 * es + pi.r1 * er, -2 * pi.db1 * eb + pi.s1 * es + pi.r1 * er);
+    // PreCalculate (VolumeToVolumeCalculatorUFast.cs:34-46): T, R, C and D are each four exponentials, +- at the
+    // two faces of either layer, that is the term at the faces that make it largest times (1 - e^(-tau_r eta_r))
+    // (1 - e^(-tau_s eta_s)), tau the thicknesses. Six complex exponentials a thread instead of sixteen (they are
+    // nearly all of its work: 1.25 -> 0.65 ms a build at 128 x 128 x 32, 0.42 ms with the registers a block of 64
+    // threads may have instead of spills), and the differences of nearly equal
+    // exponentials at small lambda lose one factor of eps / (tau eta) instead of the product of both: against 40
+    // digits over 0 to 6 km, 1e-3 to 10 Hz and lambda 1e-9 to 3, the mean error falls from 2e-11..2e-14 to
+    // 3e-14..4e-15. No intermediate exceeds the largest of the four terms.
+    const double2 xr = cexp_d(-(pi.r2 - pi.r1) * er), xs = cexp_d(-(pi.s2 - pi.s1) * es);
+    const double2 faces = (c_(1) - xr) * (c_(1) - xs);
+    const double2 T = cexp_d(-pi.r1 * er - pi.s1 * es + 2 * pi.dt * et) * faces;
+    const double2 Rv = cexp_d(-2 * pi.db1 * eb + pi.s2 * es + pi.r2 * er) * faces;
     double2 C = c_(0), D = c_(0);
     const double2 F = -2 * pi.db1 * eb + 2 * pi.dt * et;
     if (pi.kase == 2) {   // rc above tr: Ctop, Dtop
-        C = e4(-pi.s1 * es + pi.r2 * er, -pi.s2 * es + pi.r2 * er, -pi.s1 * es + pi.r1 * er, -pi.s2 * es + pi.r1 * er);
-        D = e4(F + pi.s2 * es - pi.r1 * er, F + pi.s1 * es - pi.r1 * er, F + pi.s2 * es - pi.r2 * er,
-               F + pi.s1 * es - pi.r2 * er);
+        C = cexp_d(-pi.s1 * es + pi.r2 * er) * faces;
+        D = cexp_d(F + pi.s2 * es - pi.r1 * er) * faces;
     } else if (pi.kase == 1) {   // rc below tr: Cbot, Dbot
-        C = e4(-pi.r1 * er + pi.s2 * es, -pi.r1 * er + pi.s1 * es, -pi.r2 * er + pi.s2 * es, -pi.r2 * er + pi.s1 * es);
-        D = e4(F - pi.s1 * es + pi.r2 * er, F - pi.s2 * es + pi.r2 * er, F - pi.s1 * es + pi.r1 * er,
-               F - pi.s2 * es + pi.r1 * er);
+        C = cexp_d(-pi.r1 * er + pi.s2 * es) * faces;
+        D = cexp_d(F - pi.s1 * es + pi.r2 * er) * faces;
     }
     const double2 zrc2 = 2.0 * lm.zeta[pi.r];
     const int ncomp = asym ? 1 : 3;
@@ -218,7 +222,7 @@ __global__ void pair_u_kernel(LayerModel lm, int npairs, const PairInfo *pairs, 
             const double2 en = E[n];
             const double2 PQ = P[n] * Q[n];
             // CalcPsi1RcAndTrMatch (:313-332)
-            const double2 part1 = tau * en - (c_(1) - cexp_d(-tau * en));
+            const double2 part1 = tau * en - (c_(1) - xr);
             const double2 part2 = PQ * ((tau * en + c_(1)) * cexp_d(-2 * dn1 * en) - cexp_d(-2 * dn1 * en + tau * en));
             psi1 = 2.0 * (part1 - part2);
             psi3 = c_(0);
@@ -253,7 +257,7 @@ __global__ void pair_u_kernel(LayerModel lm, int npairs, const PairInfo *pairs, 
             const double2 kk = (c_(0, lm.omega) * lm.zeta[n]) * c_(kMu0);
             const double2 en = E[n];
             const double2 PQ = P[n] * Q[n];
-            const double2 part1 = -(c_(1) - cexp_d(-tau * en));
+            const double2 part1 = -(c_(1) - xr);
             const double2 part2 = PQ * (cexp_d(-(2 * ln - tau) * en) - cexp_d(-2 * ln * en));
             const double2 part3 = (kk / c_(l * l)) * (c_(1) - PQ * cexp_d(-2 * ln * en)) * (tau * en);
             const double2 psi5 = 2.0 * (part1 + part2 + part3);
@@ -266,45 +270,116 @@ __global__ void pair_u_kernel(LayerModel lm, int npairs, const PairInfo *pairs, 
 }
 
 // ---- K3: Hankel filter onto the merged rho grid -------------------------------------------
-// I[comp][pair][k] = sgn * (sum_j hank[430-j] U[pair][item][comp][idx+j]) / (2 pi rho_k)
-__global__ void hankel_kernel(int npairs, int nitems, int ncomp, int nlam_max, const double2 *U, int nmerged,
-                              const int *m_item, const int *m_idx, const double *radii, const double *hank0,
-                              const double *hank1, int asym, double2 *I)
+// For every (row p, item, component): I[k][c][p] = sgn_c (sum_j hank[430 - j] U[p][item][c][ix + j]) / (den rho_k),
+// k the place of the item's radius ix among the merged radii; component c uses J0 where bit c of j0 is set.
+// The filter is the same for every row, so the sums are a product of the banded Toeplitz matrix
+// H[ix][lambda] = hank[430 - (lambda - ix)] with the rows' U: 16 radii x 4 lambdas x 8 rows (Re, Im) per
+// 16x16x4 MFMA, one wave per 8 rows with up to 8 radius tiles at once, tiles outside the band skipped. H comes
+// from a zero-padded filter in LDS, U straight from memory, read once. At 128 x 128 x 32 the 5 GFLOP take
+// 136 us where one thread per radius, whose neighbours read other items' rows, took 1460.
+struct HankelArgs {
+    int np, nitems, ncomp, nlam_max, nrho_max;
+    const double2 *U;
+    const int *nlam, *mpos;       // mpos[item][ix]: the radius's place
+    const double *radii, *h0, *h1;
+    int j0;
+    double sgn[5], den;
+    double2 *I;
+};
+constexpr int kHTiles = 8, kHPad = 16 * kHTiles - 1;
+constexpr int kHSteps = (kTaps - 1 + 16 * kHTiles + 15) / 16 * 4;             // k-steps of a full group
+constexpr int kHTable = kHPad + 4 * kHSteps;
+
+__global__ __launch_bounds__(256) void hankel_kernel(HankelArgs a)
 {
-    const int k = blockIdx.x * blockDim.x + threadIdx.x;
-    const int p = blockIdx.y;
-    const int c = blockIdx.z;
-    if (k >= nmerged || p >= npairs || c >= ncomp) return;
-    const int it = m_item[k], idx = m_idx[k];
-    const double *hank = asym ? hank0 : hank1;      // I3 with J0; I1, I2, I5 with J1
-    const double2 *f = U + (((int64_t)p * nitems + it) * ncomp + c) * nlam_max + idx;
-    double re = 0, im = 0;
-    for (int j = 0; j < kTaps; ++j) {
-        const double h = hank[kTaps - 1 - j];
-        const double2 v = f[j];
-        re += v.x * h;
-        im += v.y * h;
+    __shared__ double h[kHTable];
+    const int it = blockIdx.y, c = blockIdx.z;
+    const double *hank = (a.j0 >> c) & 1 ? a.h0 : a.h1;
+    for (int x = threadIdx.x; x < kHTable; x += blockDim.x) {
+        const int j = x - kHPad;
+        h[x] = j >= 0 && j < kTaps ? hank[kTaps - 1 - j] : 0.0;
     }
-    const double den = 2 * kPi * radii[k];
-    const double sgn = (!asym && c == 0) ? -1.0 : 1.0;   // I1 = -I1/(2 pi rho)
-    I[((int64_t)c * npairs + p) * nmerged + k] = make_double2(sgn * re / den, sgn * im / den);
+    __syncthreads();
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int p0 = (blockIdx.x * 4 + wave) * 8;
+    if (p0 >= a.np) return;
+    const int n = lane & 15, kl = lane >> 4, p = p0 + (n >> 1), part = n & 1;
+    const int nlam = a.nlam[it], nrho = nlam - kTaps;
+    const double *u = reinterpret_cast<const double *>(
+                          a.U + (((int64_t)min(p, a.np - 1) * a.nitems + it) * a.ncomp + c) * a.nlam_max) + part;
+    const double *hl = h + kHPad + kl - n;                             // H[i = n][k = kl], plus 4 step - 16 tile
+    for (int ix0 = 0; ix0 < nrho; ix0 += 16 * kHTiles) {
+        const int tiles = min(kHTiles, (nrho - ix0 + 15) / 16);
+        const int chunks = (kTaps - 1 + 16 * tiles + 15) / 16;         // of 4 k-steps
+        auto get = [&](int step) __attribute__((always_inline)) {      // past the row's end: no radius uses it
+            const int k = ix0 + 4 * step + kl;
+            const double v = u[2 * min(k, nlam - 1)];
+            return k < nlam ? v : 0.0;
+        };
+        mfma_d4 acc[kHTiles];
+#pragma unroll
+        for (int t = 0; t < kHTiles; ++t) acc[t] = mfma_d4{0, 0, 0, 0};
+        double bn[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) bn[q] = get(q);
+        for (int ch = 0; ch < chunks; ++ch) {
+            double b[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) b[q] = bn[q];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) bn[q] = get(4 * (ch + 1) + q);
+            const double *hc = hl + 16 * ch;
+#pragma unroll
+            for (int t = 0; t < kHTiles; ++t) {
+                // radii 16 t .. 16 t + 15 use lambdas 16 t .. 16 t + 15 + 430 of this group
+                if (t < tiles && t <= ch && 16 * ch <= 16 * t + 15 + kTaps - 1) {
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) acc[t] = mfma16(hc[4 * q - 16 * t], b[q], acc[t]);
+                }
+            }
+        }
+#pragma unroll
+        for (int t = 0; t < kHTiles; ++t)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int ix = ix0 + 16 * t + mfma_row<double>(lane, r);
+                if (ix < nrho && p < a.np) {
+                    const int k = a.mpos[it * a.nrho_max + ix];
+                    reinterpret_cast<double *>(a.I)[(((int64_t)k * a.ncomp + c) * a.np + p) * 2 + part] =
+                        a.sgn[c] * acc[t][r] / (a.den * a.radii[k]);
+                }
+            }
+    }
+}
+
+void launch_hankel(const HankelArgs &a, hipStream_t s)
+{
+    hipLaunchKernelGGL(hankel_kernel, dim3((unsigned)ceil_div(a.np, 32), a.nitems, a.ncomp), dim3(256), 0, s, a);
+    XTR_LAUNCH_CHECK("hankel_kernel");
 }
 
 // ---- K4: segments --------------------------------------------------------------------------
-__global__ void segments_kernel(int npairs, int ncomp, int nmerged, const double *radii, const double2 *I,
-                                double2 *segA, double2 *segB)
+// segA, segB and I are [k][comp][row]; `stride` values per radius
+__global__ __launch_bounds__(256) void segments_kernel(int64_t stride, int64_t total, const double *radii, const double2 *I,
+                                                       double2 *segA, double2 *segB)
 {
-    const int p = blockIdx.x * blockDim.x + threadIdx.x;
-    const int c = blockIdx.y;
-    const int k = blockIdx.z;
-    if (p >= npairs) return;
-    const double s = radii[k], u = radii[k + 1], div = u - s;
-    const double2 i0 = I[((int64_t)c * npairs + p) * nmerged + k];
-    const double2 i1 = I[((int64_t)c * npairs + p) * nmerged + k + 1];
-    const double2 a = make_double2((i1.x - i0.x) / div, (i1.y - i0.y) / div);
-    const int64_t o = ((int64_t)k * ncomp + c) * npairs + p;
-    segA[o] = a;
-    segB[o] = make_double2(i0.x - a.x * s, i0.y - a.y * s);
+    for (int64_t o = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; o < total; o += (int64_t)gridDim.x * blockDim.x) {
+        const int64_t k = o / stride;
+        const double s = radii[k], u = radii[k + 1], div = u - s;
+        const double2 i0 = I[o], i1 = I[o + stride];
+        const double2 a = make_double2((i1.x - i0.x) / div, (i1.y - i0.y) / div);
+        segA[o] = a;
+        segB[o] = make_double2(i0.x - a.x * s, i0.y - a.y * s);
+    }
+}
+
+void launch_segments(int ncomp, int np, int nmerged, const double *radii, const double2 *I, double2 *segA, double2 *segB,
+                     hipStream_t s)
+{
+    const int64_t stride = (int64_t)ncomp * np, total = (nmerged - 1) * stride;
+    hipLaunchKernelGGL(segments_kernel, dim3((unsigned)std::min<int64_t>(ceil_div(total, 256), 4096)), dim3(256), 0, s,
+                       stride, total, radii, I, segA, segB);
+    XTR_LAUNCH_CHECK("segments_kernel");
 }
 
 // ---- K5: lateral integration, mirroring, device layout ---------------------------------------
@@ -342,7 +417,7 @@ __device__ inline Factors factors(double s, double u, double rs, double ru, doub
 }
 
 struct LatArgs {
-    int nx, ny, nz, npairs, asym, nr;
+    int nx, ny, nz, npairs, nr;
     int p0;                       // first pair of this chunk
     int folded;                   // G holds blocks [Nx+1][Ny+1], else [2Nx][2Ny]
     double dx, dy;
@@ -354,125 +429,182 @@ struct LatArgs {
     int xs[4], ys[4];             // mirror parities, q-order
 };
 
-// q-order: asym {xz, yz}; symm {xx, yy, zz, xy}
-struct Q4 { double2 q[4]; };
+// One stretch of an edge with its ends on one side of the axis: at distance v from the other axis, from s to u
+// along it, through the segments left.index .. right.index (Integrate, GreenTensorCalculator.cs:367-411).
+struct Stretch {
+    Knot left, right;
+    double s, u, v;
+    int sign, mirrored;           // sign of the edge; the stretch lies on the axis's negative side
+    __device__ Factors at(const double *radii, int e) const
+    {
+        const int i = left.index + e;
+        const bool first = e == 0, last = i == right.index;
+        const double r1 = first ? left.radius : radii[i], r2 = last ? right.radius : radii[i + 1];
+        return factors(first ? s : sqrt(r1 * r1 - v * v), last ? u : sqrt(r2 * r2 - v * v), r1, r2, v);
+    }
+};
 
-__device__ inline void add_seg(const LatArgs &a, int p, const Factors &f, int seg, bool alongY, Q4 &Q)
+// Stretch e = 0..7 of the four edges of a cell (x1, x2) x (y1, y2): edges along x at y1 (sign -1) and y2 (+1), then
+// along y at x1, x2 (RunAlongX :254-298, RunAlongY :318-361), each in one stretch, or in two from the axis outwards
+// where it crosses it; false: this one does not exist.
+struct StretchEnds {
+    double s, u, v;               // along the edge, and its distance from the axis parallel to it
+    double l, r;                  // the coordinates along the edge whose radii bound it
+    int sign, mirrored;
+};
+__device__ inline bool stretch_ends(int e, double x1, double x2, double y1, double y2, StretchEnds &t)
 {
-    const int np = a.npairs;
-    if (a.asym) {
-        const int64_t o = (int64_t)seg * np + p;
-        const double2 A3 = a.segA[o], B3 = a.segB[o];
-        double2 &q = alongY ? Q.q[0] : Q.q[1];       // AlongY -> Qxz, AlongX -> Qyz (D1)
-        q = q + f.d1a * A3;
-        q = q + f.d1b * B3;
-        return;
-    }
-    const int64_t o1 = ((int64_t)seg * 3 + 0) * np + p, o2 = o1 + np, o5 = o2 + np;
-    const double2 A1 = a.segA[o1], B1 = a.segB[o1], A2 = a.segA[o2], B2 = a.segB[o2];
-    const double2 A5 = a.segA[o5], B5 = a.segB[o5];
-    if (!alongY) {   // AddToQBuffAlongXElectric (GreenTensorCalculator.cs:505-516)
-        Q.q[0] = Q.q[0] + f.d2a * A1; Q.q[0] = Q.q[0] + f.d2b * B1;
-        Q.q[1] = Q.q[1] + f.d2a * A2; Q.q[1] = Q.q[1] + f.d2b * B2;
-        Q.q[2] = Q.q[2] + f.d2a * A5; Q.q[2] = Q.q[2] + f.d2b * B5;
-        Q.q[3] = Q.q[3] + f.d3a * A2; Q.q[3] = Q.q[3] + f.d3b * B2;
-    } else {         // AddToQBuffAlongYElectric (:517-528)
-        Q.q[0] = Q.q[0] + f.d2a * A2; Q.q[0] = Q.q[0] + f.d2b * B2;
-        Q.q[1] = Q.q[1] + f.d2a * A1; Q.q[1] = Q.q[1] + f.d2b * B1;
-        Q.q[2] = Q.q[2] + f.d2a * A5; Q.q[2] = Q.q[2] + f.d2b * B5;
-        Q.q[3] = Q.q[3] + f.d3a * A1; Q.q[3] = Q.q[3] + f.d3b * B1;
-    }
+    const int along_y = e >> 2, far = (e >> 1) & 1, half = e & 1;
+    const double a1 = along_y ? y1 : x1, a2 = along_y ? y2 : x2;
+    t.v = along_y ? (far ? x2 : x1) : (far ? y2 : y1);
+    t.sign = far ? 1 : -1;
+    t.mirrored = 0;
+    const int pos = (int)(a1 > 0) & (int)(a2 > 0), neg = (int)(a1 < 0) & (int)(a2 < 0);
+    if (pos) { t.s = t.l = a1; t.u = t.r = a2; return half == 0; }
+    if (neg) { t.l = a2; t.r = a1; t.s = -a2; t.u = -a1; t.mirrored = 1; return half == 0; }
+    t.s = t.l = 0;
+    if (half == 0) { t.u = -a1; t.r = a1; t.mirrored = 1; }
+    else { t.u = t.r = a2; }
+    return true;
 }
 
-// Integrate (GreenTensorCalculator.cs:367-411)
-__device__ inline Q4 integrate(const LatArgs &a, int p, Knot left, Knot right, double s, double u, double v, bool alongY)
+// The four edge integrals of one cell (x1, x2) x (y1, y2) as weights on the segments I_c(rho) = A_c rho + B_c they
+// cross. A component's value is sum over segments of w . (A, B); w holds, for the edges along x and along y, the
+// signed factors d1, d2, d3 (each for A and B) summed over the edge pair: sign -1 for the nearer edge, +1 for the
+// farther. What FillResultAlongX/Y (:413-437) multiply by the QSigns tables (QSign.cs:31-38, 64-67) is a sign of
+// the component and, for d3 only, the opposite sign on a stretch mirrored about the axis (rows AlongXSymm,
+// AlongYSymm); the latter is in the weights here, the former with the components' sums.
+// The weights are the same for every pair of layers, so a team of threads forms them once in LDS: knots by binary
+// search, then a logarithm and two square roots for each (segment, stretch), then the sums. Each coefficient is
+// then read once per cell and segment instead of once per edge and segment.
+enum { W1A, W1B, W2A, W2B, W3A, W3B, WN };
+template <int SEGS>
+struct CellWeights {
+    Stretch st[8];
+    int is[8];
+    double f[SEGS][8][WN];
+    double w[SEGS][2][WN];        // [edges along x, along y]
+    // the cell's stretches; returns through lo, hi the segments they cross (after the team's next sync)
+    __device__ void ends(int tid, const double *radii, int nr, double x1, double x2, double y1, double y2)
+    {
+        if (tid >= 16) return;
+        const int e = tid >> 1, side = tid & 1;
+        StretchEnds t;
+        const bool there = stretch_ends(e, x1, x2, y1, y2, t);
+        const double c = side ? t.r : t.l;
+        const Knot k = e < 4 ? make_knot(radii, nr, c, t.v) : make_knot(radii, nr, t.v, c);
+        if (side) {
+            st[e].right = k;
+        } else {
+            st[e].left = k;
+            st[e].s = t.s;
+            st[e].u = t.u;
+            st[e].v = t.v;
+            st[e].sign = t.sign;
+            st[e].mirrored = t.mirrored;
+            is[e] = there;
+        }
+    }
+    __device__ void range(int &lo, int &hi) const
+    {
+        lo = 1 << 30;
+        hi = -1;
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+            if (is[e]) {
+                lo = min(lo, st[e].left.index);
+                hi = max(hi, st[e].right.index);
+            }
+    }
+    __device__ void factors_of(int tid, int nt, const double *radii, int seg0, int n)
+    {
+        for (int t = tid; t < 8 * n; t += nt) {
+            const int k = t >> 3, e = t & 7, i = seg0 + k - st[e].left.index;
+            double d[WN] = {0, 0, 0, 0, 0, 0};
+            if (is[e] && i >= 0 && seg0 + k <= st[e].right.index) {
+                const Factors q = st[e].at(radii, i);
+                const double sg = st[e].sign, s3 = st[e].mirrored ? sg : -sg;
+                d[W1A] = sg * q.d1a; d[W1B] = sg * q.d1b;
+                d[W2A] = sg * q.d2a; d[W2B] = sg * q.d2b;
+                d[W3A] = s3 * q.d3a; d[W3B] = s3 * q.d3b;
+            }
+#pragma unroll
+            for (int c = 0; c < WN; ++c) f[k][e][c] = d[c];
+        }
+    }
+    __device__ void sum(int tid, int nt, int n)
+    {
+        for (int t = tid; t < 2 * WN * n; t += nt) {
+            const int k = t / (2 * WN), r = t % (2 * WN), ax = r / WN, c = r % WN;
+            w[k][ax][c] = (f[k][4 * ax][c] + f[k][4 * ax + 1][c]) + (f[k][4 * ax + 2][c] + f[k][4 * ax + 3][c]);
+        }
+    }
+};
+
+__device__ __forceinline__ double2 wab(const double (&w)[WN], int c, double2 q, double2 A, double2 B)
 {
-    Q4 Q;
-    for (int t = 0; t < 4; ++t) Q.q[t] = c_(0);
-    const int i1 = left.index, i2 = right.index;
-    if (i1 == i2) {
-        add_seg(a, p, factors(s, u, left.radius, right.radius, v), i1, alongY, Q);
-        return Q;
-    }
-    double r1 = left.radius, r2 = a.radii[i1 + 1];
-    double sj = s, uj = sqrt(r2 * r2 - v * v);
-    add_seg(a, p, factors(sj, uj, r1, r2, v), i1, alongY, Q);
-    for (int i = i1 + 1; i < i2; ++i) {
-        r1 = r2;
-        r2 = a.radii[i + 1];
-        sj = uj;
-        uj = sqrt(r2 * r2 - v * v);
-        add_seg(a, p, factors(sj, uj, r1, r2, v), i, alongY, Q);
-    }
-    sj = uj; uj = u; r1 = r2; r2 = right.radius;
-    add_seg(a, p, factors(sj, uj, r1, r2, v), i2, alongY, Q);
-    return Q;
+    return make_double2(fma(w[c], A.x, fma(w[c + 1], B.x, q.x)), fma(w[c], A.y, fma(w[c + 1], B.y, q.y)));
 }
 
-// QSigns (QSign.cs:64-67) in q-order; rows AlongX, AlongY, AlongXSymm, AlongYSymm
-__constant__ int kQsAsym[4][2] = {{1, 1}, {1, 1}, {-1, 1}, {1, -1}};
-__constant__ int kQsSymm[4][4] = {{1, -1, -1, -1}, {-1, 1, -1, -1}, {1, -1, -1, 1}, {-1, 1, -1, 1}};
+// One workgroup per cell and a share of the pairs. Bound by the L2 reads of the segments' coefficients (96 bytes
+// a pair and segment). At 128 x 128 x 32: 0.73 ms for both sets; 3.6 ms with every thread working out the edges'
+// geometry for its own pair, 1.16 ms with the geometry shared but one pass over the segments per edge.
+constexpr int kCellSegs = 32;
 
-__device__ inline void fill(const LatArgs &a, Q4 &G, const Q4 &Q, int sign, int qsel)
-{
-    const int nq = a.asym ? 2 : 4;
-    for (int t = 0; t < nq; ++t) {
-        const int qs = a.asym ? kQsAsym[qsel][t] : kQsSymm[qsel][t];
-        G.q[t] = G.q[t] + (double)(sign * qs) * Q.q[t];
-    }
-}
-
+template <int ASYM>
 __global__ __launch_bounds__(256) void lateral_kernel(LatArgs a)
 {
+    __shared__ CellWeights<kCellSegs> cw;
     const int64_t cell = blockIdx.x;
     const int i = (int)(cell / a.ny), j = (int)(cell % a.ny);
-    const int p = blockIdx.y * blockDim.x + threadIdx.x;
-    if (p >= a.npairs) return;
-    const double dx = a.dx, dy = a.dy;
-    Q4 G;
-    for (int t = 0; t < 4; ++t) G.q[t] = c_(0);
-    // edges along x at y = dy(jj - 0.5), jj = j (sign -1) and j + 1 (sign +1)   [RunAlongX :254-298]
-    for (int e = 0; e < 2; ++e) {
-        const int jj = j + e;
-        const int sign = e == 0 ? -1 : 1;
-        const double y = dy * (jj - 0.5);
-        const double x1 = dx * (i - 0.5), x2 = dx * (i + 0.5);
-        if (x1 > 0 && x2 > 0) {
-            const Knot kl = make_knot(a.radii, a.nr, x1, y), kr = make_knot(a.radii, a.nr, x2, y);
-            fill(a, G, integrate(a, p, kl, kr, x1, x2, y, false), sign, 0);
-        } else {
-            const Knot kz = make_knot(a.radii, a.nr, 0, y);
-            const Knot kl = make_knot(a.radii, a.nr, x1, y), kr = make_knot(a.radii, a.nr, x2, y);
-            fill(a, G, integrate(a, p, kz, kl, 0, -x1, y, false), sign, 2);
-            fill(a, G, integrate(a, p, kz, kr, 0, x2, y, false), sign, 0);
-        }
+    const int p = blockIdx.y * blockDim.x + threadIdx.x, np = a.npairs;
+    cw.ends(threadIdx.x, a.radii, a.nr, a.dx * (i - 0.5), a.dx * (i + 0.5), a.dy * (j - 0.5), a.dy * (j + 0.5));
+    __syncthreads();
+    int lo, hi;
+    cw.range(lo, hi);
+    // asym {xz, yz}; symm {xx, yy, zz, xy}
+    constexpr int nq = ASYM ? 2 : 4;
+    double2 G[nq];
+#pragma unroll
+    for (int t = 0; t < nq; ++t) G[t] = c_(0);
+    for (int seg0 = lo; seg0 <= hi; seg0 += kCellSegs) {
+        const int n = min(kCellSegs, hi - seg0 + 1);
+        cw.factors_of(threadIdx.x, blockDim.x, a.radii, seg0, n);
+        __syncthreads();
+        cw.sum(threadIdx.x, blockDim.x, n);
+        __syncthreads();
+        if (p < np)
+#pragma unroll 2
+            for (int k = 0; k < n; ++k) {
+                const double (&wx)[WN] = cw.w[k][0], (&wy)[WN] = cw.w[k][1];
+                const int64_t o = (int64_t)(seg0 + k) * (ASYM ? 1 : 3) * np + p;
+                if constexpr (ASYM) {      // edges along y give xz, along x yz (AddToQBuff..., D1)
+                    const double2 A3 = a.segA[o], B3 = a.segB[o];
+                    G[0] = wab(wy, W1A, G[0], A3, B3);
+                    G[1] = wab(wx, W1A, G[1], A3, B3);
+                } else {                   // AddToQBuffAlongXElectric (:505-516), AlongY (:517-528)
+                    const double2 A1 = a.segA[o], B1 = a.segB[o], A2 = a.segA[o + np], B2 = a.segB[o + np];
+                    const double2 A5 = a.segA[o + 2 * np], B5 = a.segB[o + 2 * np];
+                    const double nyw[WN] = {0, 0, -wy[W2A], -wy[W2B], 0, 0}, nxw[WN] = {0, 0, -wx[W2A], -wx[W2B], 0, 0};
+                    G[0] = wab(nyw, W2A, wab(wx, W2A, G[0], A1, B1), A2, B2);
+                    G[1] = wab(nxw, W2A, wab(wy, W2A, G[1], A1, B1), A2, B2);
+                    G[2] = wab(nyw, W2A, wab(nxw, W2A, G[2], A5, B5), A5, B5);
+                    G[3] = wab(wy, W3A, wab(wx, W3A, G[3], A2, B2), A1, B1);
+                }
+            }
+        __syncthreads();                                       // the weights are read
     }
-    // edges along y at x = dx(ii - 0.5), ii = i (sign -1) and i + 1 (sign +1)   [RunAlongY :318-361]
-    for (int e = 0; e < 2; ++e) {
-        const int ii = i + e;
-        const int sign = e == 0 ? -1 : 1;
-        const double x = dx * (ii - 0.5);
-        const double y1 = dy * (j - 0.5), y2 = dy * (j + 0.5);
-        if (y1 > 0 && y2 > 0) {
-            const Knot kl = make_knot(a.radii, a.nr, x, y1), kr = make_knot(a.radii, a.nr, x, y2);
-            fill(a, G, integrate(a, p, kl, kr, y1, y2, x, true), sign, 1);
-        } else {
-            const Knot kz = make_knot(a.radii, a.nr, x, 0);
-            const Knot kl = make_knot(a.radii, a.nr, x, y1), kr = make_knot(a.radii, a.nr, x, y2);
-            fill(a, G, integrate(a, p, kz, kl, 0, -y1, x, true), sign, 3);
-            fill(a, G, integrate(a, p, kz, kr, 0, y2, x, true), sign, 1);
-        }
-    }
+    if (p >= np) return;
     // write G(i,j) and, into a full tensor, its mirror images (GreenTensorFftPopulator.cs:88-148); of a folded
     // one the FFT forms the images from the parities as it reads
-    const int nq = a.asym ? 2 : 4;
     const int64_t nx2 = 2LL * a.nx, ny2 = a.folded ? a.ny + 1 : 2LL * a.ny;
     // asym pairs are rc-major (p = rc*nz + tr); the device block stores them swizzled
     const int pa = a.p0 + p;
-    const int pd = a.asym ? asym_pos(pa / a.nz, pa % a.nz, a.nz, asym_swizzle_mask(a.nz)) : pa;
+    const int pd = ASYM ? asym_pos(pa / a.nz, pa % a.nz, a.nz, asym_swizzle_mask(a.nz)) : pa;
+#pragma unroll
     for (int t = 0; t < nq; ++t) {
         const int64_t o = a.off[t] + pd;
-        const double2 g = G.q[t];
+        const double2 g = G[t];
         a.G[((int64_t)i * ny2 + j) * a.gblk + o] = g;
         if (a.folded) continue;
         if (i >= 1) a.G[((nx2 - i) * ny2 + j) * a.gblk + o] = (double)a.xs[t] * g;
@@ -608,17 +740,18 @@ struct Pack {
 
 // The scalar plan and the filter on the device, and the layer recursions of every (item, lambda).
 struct PlanDev {
-    const int *nlam, *mitem, *midx;
+    const int *nlam, *mpos;
     const double *lam, *radii, *h0, *h1;
+    const LayerModel *lm;
     double2 *eta, *ex, *p1, *q1, *ps, *qs;
 };
 struct PlanHost {
-    int nitems = 0, nlam_max = 0, nmerged = 0;
+    int nitems = 0, nlam_max = 0, nmerged = 0, nrho_max = 0;
     std::vector<int> nlam;
     Pack pack;
     size_t at[7];
     size_t auxn = 0;
-    PlanHost(const HostPlan &hp, const GreenInput &in, int nl)
+    PlanHost(const HostPlan &hp, const GreenInput &in, const LayerModel &lm)
     {
         nitems = (int)hp.rho.size();
         nmerged = (int)hp.merged.size();
@@ -629,35 +762,39 @@ struct PlanHost {
         std::vector<double> flat((size_t)nitems * nlam_max, 0.0);
         for (int it = 0; it < nitems; ++it) std::copy(hp.lam[it].begin(), hp.lam[it].end(), flat.begin() + (size_t)it * nlam_max);
         at[0] = pack.add(nlam);
-        at[1] = pack.add(hp.m_item);
-        at[2] = pack.add(hp.m_idx);
-        at[3] = pack.add(flat);
-        at[4] = pack.add(hp.merged);
-        at[5] = pack.add(in.hank0);
-        at[6] = pack.add(in.hank1);
-        auxn = (size_t)nitems * nlam_max * nl;
+        nrho_max = nlam_max - kTaps;
+        std::vector<int> mpos((size_t)nitems * nrho_max, 0);
+        for (int k = 0; k < nmerged; ++k)
+            if (hp.m_item[k] >= 0) mpos[(size_t)hp.m_item[k] * nrho_max + hp.m_idx[k]] = k;
+        at[1] = pack.add(mpos);
+        at[2] = pack.add(flat);
+        at[3] = pack.add(hp.merged);
+        at[4] = pack.add(in.hank0);
+        at[5] = pack.add(in.hank1);
+        at[6] = pack.add(std::vector<LayerModel>{lm});
+        auxn = (size_t)nitems * nlam_max * lm.nl;
     }
     size_t device_bytes() const
     {
         return GreenScratch::padded(pack.bytes.size()) + 6 * GreenScratch::padded(auxn * sizeof(double2));
     }
     // uploads the pack (its device address into base) and runs the recursions; the pack must outlive them
-    PlanDev upload(GreenScratch &work, const LayerModel &lm, unsigned char *&base, hipStream_t s) const
+    PlanDev upload(GreenScratch &work, unsigned char *&base, hipStream_t s) const
     {
         base = work.take<unsigned char>(pack.bytes.size());
         XTR_CHECK(hipMemcpyAsync(base, pack.bytes.data(), pack.bytes.size(), hipMemcpyHostToDevice, s));
         PlanDev d;
         d.nlam = (const int *)(base + at[0]);
-        d.mitem = (const int *)(base + at[1]);
-        d.midx = (const int *)(base + at[2]);
-        d.lam = (const double *)(base + at[3]);
-        d.radii = (const double *)(base + at[4]);
-        d.h0 = (const double *)(base + at[5]);
-        d.h1 = (const double *)(base + at[6]);
+        d.mpos = (const int *)(base + at[1]);
+        d.lam = (const double *)(base + at[2]);
+        d.radii = (const double *)(base + at[3]);
+        d.h0 = (const double *)(base + at[4]);
+        d.h1 = (const double *)(base + at[5]);
+        d.lm = (const LayerModel *)(base + at[6]);
         double2 **aux[6] = {&d.eta, &d.ex, &d.p1, &d.q1, &d.ps, &d.qs};
         for (auto *a : aux) *a = work.take<double2>(auxn);
         dim3 grid((unsigned)ceil_div(nlam_max, 128), nitems);
-        hipLaunchKernelGGL(layer_aux_kernel, grid, dim3(128), 0, s, lm, nitems, nlam_max, d.nlam, d.lam, d.eta, d.ex,
+        hipLaunchKernelGGL(layer_aux_kernel, grid, dim3(128), 0, s, d.lm, nitems, nlam_max, d.nlam, d.lam, d.eta, d.ex,
                            d.p1, d.q1, d.ps, d.qs);
         XTR_LAUNCH_CHECK("layer_aux_kernel");
         return d;
@@ -692,9 +829,9 @@ int layer_at_depth(const Section &s, double depth)   // ScalarMathUtils.cs:15-31
 
 }  // namespace
 
-// The pairs of one set pass through the stages in chunks whose U stays in the 256 MB Infinity Cache between
-// pair_u and hankel, which also bounds the scratch (about 130 MB) whatever nz.
-constexpr size_t kChunkBytes = (size_t)64 << 20;
+// The pairs of one set pass through the stages in equal chunks whose U stays in the 256 MB Infinity Cache
+// between pair_u and hankel, which also bounds the scratch (about 250 MB) whatever nz.
+constexpr size_t kChunkBytes = (size_t)160 << 20;
 
 void build_green_atoa(const GreenInput &in, GreenScratch &work, double2 *G, bool folded, const double2 *tw_x,
                       const double2 *tw_y, hipStream_t s)
@@ -703,7 +840,7 @@ void build_green_atoa(const GreenInput &in, GreenScratch &work, double2 *G, bool
     const int nz = g.nz;
     const LayerModel lm = layer_model(in);
     const HostPlan hp = make_plan(in);
-    PlanHost ph(hp, in, lm.nl);
+    PlanHost ph(hp, in, lm);
 
     // transceiver pairs: Combine (rc-major) for asym, CombineSymm (tr-major, rc <= tr) for symm
     std::vector<PairInfo> pairs[2];
@@ -734,7 +871,8 @@ void build_green_atoa(const GreenInput &in, GreenScratch &work, double2 *G, bool
         pairs_at[asym] = ph.pack.add(pairs[asym]);
         const int np = (int)pairs[asym].size(), ncomp = asym ? 1 : 3;
         const size_t u1 = (size_t)ph.nitems * ncomp * ph.nlam_max;     // U of one pair
-        chunk[asym] = (int)std::min<size_t>(np, std::max<size_t>(1, kChunkBytes / (u1 * sizeof(double2)) / 256) * 256);
+        const int64_t chunks = ceil_div((int64_t)(np * u1 * sizeof(double2)), (int64_t)kChunkBytes);
+        chunk[asym] = (int)std::min<int64_t>(np, ceil_div(ceil_div(np, chunks), 8) * 8);   // 8 rows a wave of hankel
         need[0] = std::max(need[0], chunk[asym] * u1);
         need[1] = std::max(need[1], (size_t)chunk[asym] * ncomp * ph.nmerged);
         need[2] = need[3] = need[1];
@@ -743,26 +881,24 @@ void build_green_atoa(const GreenInput &in, GreenScratch &work, double2 *G, bool
     for (size_t n : need) bytes += GreenScratch::padded(n * sizeof(double2));
     work.reserve(bytes);
     unsigned char *base;
-    const PlanDev d = ph.upload(work, lm, base, s);
+    const PlanDev d = ph.upload(work, base, s);
     double2 *U = work.take<double2>(need[0]), *I = work.take<double2>(need[1]), *segA = work.take<double2>(need[2]),
             *segB = work.take<double2>(need[3]);
     if (!folded) XTR_CHECK(hipMemsetAsync(G, 0, (size_t)g.L() * g.gblk() * sizeof(double2), s));
 
-    const int nitems = ph.nitems, nlam_max = ph.nlam_max, nmerged = ph.nmerged, nseg = nmerged - 1;
+    const int nitems = ph.nitems, nlam_max = ph.nlam_max, nmerged = ph.nmerged;
     for (int asym = 1; asym >= 0; --asym) {
         const int ncomp = asym ? 1 : 3, all = (int)pairs[asym].size();
         for (int p0 = 0; p0 < all; p0 += chunk[asym]) {
             const int np = std::min(chunk[asym], all - p0);
             const PairInfo *dp = (const PairInfo *)(base + pairs_at[asym]) + p0;
-            hipLaunchKernelGGL(pair_u_kernel, dim3((unsigned)ceil_div(nlam_max, 64), nitems, np), dim3(64), 0, s, lm, np,
+            hipLaunchKernelGGL(pair_u_kernel, dim3((unsigned)ceil_div(nlam_max, 64), nitems, np), dim3(64), 0, s, d.lm, np,
                                dp, asym, nitems, nlam_max, d.nlam, d.lam, d.eta, d.ex, d.p1, d.q1, d.ps, d.qs, U);
             XTR_LAUNCH_CHECK("pair_u_kernel");
-            hipLaunchKernelGGL(hankel_kernel, dim3((unsigned)ceil_div(nmerged, 128), np, ncomp), dim3(128), 0, s, np,
-                               nitems, ncomp, nlam_max, U, nmerged, d.mitem, d.midx, d.radii, d.h0, d.h1, asym, I);
-            XTR_LAUNCH_CHECK("hankel_kernel");
-            hipLaunchKernelGGL(segments_kernel, dim3((unsigned)ceil_div(np, 128), ncomp, nseg), dim3(128), 0, s, np,
-                               ncomp, nmerged, d.radii, I, segA, segB);
-            XTR_LAUNCH_CHECK("segments_kernel");
+            // I3 with J0; I1, I2, I5 with J1, I1 negated (HankelCoefficients.cs:103-118, ScalarMathUtils.cs:189-241)
+            launch_hankel(HankelArgs{np, nitems, ncomp, nlam_max, ph.nrho_max, U, d.nlam, d.mpos, d.radii, d.h0, d.h1,
+                                     asym, {asym ? 1.0 : -1.0, 1, 1, 1, 1}, 2 * kPi, I}, s);
+            launch_segments(ncomp, np, nmerged, d.radii, I, segA, segB, s);
             LatArgs la{};
             la.nx = g.nx;
             la.ny = g.ny;
@@ -770,7 +906,6 @@ void build_green_atoa(const GreenInput &in, GreenScratch &work, double2 *G, bool
             la.npairs = np;
             la.p0 = p0;
             la.folded = folded ? 1 : 0;
-            la.asym = asym;
             la.nr = nmerged;
             la.dx = in.dx;
             la.dy = in.dy;
@@ -789,8 +924,10 @@ void build_green_atoa(const GreenInput &in, GreenScratch &work, double2 *G, bool
                 for (int t = 0; t < 3; ++t) { la.xs[t] = 1; la.ys[t] = 1; }
                 la.xs[3] = -1; la.ys[3] = -1;
             }
-            dim3 grid((unsigned)((int64_t)g.nx * g.ny), (unsigned)ceil_div(np, 256));
-            hipLaunchKernelGGL(lateral_kernel, grid, dim3(std::min(256, ((np + 63) / 64) * 64)), 0, s, la);
+            const int wgs = (int)ceil_div(np, 256);                  // of a cell, with equal shares of the pairs
+            const dim3 grid((unsigned)((int64_t)g.nx * g.ny), wgs), nt((unsigned)(ceil_div(ceil_div(np, wgs), 64) * 64));
+            if (asym) hipLaunchKernelGGL(lateral_kernel<1>, grid, nt, 0, s, la);
+            else hipLaunchKernelGGL(lateral_kernel<0>, grid, nt, 0, s, la);
             XTR_LAUNCH_CHECK("lateral_kernel");
         }
     }
@@ -839,7 +976,7 @@ __device__ inline double2 dbot_(const LayerModel &lm, const double2 *E, int r, i
 // :58-108, VolumeToPointCalculatorU.cs:34-337, ScalarMathUtils.NormalizeBeforeHankelForE/H).
 // electric: comps I1..I5 <- U1 (A1 set) * i w mu0 / 2, U2 / 2z, U3 l / 2z, U4 (-l) / 2z, U5 l^2 / 2z
 // magnetic: comps I1..I4 <- U31, U4Sigma, U1Sigma * l, U11 * l
-__global__ void point_u_kernel(LayerModel lm, int nz, const PointInfo *pts, int electric, int nitems, int nlam_max,
+__global__ __launch_bounds__(64) void point_u_kernel(const LayerModel *lmp, int nz, const PointInfo *pts, int electric, int nitems, int nlam_max,
                                const int *nlam, const double *lam, const double2 *eta, const double2 *ex,
                                const double2 *p1, const double2 *q1, const double2 *ps, const double2 *qs,
                                double2 *U)
@@ -849,6 +986,7 @@ __global__ void point_u_kernel(LayerModel lm, int nz, const PointInfo *pts, int 
     const int tr = blockIdx.z;
     if (it >= nitems || m >= nlam[it] || tr >= nz) return;
     const PointInfo pi = pts[tr];
+    const LayerModel &lm = *lmp;
     const int nl = lm.nl;
     const int64_t base = ((int64_t)it * nlam_max + m) * nl;
     const double2 *E = eta + base, *X = ex + base;
@@ -920,185 +1058,109 @@ __global__ void point_u_kernel(LayerModel lm, int nz, const PointInfo *pts, int 
     }
 }
 
-// Hankel filter in the non-fast order of HankelCoefficients.ConvoluteWith (:86-99) and
-// NormalizeAfterHankelForE/H (ScalarMathUtils.cs:131-155): comp c uses J1 or J0 and the factor
-// sign / (den rho). electric: J1 -, J1 +, J0 +, J0 +, J1 + with den 2 pi; magnetic: J1 -, J1 -,
-// J0 -, J0 + with den 4 pi.
-__device__ inline double2 atoo_hankel_at(int nitems, int ncomp, int nlam_max, const double2 *U, int tr, int it,
-                                         int idx, int c, double rho, const double *hank0, const double *hank1,
-                                         int electric)
+// The zero-rho point (CalculateZeroRhoForE/H, ScalarMathUtils.cs:33-81), radius 0 of the merged ones: I1, I2
+// (and I5) are 0 there, I3 and I4 are (f[1] a^2 - f[2]) / (a^2 - 1) from the first item's 2nd and 3rd radii (at
+// k1, k2), a the rho step.
+__global__ void zero_rho_kernel(int nz, int ncomp, int k1, int k2, double alpha2, double2 *I)
 {
-    const bool j0 = c == 2 || c == 3;
-    const double *hank = j0 ? hank0 : hank1;
-    const double sgn = electric ? (c == 0 ? -1.0 : 1.0) : (c == 3 ? 1.0 : -1.0);
-    const double den = (electric ? 2 * kPi : 4 * kPi) * rho;
-    const double2 *f = U + (((int64_t)tr * nitems + it) * ncomp + c) * nlam_max + idx;
-    double re = 0, im = 0;
-    for (int j = 0; j < kTaps; ++j) {
-        const double h = hank[j];
-        const double2 v = f[kTaps - 1 - j];
-        re += v.x * h;
-        im += v.y * h;
-    }
-    return make_double2(sgn * re / den, sgn * im / den);
-}
-
-// A merged radius with item -1 is the zero-rho point (CalculateZeroRhoForE/H, ScalarMathUtils.cs:33-81):
-// I1, I2 (and I5) are 0 there, I3 and I4 are (f[1] a^2 - f[2]) / (a^2 - 1) from the first item's 2nd and
-// 3rd radii rho01, rho02, a the rho step.
-__global__ void atoo_hankel_kernel(int nz, int nitems, int ncomp, int nlam_max, const double2 *U, int nmerged,
-                                   const int *m_item, const int *m_idx, const double *radii, const double *hank0,
-                                   const double *hank1, int electric, double rho01, double rho02, double alpha2,
-                                   double2 *I)
-{
-    const int k = blockIdx.x * blockDim.x + threadIdx.x;
-    const int tr = blockIdx.y;
-    const int c = blockIdx.z;
-    if (k >= nmerged || tr >= nz || c >= ncomp) return;
-    const int it = m_item[k], idx = m_idx[k];
-    double2 v;
-    if (it >= 0) {
-        v = atoo_hankel_at(nitems, ncomp, nlam_max, U, tr, it, idx, c, radii[k], hank0, hank1, electric);
-    } else if (c == 2 || c == 3) {
-        const double2 f1 = atoo_hankel_at(nitems, ncomp, nlam_max, U, tr, 0, 1, c, rho01, hank0, hank1, electric);
-        const double2 f2 = atoo_hankel_at(nitems, ncomp, nlam_max, U, tr, 0, 2, c, rho02, hank0, hank1, electric);
+    const int e = blockIdx.x * blockDim.x + threadIdx.x;
+    if (e >= ncomp * nz) return;
+    const int c = e / nz;
+    double2 v = make_double2(0, 0);
+    if (c == 2 || c == 3) {
+        const double2 f1 = I[(int64_t)k1 * ncomp * nz + e], f2 = I[(int64_t)k2 * ncomp * nz + e];
         v = make_double2((f1.x * alpha2 - f2.x) / (alpha2 - 1), (f1.y * alpha2 - f2.y) / (alpha2 - 1));
-    } else {
-        v = make_double2(0, 0);
     }
-    I[((int64_t)c * nz + tr) * nmerged + k] = v;
+    I[e] = v;
 }
 
 struct AoArgs {
-    int nx, ny, nz, nr, electric, ncomp, ntc;
+    int nx, ny, nz, nr;
     double dx, dy;
     double xs, ys;                // minus the level's shift (AtoOLevelGreenTensorCalculator.cs:119-125)
     const double2 *segA, *segB;   // [seg][comp][tr]
     const double *radii;
-    double2 *G;                   // [2Nx][2Ny][ntc][nz]
-    int slot[AO_N];               // compact component index of each slot, -1 if not computed
+    double2 *G;                   // [2Nx][2Ny][components][nz], components as in atoo_components
 };
 
-struct Q9 { double2 q[AO_N]; };
+// One wave per lateral offset (i, j) in (-Nx, Nx) x (-Ny, Ny), lanes the transmitter layers: the four edge
+// integrals of RunAlongX / RunAlongY (GreenTensorCalculator.cs:192-281), written at TransformI/J
+// (AtoOLevelGreenTensorCalculator.cs:106-117). The wave forms its offset's weights itself (CellWeights), 8 segments
+// at a time, a thread for each (segment, stretch). At 128 x 128 x 32: 0.26 and 0.22 ms; 0.64 ms each with every
+// thread working out the geometry.
+constexpr int kAoWaves = 4, kAoSegs = 8;
 
-// AddToQBuffAlong{X,Y}{Electric,Magnetic} (GreenTensorCalculator.cs:505-560); comps I1..I5 at 0..4
-__device__ inline void ao_add(const AoArgs &a, int tr, const Factors &f, int seg, bool alongY, Q9 &Q)
+template <int ELECTRIC>
+__global__ __launch_bounds__(64 * kAoWaves) void atoo_lateral_kernel(AoArgs a)
 {
-    auto A = [&](int ic) { return a.segA[((int64_t)seg * a.ncomp + (ic - 1)) * a.nz + tr]; };
-    auto B = [&](int ic) { return a.segB[((int64_t)seg * a.ncomp + (ic - 1)) * a.nz + tr]; };
-    auto add = [&](int slot, int ic, double da, double db) {
-        Q.q[slot] = Q.q[slot] + da * A(ic);
-        Q.q[slot] = Q.q[slot] + db * B(ic);
-    };
-    if (a.electric) {
-        if (!alongY) {
-            add(AO_XX, 1, f.d2a, f.d2b); add(AO_YY, 2, f.d2a, f.d2b); add(AO_ZZ, 5, f.d2a, f.d2b);
-            add(AO_XY, 2, f.d3a, f.d3b); add(AO_YZ, 3, f.d1a, f.d1b); add(AO_ZY, 4, f.d1a, f.d1b);
-        } else {
-            add(AO_XX, 2, f.d2a, f.d2b); add(AO_YY, 1, f.d2a, f.d2b); add(AO_ZZ, 5, f.d2a, f.d2b);
-            add(AO_XY, 1, f.d3a, f.d3b); add(AO_XZ, 3, f.d1a, f.d1b); add(AO_ZX, 4, f.d1a, f.d1b);
-        }
-    } else {
-        if (!alongY) {
-            add(AO_XX, 2, f.d3a, f.d3b); add(AO_YX, 1, f.d2a, f.d2b); add(AO_XY, 2, f.d2a, f.d2b);
-            add(AO_XZ, 3, f.d1a, f.d1b); add(AO_ZX, 4, f.d1a, f.d1b);
-        } else {
-            add(AO_YX, 2, f.d2a, f.d2b); add(AO_XY, 1, f.d2a, f.d2b); add(AO_XX, 1, f.d3a, f.d3b);
-            add(AO_YZ, 3, f.d1a, f.d1b); add(AO_ZY, 4, f.d1a, f.d1b);
-        }
-    }
-}
-
-__device__ inline Q9 ao_integrate(const AoArgs &a, int tr, Knot left, Knot right, double s, double u, double v,
-                                  bool alongY)
-{
-    Q9 Q;
-    for (int t = 0; t < AO_N; ++t) Q.q[t] = c_(0);
-    const int i1 = left.index, i2 = right.index;
-    if (i1 == i2) {
-        ao_add(a, tr, factors(s, u, left.radius, right.radius, v), i1, alongY, Q);
-        return Q;
-    }
-    double r1 = left.radius, r2 = a.radii[i1 + 1];
-    double sj = s, uj = sqrt(r2 * r2 - v * v);
-    ao_add(a, tr, factors(sj, uj, r1, r2, v), i1, alongY, Q);
-    for (int i = i1 + 1; i < i2; ++i) {
-        r1 = r2;
-        r2 = a.radii[i + 1];
-        sj = uj;
-        uj = sqrt(r2 * r2 - v * v);
-        ao_add(a, tr, factors(sj, uj, r1, r2, v), i, alongY, Q);
-    }
-    sj = uj; uj = u; r1 = r2; r2 = right.radius;
-    ao_add(a, tr, factors(sj, uj, r1, r2, v), i2, alongY, Q);
-    return Q;
-}
-
-// QSigns (QSign.cs:31-38) by slot; rows AlongX, AlongY, AlongXSymm, AlongYSymm
-__constant__ int kQsE[4][AO_N] = {{1, -1, -1, -1, 0, 1, 1, 1, 1},
-                                  {-1, 1, -1, -1, 0, 1, 1, 1, 1},
-                                  {1, -1, -1, 1, 0, -1, 1, -1, 1},
-                                  {-1, 1, -1, 1, 0, 1, -1, 1, -1}};
-__constant__ int kQsH[4][AO_N] = {{-1, -1, 0, -1, 1, 1, 1, 1, 1},
-                                  {-1, -1, 0, 1, -1, 1, 1, 1, 1},
-                                  {1, 1, 0, -1, 1, 1, -1, 1, -1},
-                                  {1, 1, 0, 1, -1, 1, 1, -1, 1}};
-
-__device__ inline void ao_fill(const AoArgs &a, Q9 &G, const Q9 &Q, int sign, int qsel)
-{
-    for (int t = 0; t < AO_N; ++t) {
-        const int qs = a.electric ? kQsE[qsel][t] : kQsH[qsel][t];
-        G.q[t] = G.q[t] + (double)(sign * qs) * Q.q[t];
-    }
-}
-
-// One thread per (lateral offset (i, j) in (-Nx, Nx) x (-Ny, Ny), transmitter layer): the four edge
-// integrals of RunAlongX / RunAlongY (GreenTensorCalculator.cs:192-281) that FillResultAlongX/Y
-// (:413-437) add into this offset, written at TransformI/J (AtoOLevelGreenTensorCalculator.cs:106-117).
-__global__ __launch_bounds__(64) void atoo_lateral_kernel(AoArgs a)
-{
-    const int ncy = 2 * a.ny - 1;
-    const int cell = blockIdx.x;
+    __shared__ CellWeights<kAoSegs> all[kAoWaves];
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    CellWeights<kAoSegs> &cw = all[wave];
+    const int ncy = 2 * a.ny - 1, cells = (2 * a.nx - 1) * ncy;
+    const int cell = blockIdx.x * kAoWaves + wave;
+    if (cell >= cells) return;                                  // waves do not meet at a barrier
     const int i = cell / ncy - (a.nx - 1), j = cell % ncy - (a.ny - 1);
-    const int tr = blockIdx.y * blockDim.x + threadIdx.x;
-    if (tr >= a.nz) return;
-    const double dx = a.dx, dy = a.dy;
-    Q9 G;
-    for (int t = 0; t < AO_N; ++t) G.q[t] = c_(0);
-    for (int e = 0; e < 2; ++e) {     // edges along x at y = dy (jj - 1/2) - ys: jj = j (-1), j + 1 (+1)
-        const int jj = j + e, sign = e == 0 ? -1 : 1;
-        const double y = dy * (jj - 0.5) - a.ys;
-        const double x1 = dx * (i - 0.5) - a.xs, x2 = dx * (i + 0.5) - a.xs;
-        const Knot kl = make_knot(a.radii, a.nr, x1, y), kr = make_knot(a.radii, a.nr, x2, y);
-        if (x1 > 0 && x2 > 0) {
-            ao_fill(a, G, ao_integrate(a, tr, kl, kr, x1, x2, y, false), sign, 0);
-        } else if (x1 < 0 && x2 < 0) {
-            ao_fill(a, G, ao_integrate(a, tr, kr, kl, -x2, -x1, y, false), sign, 2);
-        } else {
-            const Knot kz = make_knot(a.radii, a.nr, 0, y);
-            ao_fill(a, G, ao_integrate(a, tr, kz, kl, 0, -x1, y, false), sign, 2);
-            ao_fill(a, G, ao_integrate(a, tr, kz, kr, 0, x2, y, false), sign, 0);
-        }
-    }
-    for (int e = 0; e < 2; ++e) {     // edges along y at x = dx (ii - 1/2) - xs: ii = i (-1), i + 1 (+1)
-        const int ii = i + e, sign = e == 0 ? -1 : 1;
-        const double x = dx * (ii - 0.5) - a.xs;
-        const double y1 = dy * (j - 0.5) - a.ys, y2 = dy * (j + 0.5) - a.ys;
-        const Knot kl = make_knot(a.radii, a.nr, x, y1), kr = make_knot(a.radii, a.nr, x, y2);
-        if (y1 > 0 && y2 > 0) {
-            ao_fill(a, G, ao_integrate(a, tr, kl, kr, y1, y2, x, true), sign, 1);
-        } else if (y1 < 0 && y2 < 0) {
-            ao_fill(a, G, ao_integrate(a, tr, kr, kl, -y2, -y1, x, true), sign, 3);
-        } else {
-            const Knot kz = make_knot(a.radii, a.nr, x, 0);
-            ao_fill(a, G, ao_integrate(a, tr, kz, kl, 0, -y1, x, true), sign, 3);
-            ao_fill(a, G, ao_integrate(a, tr, kz, kr, 0, y2, x, true), sign, 1);
-        }
-    }
+    // LDS writes of this wave become visible to it in order; the fence only keeps the compiler from moving them
+    auto sync = [] { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); __builtin_amdgcn_wave_barrier(); };
+    cw.ends(lane, a.radii, a.nr, a.dx * (i - 0.5) - a.xs, a.dx * (i + 0.5) - a.xs, a.dy * (j - 0.5) - a.ys,
+            a.dy * (j + 0.5) - a.ys);
+    sync();
+    int lo, hi;
+    cw.range(lo, hi);
+    constexpr int nc = ELECTRIC ? 5 : 4, no = ELECTRIC ? 8 : 7;
     const int64_t ti = i < 0 ? 2 * a.nx + i : i, tj = j < 0 ? 2 * a.ny + j : j;
-    double2 *dst = a.G + (ti * 2 * a.ny + tj) * (int64_t)(a.ntc * a.nz) + tr;
-    for (int t = 0; t < AO_N; ++t)
-        if (a.slot[t] >= 0) dst[(int64_t)a.slot[t] * a.nz] = G.q[t];
+    for (int tr0 = 0; tr0 < a.nz; tr0 += 64) {
+        const int tr = tr0 + lane;
+        double2 G[no];
+#pragma unroll
+        for (int t = 0; t < no; ++t) G[t] = c_(0);
+        for (int seg0 = lo; seg0 <= hi; seg0 += kAoSegs) {
+            const int n = min(kAoSegs, hi - seg0 + 1);
+            cw.factors_of(lane, 64, a.radii, seg0, n);
+            sync();
+            cw.sum(lane, 64, n);
+            sync();
+            if (tr < a.nz)
+                for (int k = 0; k < n; ++k) {
+                    const double (&wx)[WN] = cw.w[k][0], (&wy)[WN] = cw.w[k][1];
+                    const double2 *A = a.segA + (int64_t)(seg0 + k) * nc * a.nz + tr;
+                    const double2 *B = a.segB + (int64_t)(seg0 + k) * nc * a.nz + tr;
+                    double2 sa[nc], sb[nc];                     // I1 .. I5 (I4)
+#pragma unroll
+                    for (int c = 0; c < nc; ++c) {
+                        sa[c] = A[(int64_t)c * a.nz];
+                        sb[c] = B[(int64_t)c * a.nz];
+                    }
+                    // AddToQBuffAlong{X,Y}{Electric,Magnetic} (GreenTensorCalculator.cs:505-560) with the signs of the
+                    // QSigns tables (QSign.cs:31-38)
+                    const double nxw[WN] = {0, 0, -wx[W2A], -wx[W2B], 0, 0}, nyw[WN] = {0, 0, -wy[W2A], -wy[W2B], 0, 0};
+                    if constexpr (ELECTRIC) {                   // xx yy zz xy xz yz zx zy
+                        G[0] = wab(nyw, W2A, wab(wx, W2A, G[0], sa[0], sb[0]), sa[1], sb[1]);
+                        G[1] = wab(nxw, W2A, wab(wy, W2A, G[1], sa[0], sb[0]), sa[1], sb[1]);
+                        G[2] = wab(nyw, W2A, wab(nxw, W2A, G[2], sa[4], sb[4]), sa[4], sb[4]);
+                        G[3] = wab(wy, W3A, wab(wx, W3A, G[3], sa[1], sb[1]), sa[0], sb[0]);
+                        G[4] = wab(wy, W1A, G[4], sa[2], sb[2]);
+                        G[5] = wab(wx, W1A, G[5], sa[2], sb[2]);
+                        G[6] = wab(wy, W1A, G[6], sa[3], sb[3]);
+                        G[7] = wab(wx, W1A, G[7], sa[3], sb[3]);
+                    } else {                                    // xx xy yx xz yz zx zy
+                        G[0] = wab(wy, W3A, wab(wx, W3A, G[0], sa[1], sb[1]), sa[0], sb[0]);
+                        G[1] = wab(wy, W2A, wab(nxw, W2A, G[1], sa[1], sb[1]), sa[0], sb[0]);
+                        G[2] = wab(nyw, W2A, wab(wx, W2A, G[2], sa[0], sb[0]), sa[1], sb[1]);
+                        G[3] = wab(wx, W1A, G[3], sa[2], sb[2]);
+                        G[4] = wab(wy, W1A, G[4], sa[2], sb[2]);
+                        G[5] = wab(wx, W1A, G[5], sa[3], sb[3]);
+                        G[6] = wab(wy, W1A, G[6], sa[3], sb[3]);
+                    }
+                }
+            sync();                                             // the weights are read
+        }
+        if (tr < a.nz) {
+            double2 *dst = a.G + (ti * 2 * a.ny + tj) * (int64_t)(no * a.nz) + tr;
+#pragma unroll
+            for (int t = 0; t < no; ++t) dst[(int64_t)t * a.nz] = G[t];
+        }
+    }
 }
 
 }  // namespace
@@ -1121,7 +1183,7 @@ void build_green_atoo_level(const GreenInput &in, GreenScratch &work, double lev
     // the level's own scalar plan (AtoOCalculator.cs:129, 151)
     const HostPlan hp = make_level_plan(in, shift_x, shift_y);
     if (hp.zero_rho && hp.rho[0].size() < 3) throw hip_error("zero-rho plan needs three radii in its first item");
-    PlanHost ph(hp, in, lm.nl);
+    PlanHost ph(hp, in, lm);
     const int nitems = ph.nitems, nlam_max = ph.nlam_max, nmerged = ph.nmerged;
     // transmitters: the anomaly layers; receiver: the level point (AuxContainer.CreateContainer)
     const int r = layer_at_depth(in.section, level_z);
@@ -1149,29 +1211,40 @@ void build_green_atoo_level(const GreenInput &in, GreenScratch &work, double lev
     for (size_t n : need) bytes += GreenScratch::padded(n * sizeof(double2));
     work.reserve(bytes);
     unsigned char *base;
-    const PlanDev d = ph.upload(work, lm, base, s);
+    const PlanDev d = ph.upload(work, base, s);
     double2 *U = work.take<double2>(need[0]), *I = work.take<double2>(need[1]), *segA = work.take<double2>(need[2]),
             *segB = work.take<double2>(need[3]);
-    hipLaunchKernelGGL(point_u_kernel, dim3((unsigned)ceil_div(nlam_max, 64), nitems, nz), dim3(64), 0, s, lm, nz,
+    hipLaunchKernelGGL(point_u_kernel, dim3((unsigned)ceil_div(nlam_max, 64), nitems, nz), dim3(64), 0, s, d.lm, nz,
                        (const PointInfo *)(base + pts_at), electric, nitems, nlam_max, d.nlam, d.lam, d.eta, d.ex, d.p1,
                        d.q1, d.ps, d.qs, U);
     XTR_LAUNCH_CHECK("point_u_kernel");
-    hipLaunchKernelGGL(atoo_hankel_kernel, dim3((unsigned)ceil_div(nmerged, 128), nz, ncomp), dim3(128), 0, s, nz,
-                       nitems, ncomp, nlam_max, U, nmerged, d.mitem, d.midx, d.radii, d.h0, d.h1, electric,
-                       hp.zero_rho ? hp.rho[0][1] : 0.0, hp.zero_rho ? hp.rho[0][2] : 0.0,
-                       log10_rho_step() * log10_rho_step(), I);
-    XTR_LAUNCH_CHECK("atoo_hankel_kernel");
-    hipLaunchKernelGGL(segments_kernel, dim3((unsigned)ceil_div(nz, 128), ncomp, nseg), dim3(128), 0, s, nz, ncomp,
-                       nmerged, d.radii, I, segA, segB);
-    XTR_LAUNCH_CHECK("segments_kernel");
+    // HankelCoefficients.ConvoluteWith (:86-99), NormalizeAfterHankelForE/H (ScalarMathUtils.cs:131-155): electric
+    // J1 -, J1 +, J0 +, J0 +, J1 + over 2 pi rho; magnetic J1 -, J1 -, J0 -, J0 + over 4 pi rho
+    HankelArgs ha{nz, nitems, ncomp, nlam_max, ph.nrho_max, U, d.nlam, d.mpos, d.radii, d.h0, d.h1, 0xc,
+                  {-1, 1, 1, 1, 1}, 2 * kPi, I};
+    if (!electric) {
+        ha.sgn[1] = ha.sgn[2] = -1;
+        ha.den = 4 * kPi;
+    }
+    launch_hankel(ha, s);
+    if (hp.zero_rho) {
+        const auto place = [&](int ix) {
+            for (int k = 0; k < nmerged; ++k)
+                if (hp.m_item[k] == 0 && hp.m_idx[k] == ix) return k;
+            throw hip_error("zero-rho plan: radius not found");
+        };
+        hipLaunchKernelGGL(zero_rho_kernel, dim3((unsigned)ceil_div(ncomp * nz, 256)), dim3(256), 0, s, nz, ncomp, place(1),
+                           place(2), log10_rho_step() * log10_rho_step(), I);
+        XTR_LAUNCH_CHECK("zero_rho_kernel");
+    }
+    launch_segments(ncomp, nz, nmerged, d.radii, I, segA, segB, s);
+    int slot[9];
+    const int ntc = atoo_components(electric, slot);
     AoArgs a{};
     a.nx = g.nx;
     a.ny = g.ny;
     a.nz = nz;
     a.nr = nmerged;
-    a.electric = electric;
-    a.ncomp = ncomp;
-    a.ntc = atoo_components(electric, a.slot);
     a.dx = in.dx;
     a.dy = in.dy;
     a.xs = -shift_x;
@@ -1180,13 +1253,12 @@ void build_green_atoo_level(const GreenInput &in, GreenScratch &work, double lev
     a.segB = segB;
     a.radii = d.radii;
     a.G = G;
-    XTR_CHECK(hipMemsetAsync(G, 0, (size_t)g.L() * a.ntc * nz * sizeof(double2), s));
-    {
-        dim3 grid((unsigned)((2 * g.nx - 1) * (2 * g.ny - 1)), (unsigned)ceil_div(nz, 64));
-        hipLaunchKernelGGL(atoo_lateral_kernel, grid, dim3(64), 0, s, a);
-        XTR_LAUNCH_CHECK("atoo_lateral_kernel");
-    }
-    launch_fft2_plain(G, 2 * g.nx, 2 * g.ny, (int64_t)a.ntc * nz, tw_x, tw_y, -1, s);
+    XTR_CHECK(hipMemsetAsync(G, 0, (size_t)g.L() * ntc * nz * sizeof(double2), s));
+    const dim3 grid((unsigned)ceil_div((2 * g.nx - 1) * (2 * g.ny - 1), kAoWaves)), nt(64 * kAoWaves);
+    if (electric) hipLaunchKernelGGL(atoo_lateral_kernel<1>, grid, nt, 0, s, a);
+    else hipLaunchKernelGGL(atoo_lateral_kernel<0>, grid, nt, 0, s, a);
+    XTR_LAUNCH_CHECK("atoo_lateral_kernel");
+    launch_fft2_plain(G, 2 * g.nx, 2 * g.ny, (int64_t)ntc * nz, tw_x, tw_y, -1, s);
     XTR_CHECK(hipStreamSynchronize(s));   // the host pack is freed on return
 }
 

@@ -36,12 +36,18 @@ void launch_fft2_plain(double2 *data, int n1, int n2, int64_t ncols, const doubl
 // nor the fold after. With the scratch kept on the handle calculate_green_tensor and one chi0 apply there
 // take 8.5 ms instead of 15 ms when hipMalloc was quick and 160-190 ms when it was not.
 struct IoMirror : IoPlain<double> {
-    int64_t gblk, S, A;
+    int gblk, S, A;
     int half, axis;           // axis 0: x, 1: y
+    // columns and blocks fit 32 bits (a division of 64 takes several times the instructions)
+    __device__ int64_t at(int64_t c, int p) const
+    {
+        const unsigned col = (unsigned)c, per = (unsigned)cpr, row = col / per;
+        return row * row_stride + (col - row * per) + p * pstride;
+    }
     // xy is odd in x and y, xz in x, yz in y
     __device__ double sign(int64_t c) const
     {
-        const int64_t o = c % gblk;
+        const int o = (int)((unsigned)c % (unsigned)gblk);
         const int xy = (int)(o >= S) & (int)(o < 2 * S), xz = (int)(o >= 4 * S) & (int)(o < 4 * S + A),
                   yz = (int)(o >= 4 * S + A);
         return (xy | (axis == 0 ? xz : yz)) ? -1.0 : 1.0;
@@ -49,21 +55,22 @@ struct IoMirror : IoPlain<double> {
     __device__ double2 load(int, int64_t c, int p) const
     {
         if (c >= ncols || p == half) return make_double2(0, 0);
-        const double2 v = buf[addr(0, c, p < half ? p : 2 * half - p)];
+        const double2 v = buf[at(c, p < half ? p : 2 * half - p)];
         const double s = p < half ? 1.0 : sign(c);
         return make_double2(s * v.x, s * v.y);
     }
     __device__ void store(int, int64_t c, int p, double2 v) const
     {
-        if (c < ncols && p <= half) buf[addr(0, c, p)] = v;
+        if (c < ncols && p <= half) buf[at(c, p)] = v;
     }
 };
 
 void launch_fft2_mirror(double2 *folded, const Geom &g, const double2 *tw_x, const double2 *tw_y, hipStream_t s)
 {
-    const int64_t gb = g.gblk(), S = g.S(), A = (int64_t)g.nz * g.nz, row = (g.ny + 1) * gb;
-    const IoMirror y{{folded, 0, g.nx * gb, gb, row, gb, 0, 0}, gb, S, A, g.ny, 1};
-    const IoMirror x{{folded, 0, row, row, 0, row, 0, 0}, gb, S, A, g.nx, 0};
+    const int64_t gb = g.gblk(), row = (g.ny + 1) * gb;
+    const int S = (int)g.S(), A = g.nz * g.nz;
+    const IoMirror y{{folded, 0, g.nx * gb, gb, row, gb, 0, 0}, (int)gb, S, A, g.ny, 1};
+    const IoMirror x{{folded, 0, row, row, 0, row, 0, 0}, (int)gb, S, A, g.nx, 0};
     const int ty = reg_length(2 * g.ny) ? FFT_TILE_REG : FFT_TILE_DEFAULT;
     const int tx = reg_length(2 * g.nx) ? FFT_TILE_REG : FFT_TILE_DEFAULT;
     launch_pencil<double, -1, IoMirror, false>(2 * g.ny, y, g.nx * gb, 1, tw_y, s, ty);
