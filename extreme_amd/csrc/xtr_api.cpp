@@ -4,9 +4,9 @@
 // The Krylov solver restates Extreme.Fgmres (Gmres.cs, FlexibleGmresSolver.cs,
 // ClassicGmresSolver.cs, FlexibleGmresWithGmresPreconditioner.cs) with the basis vectors in
 // HBM: the host keeps the (m+1)^2 Hessenberg matrix and the Givens rotations in FP64 and
-// drives the kernels; every Gram-Schmidt pass costs one device->host copy of the j+1
-// projections and the new norm, which is exactly what the iterated classical Gram-Schmidt
-// test (Gmres.cs:297-300) needs to decide on a second pass.
+// drives the kernels; a Gram-Schmidt pass puts the j+1 projections and the new norm into host memory,
+// which is exactly what the iterated classical Gram-Schmidt test (Gmres.cs:297-300) needs to decide
+// on a second pass.
 #include "xtr_green.h"
 #include "xtr_kernels.h"
 #include "xtr_learned.h"
@@ -19,7 +19,6 @@
 #include <chrono>
 #include <cmath>
 #include <complex>
-#include <condition_variable>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -28,7 +27,7 @@
 #include <memory>
 #include <mutex>
 #include <string>
-#include <thread>
+#include <ucontext.h>
 #include <type_traits>
 #include <vector>
 
@@ -136,21 +135,10 @@ std::string shortest(double v)
     return b;
 }
 
-// Waits for everything submitted to `s` so far by polling an event: the host resumes as soon as
-// the GPU passes the marker instead of being woken from a blocking wait.
-inline void spin_wait(hipStream_t s, hipEvent_t ev)
-{
-    XTR_CHECK(hipEventRecord(ev, s));
-    hipError_t e;
-    while ((e = hipEventQuery(ev)) == hipErrorNotReady) {
-    }
-    XTR_CHECK(e);
-}
-
 }  // namespace
 
 namespace {
-struct Slot;   // Krylov storage, stream and reduction scratch of one right-hand side (below)
+struct Slot;   // Krylov storage and reduction scratch of one right-hand side (below)
 }
 
 struct xtr_op {
@@ -201,7 +189,7 @@ struct xtr_op {
     size_t ev_used = 0;
     std::mutex apply_mu;
 
-    // Per right-hand side: a stream, the Krylov bases of the outer FGMRES and the inner GMRES, the
+    // Per right-hand side: the Krylov bases of the outer FGMRES and the inner GMRES, the
     // refinement vectors and the reduction scratch, allocated on first use and kept for later solves
     // (grown when a solve needs more), so that a solve allocates nothing once the handle has run one
     // of its shape. Slot kMaxRhs holds the FP64 norms of the mixed-precision refinement.
@@ -397,46 +385,95 @@ cd zeta_of(double sigma, double omega) { return cd(sigma, -omega * kEps0); }   /
 // FGMRES / GMRES on device vectors
 // ---------------------------------------------------------------------------------------------
 
-// One operator apply of a solve's vector x into y: complex128 vectors, or complex64 ones in the
-// correction solves of the mixed-precision refinement.
-using ApplyFn = std::function<void(const void *x, void *y)>;
+// What a solve asks of the GPU, one operation at a time. Solves of several right-hand sides advance in step
+// (Lockstep below): an operation they all ask for is then one launch, or one apply, for all of them.
+enum class StepOp { none, apply, cgs, norm, residual, call };
+struct StepReq {
+    StepOp op = StepOp::none;
+    const void *V = nullptr, *u = nullptr;   // apply: V = x; as in xtr::StepRhs otherwise
+    void *w = nullptr, *next = nullptr;      // apply: w = y
+    int cnt = 0, mul = 0;
+    const std::function<void()> *call = nullptr;
+    // norm's result is only needed after the next request that waits
+    bool has_result() const { return op == StepOp::cgs || op == StepOp::residual; }
+};
+
+// Small results of kernels in host memory that the host polls: begin(n) marks n values as missing, and a value
+// is there when it is no longer the mark (a NaN that arithmetic does not make).
+class Polled {
+public:
+    explicit Polled(size_t n) : buf_(n) {}
+    double *dev() const { return buf_.dev; }
+    const double *begin(int n)
+    {
+        n_ = n;
+        for (int i = 0; i < n; ++i) __atomic_store_n((uint64_t *)buf_.p + i, kMark, __ATOMIC_RELAXED);
+        return buf_.p;
+    }
+    bool ready()
+    {
+        // the last ones first: they are the likeliest to be missing
+        while (n_ > 0 && __atomic_load_n((uint64_t *)buf_.p + n_ - 1, __ATOMIC_ACQUIRE) != kMark) --n_;
+        return n_ == 0;
+    }
+    const double *p() const { return buf_.p; }
+
+private:
+    static constexpr uint64_t kMark = 0x7ff4'5e17'a11d'0badull;
+    MappedBuf<double> buf_;
+    int n_ = 0;
+};
 
 struct SolveCtx {
     hipStream_t stream;
-    ApplyFn apply;
+    // carries one request out; returns when its result, if it has one, is on the host
+    std::function<void(const StepReq &)> run;
     int64_t matvecs = 0;
     int64_t dots = 0;
     xtr_iteration_fn on_iter = nullptr;
     void *user = nullptr;
     int rhs_index = 0;
-    // reduction scratch shared by the outer and inner solvers of one solve
-    DevBuf<double2> partial_c;   // [32][kRedBlocks]
-    DevBuf<double> partial_r;    // [kRedBlocks]
-    DevBuf<double2> h_dev;       // [32] projections
-    DevBuf<double> norm_dev;     // [1]
+    DevBuf<double2> partial_c;   // [32][kRedBlocks] partial sums of the projections
+    DevBuf<double> partial_r;    // [kRedBlocks] of a squared norm
     // pairs (v_j, z_j) of the flexible preconditioner, copied out while count < cap
     double2 *const *harvest_v = nullptr;
     double2 *const *harvest_z = nullptr;
     int harvest_cap = 0, harvest_count = 0;
-    MappedBuf<double2> h_host{32};   // the projections, written by the reduction kernel
-    MappedBuf<double> nn_host{1};    // the squared norm, likewise
-    hipEvent_t ev = nullptr;
-    SolveCtx() : partial_c(32 * xtr::kRedBlocks), partial_r(xtr::kRedBlocks), h_dev(32), norm_dev(1)
-    {
-        XTR_CHECK(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
-    }
-    ~SolveCtx()
-    {
-        if (ev) (void)hipEventDestroy(ev);
-    }
+    Polled h_host{64};                  // the projections (re, im)
+    Polled n_host{xtr::kRedBlocks};     // partial sums of the squared norm of a cgs or residual
+    Polled b_host{xtr::kRedBlocks};     // of a norm
+    SolveCtx() : partial_c(32 * xtr::kRedBlocks), partial_r(xtr::kRedBlocks) {}
     SolveCtx(const SolveCtx &) = delete;
     SolveCtx &operator=(const SolveCtx &) = delete;
-    void wait() { spin_wait(stream, ev); }
+    bool ready() { return n_host.ready() && h_host.ready() && b_host.ready(); }
+    // Waits for the results asked for. A stream that has run dry, or failed, ends the wait whatever was stored.
+    void wait()
+    {
+        for (unsigned spin = 1; !ready(); ++spin) {
+            __builtin_ia32_pause();
+            if (spin % 4096 == 0) {
+                const hipError_t e = hipStreamQuery(stream);
+                if (e == hipErrorNotReady) continue;
+                XTR_CHECK(e);
+                return;
+            }
+        }
+    }
+    // norms from the partial sums of an n-vector's reduction
+    double norm(const Polled &p, int64_t n) const { return std::sqrt(xtr::sum_partials(p.p(), xtr::reduction_blocks(n))); }
+    // a launch or a callback of this right-hand side alone
+    void call(const std::function<void()> &f)
+    {
+        StepReq r;
+        r.op = StepOp::call;
+        r.call = &f;
+        run(r);
+    }
     // ready for a new solve on stream s: counters, callbacks and harvest cleared
     void reset(hipStream_t s)
     {
         stream = s;
-        apply = nullptr;
+        run = nullptr;
         matvecs = dots = 0;
         on_iter = nullptr;
         user = nullptr;
@@ -460,8 +497,6 @@ inline void grow(DevBuf<VT> &b, size_t need)
 }
 
 struct Slot {
-    hipStream_t stream = nullptr;
-    hipEvent_t ready = nullptr;   // the solve's vector is ready for the shared apply (ApplyGate)
     SolveCtx ctx;
     GmresBufs<double2> outer, inner;
     GmresBufs<float2> outer32, inner32;   // complex64 bases of the mixed-precision correction solves
@@ -469,25 +504,6 @@ struct Slot {
     DevBuf<float2> r32, d32;      // the same in complex64, for correction solves on complex64 vectors
     template <typename VT> GmresBufs<VT> &outer_bufs();
     template <typename VT> GmresBufs<VT> &inner_bufs();
-    Slot()
-    {
-        XTR_CHECK(hipEventCreateWithFlags(&ready, hipEventDisableTiming));
-        const hipError_t e = hipStreamCreateWithFlags(&stream, hipStreamDefault);
-        if (e != hipSuccess) {
-            (void)hipEventDestroy(ready);
-            XTR_CHECK(e);
-        }
-    }
-    ~Slot()
-    {
-        if (stream) {
-            (void)hipStreamSynchronize(stream);
-            (void)hipStreamDestroy(stream);
-        }
-        if (ready) (void)hipEventDestroy(ready);
-    }
-    Slot(const Slot &) = delete;
-    Slot &operator=(const Slot &) = delete;
 };
 
 }  // namespace
@@ -594,6 +610,52 @@ double net_gradients(xtr_net *net, int ns, const double2 *const *v, const double
     return total / ns;
 }
 
+// The requests of several right-hand sides that are of one kind, in one launch each (two for cgs), or one apply.
+template <typename VT>
+void launch_steps(xtr_op *op, StepOp kind, int nr, const StepReq *const *req, SolveCtx *const *ctx, const double2 *const *R,
+                  hipStream_t s)
+{
+    if (kind == StepOp::apply) {
+        xtr::RhsPtrs v{};
+        for (int i = 0; i < nr; ++i) {
+            v.x[i] = (const double2 *)req[i]->V;
+            v.y[i] = (double2 *)req[i]->w;
+            v.R[i] = R[i];
+        }
+        op->apply_raw(v, nr, s, std::is_same<VT, float2>::value);
+        return;
+    }
+    const int64_t n = op->g.n();
+    xtr::StepArgs<VT> a{};
+    for (int i = 0; i < nr; ++i) {
+        Polled &to = kind == StepOp::norm ? ctx[i]->b_host : ctx[i]->n_host;
+        to.begin(xtr::reduction_blocks(n));
+        ctx[i]->h_host.begin(2 * req[i]->cnt);
+        a.rhs[i] = xtr::StepRhs<VT>{(const VT *)req[i]->V, (const VT *)req[i]->u, (VT *)req[i]->w,
+                                    (VT *)req[i]->next,    ctx[i]->partial_c.p,   ctx[i]->partial_r.p,
+                                    (double2 *)ctx[i]->h_host.dev(), to.dev(), req[i]->cnt, req[i]->mul};
+    }
+    if (kind == StepOp::cgs) xtr::launch_cgs_step(a, nr, n, s);
+    else xtr::launch_step_norm(a, nr, n, s);
+}
+
+// A solve alone: its requests are launched as they come, on the operator's stream.
+template <typename VT>
+void run_alone(xtr_op *op, SolveCtx &ctx)
+{
+    SolveCtx *c = &ctx;
+    ctx.run = [op, c](const StepReq &r) {
+        if (r.op == StepOp::call) {
+            (*r.call)();
+            return;
+        }
+        const StepReq *rp = &r;
+        const double2 *R = nullptr;
+        launch_steps<VT>(op, r.op, 1, &rp, &c, &R, c->stream);
+        if (r.has_result()) c->wait();
+    };
+}
+
 // GmresSolver (Gmres.cs) on vectors of element type VT: double2 (complex128, the reference's
 // arithmetic) or float2 (complex64, the correction solves of the mixed-precision refinement). Dots,
 // norms, the Hessenberg matrix and the Givens rotations are FP64 either way.
@@ -633,36 +695,59 @@ struct Gmres {
 
     void matvec(const VT *x, VT *y)
     {
-        ctx->apply(x, y);
+        StepReq r;
+        r.op = StepOp::apply;
+        r.V = x;
+        r.w = y;
+        ctx->run(r);
         ctx->matvecs++;
     }
 
-    double norm(const VT *v)
+    // asks for |v|; its value is there after the next residual
+    void norm(const VT *v)
     {
-        xtr::launch_norm2(v, n, ctx->partial_r.p, ctx->stream);
-        xtr::launch_reduce_r(ctx->partial_r.p, ctx->norm_dev.p, ctx->stream, ctx->nn_host.dev);
-        ctx->wait();
+        StepReq r;
+        r.op = StepOp::norm;
+        r.w = (void *)v;
+        ctx->run(r);
         ctx->dots++;
-        return std::sqrt(ctx->nn_host.p[0]);
     }
 
-    // ClassicalGramSchmidtIteration (Gmres.cs:302-313) fused with the norm of the new w.
+    // w = b - ax and its norm; next: (1 / |w|) w
+    double residual(const VT *b, const VT *ax, VT *next)
+    {
+        StepReq r;
+        r.op = StepOp::residual;
+        r.V = b;
+        r.u = ax;
+        r.w = w;
+        r.next = next;
+        r.mul = 1;
+        ctx->run(r);
+        ctx->dots++;
+        return ctx->norm(ctx->n_host, n);
+    }
+
+    // ClassicalGramSchmidtIteration (Gmres.cs:302-313) fused with the norm of the new w, and w / |w| as the next
+    // basis vector
     void cgs(int jH, double &dloo, double &dnormw)
     {
         const int cnt = jH + 1;
-        xtr::launch_block_dots(V, cnt, w, n, ctx->partial_c.p, ctx->stream);
-        xtr::launch_reduce_c(ctx->partial_c.p, cnt, ctx->h_dev.p, ctx->stream, ctx->h_host.dev);
-        xtr::launch_cgs_update(V, cnt, ctx->h_dev.p, w, n, ctx->partial_r.p, ctx->stream);
-        xtr::launch_reduce_r(ctx->partial_r.p, ctx->norm_dev.p, ctx->stream, ctx->nn_host.dev);
-        ctx->wait();
+        StepReq r;
+        r.op = StepOp::cgs;
+        r.V = V;
+        r.w = w;
+        r.next = jH < m - 1 ? col(V, jH + 1) : nullptr;
+        r.cnt = cnt;
+        ctx->run(r);
         double s = 0;
         for (int k = 0; k < cnt; ++k) {
-            const cd d(ctx->h_host.p[k].x, ctx->h_host.p[k].y);
+            const cd d(ctx->h_host.p()[2 * k], ctx->h_host.p()[2 * k + 1]);
             h(k, jH) += d;                              // Zaxpy(jH+1, One, dots, H[:,jH])
             s += d.real() * d.real() + d.imag() * d.imag();
         }
         dloo = s;                                       // Dznrm2^2
-        dnormw = std::sqrt(ctx->nn_host.p[0]);
+        dnormw = ctx->norm(ctx->n_host, n);
         ctx->dots += cnt + 1;
     }
 
@@ -697,7 +782,7 @@ struct Gmres {
         if (flexible) {
             if (net) {
                 if constexpr (std::is_same<VT, double2>::value)
-                    net_precondition(net, col(V, jH), col(Z, jH), ctx->stream);
+                    ctx->call([&] { net_precondition(net, col(V, jH), col(Z, jH), ctx->stream); });
                 else
                     throw std::invalid_argument("the learned preconditioner runs on complex128 vectors");
             } else {
@@ -707,15 +792,18 @@ struct Gmres {
             }
             if (ctx->harvest_count < ctx->harvest_cap) {
                 const int k = ctx->harvest_count++;
-                XTR_CHECK(hipMemcpyAsync(ctx->harvest_v[k], col(V, jH), n * sizeof(VT), hipMemcpyDeviceToDevice,
-                                         ctx->stream));
-                XTR_CHECK(hipMemcpyAsync(ctx->harvest_z[k], col(Z, jH), n * sizeof(VT), hipMemcpyDeviceToDevice,
-                                         ctx->stream));
+                copy(col(V, jH), (VT *)ctx->harvest_v[k]);
+                copy(col(Z, jH), (VT *)ctx->harvest_z[k]);
             }
             matvec(col(Z, jH), w);
         } else {
             matvec(col(V, jH), w);
         }
+    }
+
+    void copy(const VT *src, VT *dst)
+    {
+        ctx->call([&] { XTR_CHECK(hipMemcpyAsync(dst, src, n * sizeof(VT), hipMemcpyDeviceToDevice, ctx->stream)); });
     }
 
     // ConstructCurrentSolution (Gmres.cs:187-196): y = H^-1 g, x += B y
@@ -730,15 +818,14 @@ struct Gmres {
         }
         xtr::Coef32 c{};
         for (int i = 0; i < jH; ++i) c.c[i] = make_double2(y[i].real(), y[i].imag());
-        if (jH > 0) xtr::launch_update_solution(flexible ? Z : V, jH, c, x, n, ctx->stream);
+        if (jH > 0) ctx->call([&] { xtr::launch_update_solution(flexible ? Z : V, jH, c, x, n, ctx->stream); });
     }
 
     // CheckBackwardError (Gmres.cs:200-230)
     double check_backward_error(double bn, const VT *rhs, const VT *x)
     {
         matvec(x, w);
-        xtr::launch_sub(rhs, w, w, n, ctx->stream);
-        const double be = norm(w) / bn;
+        const double be = residual(rhs, w, nullptr) / bn;
         if (be >= tol && backward_check == 2)
             throw std::runtime_error("be = " + shortest(be) + ", tolerance = " + shortest(tol));
         return be;
@@ -767,7 +854,6 @@ struct Gmres {
                     throw std::runtime_error("a Krylov vector holds NaN or Inf: the operator produced non-finite values");
             } while ((2.0 * dnormw <= std::sqrt(dloo)) && (north < 3));
             h(jH + 1, jH) = dnormw;
-            if (jH < m - 1) xtr::launch_div(w, dnormw, col(V, jH + 1), n, ctx->stream);
             for (int j = 0; j < jH; ++j) zrot1(h(j, jH), h(j + 1, jH), gc[j], gs[j]);
             zrotg(h(jH, jH), h(jH + 1, jH), gc[jH], gs[jH]);
             zrot1(h(jH, m), h(jH + 1, m), gc[jH], gs[jH]);
@@ -775,7 +861,8 @@ struct Gmres {
             h(jH + 1, jH) = 0;
             bea = std::abs(h(jH + 1, m)) / bn;
             ++iter_counter;
-            if (flexible && ctx->on_iter) ctx->on_iter(ctx->user, ctx->rhs_index, iter_counter, bea);
+            if (flexible && ctx->on_iter)
+                ctx->call([&] { ctx->on_iter(ctx->user, ctx->rhs_index, iter_counter, bea); });
             ++jH;
         } while (bea > tol && jH < m);
         return bea;
@@ -786,37 +873,37 @@ struct Gmres {
     {
         construct(jH, x);
         matvec(x, r0);
-        xtr::launch_sub(rhs, r0, w, n, ctx->stream);
-        return norm(w);
+        return residual(rhs, r0, col(V, 0));
     }
 
     // GmresSolver.Solve (Gmres.cs:77-143), initial guess supplied
     void solve(const VT *rhs, const VT *x0, VT *result, double &bea_out, double &be_out, int &conv)
     {
         iter_counter = 0;
-        const double bn = norm(rhs);
+        norm(rhs);                                      // read together with the residual's
+        matvec(x0, r0);
+        double beta = residual(rhs, r0, col(V, 0));
+        const double bn = ctx->norm(ctx->b_host, n);
         // NaN or Inf would end the iteration as if converged (bea > tol is false): refuse instead
         if (!std::isfinite(bn)) throw std::runtime_error("the right-hand side holds NaN or Inf");
         if (bn == 0) {
+            ctx->matvecs--;                             // of a residual that is not used
+            ctx->dots--;
             bea_out = 0; be_out = 0; conv = 1;
             return;
         }
-        matvec(x0, r0);
-        xtr::launch_sub(rhs, r0, w, n, ctx->stream);
-        double beta = norm(w);
         if (!std::isfinite(beta)) throw std::runtime_error("the initial residual holds NaN or Inf (operator or initial guess)");
         if (beta == 0) {   // CheckForExactSolution: ResultInfo.Converged(0, 0, 1) (Gmres.cs:104-107)
-            if (result != x0) XTR_CHECK(hipMemcpyAsync(result, x0, n * sizeof(VT), hipMemcpyDeviceToDevice, ctx->stream));
+            if (result != x0) copy(x0, result);
             bea_out = 0; be_out = 0; conv = 1;
             iter_counter = 1;
             return;
         }
         double bea = -1, be = -1;
         int iter = 0;
-        if (result != x0) XTR_CHECK(hipMemcpyAsync(result, x0, n * sizeof(VT), hipMemcpyDeviceToDevice, ctx->stream));
+        if (result != x0) copy(x0, result);
         for (;;) {
-            xtr::launch_mul(w, 1 / beta, col(V, 0), n, ctx->stream);
-            h(0, m) = beta;
+            h(0, m) = beta;                             // V_0 = (1 / beta) w is there
             for (int i = 1; i <= m; ++i) h(i, m) = 0;
             int jH = 0;
             bea = krylov(bn, jH);
@@ -836,109 +923,180 @@ struct Gmres {
 
 // FlexibleGmresWithGmresPreconditioner (:29-58) on one right-hand side.
 template <typename VT>
-void run_fgmres(int64_t n, const xtr_gmres_params &p, Slot &sl, const VT *b, VT *x, xtr_result_info &info,
+struct Fgmres {
+    SolveCtx &ctx;
+    std::unique_ptr<Gmres<VT>> inner, outer;
+    Fgmres(int64_t n, const xtr_gmres_params &p, Slot &sl, xtr_net *net = nullptr) : ctx(sl.ctx)
+    {
+        if (!std::is_same<VT, double2>::value)
+            require(ctx.harvest_cap == 0, "pairs are harvested from complex128 solves only");
+        require(p.outer_buffer_length >= 1 && p.outer_buffer_length <= 31, "OuterBufferLength must be 1..31");
+        require(p.inner_buffer_length >= 1 && p.inner_buffer_length <= 31, "InnerBufferLength must be 1..31");
+        require(p.max_repeat_number >= 1, "MaxRepeatsNumber must be >= 1");
+        if (!net) {
+            inner = std::make_unique<Gmres<VT>>(n, p.inner_buffer_length, false, &ctx, sl.inner_bufs<VT>());
+            inner->tol = p.tolerance;
+            inner->max_repeat = 1;
+            inner->backward_check = 0;
+        }
+        outer = std::make_unique<Gmres<VT>>(n, p.outer_buffer_length, true, &ctx, sl.outer_bufs<VT>());
+        outer->tol = p.tolerance;
+        outer->max_repeat = p.max_repeat_number;
+        outer->backward_check = p.backward_error_checking;
+        outer->inner = inner.get();
+        outer->net = net;
+    }
+    void solve(const VT *b, VT *x, xtr_result_info &info)
+    {
+        auto t0 = std::chrono::steady_clock::now();
+        double bea = -1, be = -1;
+        int conv = 0;
+        outer->solve(b, x, x, bea, be, conv);
+        ctx.call([&] { XTR_CHECK(hipStreamSynchronize(ctx.stream)); });
+        auto t1 = std::chrono::steady_clock::now();
+        info.converged = conv;
+        info.arnoldi_backward_error = bea;
+        info.backward_error = be;
+        info.number_of_iterations = outer->iter_counter;
+        info.matvecs = ctx.matvecs;
+        info.dot_products = ctx.dots;
+        info.seconds = std::chrono::duration<double>(t1 - t0).count();
+    }
+};
+
+// One right-hand side by itself, on the operator's stream.
+template <typename VT>
+void run_fgmres(xtr_op *op, const xtr_gmres_params &p, Slot &sl, const VT *b, VT *x, xtr_result_info &info,
                 xtr_net *net = nullptr)
 {
-    SolveCtx &ctx = sl.ctx;
-    if (!std::is_same<VT, double2>::value)
-        require(ctx.harvest_cap == 0, "pairs are harvested from complex128 solves only");
-    require(p.outer_buffer_length >= 1 && p.outer_buffer_length <= 31, "OuterBufferLength must be 1..31");
-    require(p.inner_buffer_length >= 1 && p.inner_buffer_length <= 31, "InnerBufferLength must be 1..31");
-    require(p.max_repeat_number >= 1, "MaxRepeatsNumber must be >= 1");
-    auto t0 = std::chrono::steady_clock::now();
-    std::unique_ptr<Gmres<VT>> inner;
-    if (!net) {
-        inner = std::make_unique<Gmres<VT>>(n, p.inner_buffer_length, false, &ctx, sl.inner_bufs<VT>());
-        inner->tol = p.tolerance;
-        inner->max_repeat = 1;
-        inner->backward_check = 0;
-    }
-    Gmres<VT> outer(n, p.outer_buffer_length, true, &ctx, sl.outer_bufs<VT>());
-    outer.tol = p.tolerance;
-    outer.max_repeat = p.max_repeat_number;
-    outer.backward_check = p.backward_error_checking;
-    outer.inner = inner.get();
-    outer.net = net;
-    double bea = -1, be = -1;
-    int conv = 0;
-    outer.solve(b, x, x, bea, be, conv);
-    XTR_CHECK(hipStreamSynchronize(ctx.stream));
-    auto t1 = std::chrono::steady_clock::now();
-    info.converged = conv;
-    info.arnoldi_backward_error = bea;
-    info.backward_error = be;
-    info.number_of_iterations = outer.iter_counter;
-    info.matvecs = ctx.matvecs;
-    info.dot_products = ctx.dots;
-    info.seconds = std::chrono::duration<double>(t1 - t0).count();
+    run_alone<VT>(op, sl.ctx);
+    Fgmres<VT>(op->g.n(), p, sl, net).solve(b, x, info);
 }
 
-// Pairs up the operator applies of solves that run side by side on their own streams: the
-// apply fires when every still-running solve has submitted one vector, so the Green tensor
-// is streamed once per round for all of them.
-struct ApplyGate {
-    xtr_op *op;
-    bool vec32;                   // the solves' vectors are complex64
-    std::mutex mu;
-    std::condition_variable cv;
-    int active;
-    int pending = 0;
-    uint64_t round = 0;
-    struct Sub { const void *x; void *y; hipStream_t s; hipEvent_t ready; const double2 *R; };
-    std::vector<Sub> subs;
-    hipEvent_t done = nullptr;
-    std::exception_ptr err;
-
-    ApplyGate(xtr_op *o, int n, bool v32) : op(o), vec32(v32), active(n)
+// Solves of several right-hand sides side by side, in step, on one host thread and the operator's stream. Each is a
+// fiber (its own stack, switched by ucontext) that runs until it asks for something of the GPU. When all have, what
+// they ask for is launched together: first whatever has no result to wait for, then the Gram-Schmidt passes and
+// residuals, whose results the host waits for once, and the apply when every solve that is still running asks for it, so that
+// the Green tensor is streamed once for all of them. Each right-hand side follows exactly the iteration of its own
+// solve. Fibers make no HIP call and no callback: those run on the caller's stack (StepOp::call).
+template <typename VT>
+class Lockstep {
+public:
+    Lockstep(xtr_op *o, int nrhs) : op_(o), fib_(nrhs) {}
+    // body(r) is right-hand side r's solve, with ctx[r]; R[r] its model's R (null: the handle's)
+    void run(const std::vector<SolveCtx *> &ctx, const std::vector<const double2 *> &R, const std::function<void(int)> &body)
     {
-        XTR_CHECK(hipEventCreateWithFlags(&done, hipEventDisableTiming));
+        const int nr = (int)fib_.size();
+        for (int r = 0; r < nr; ++r) {
+            Fiber &f = fib_[r];
+            f.stack.reset(new char[kStack]);
+            f.body = [&body, r] { body(r); };
+            ctx[r]->run = [this, r](const StepReq &q) { ask(r, q); };
+            if (getcontext(&f.ctx) != 0) throw std::runtime_error("getcontext failed");
+            f.ctx.uc_stack.ss_sp = f.stack.get();
+            f.ctx.uc_stack.ss_size = kStack;
+            f.ctx.uc_link = &main_;
+            const uintptr_t p = (uintptr_t)&f;
+            makecontext(&f.ctx, (void (*)())&Lockstep::entry, 2, (unsigned)(p >> 32), (unsigned)p);
+        }
+        for (int r = 0; r < nr; ++r) resume(r);
+        for (;;) {
+            std::vector<int> who[6];                          // by StepOp
+            int live = 0;
+            for (int r = 0; r < nr; ++r)
+                if (!fib_[r].done) {
+                    who[(int)fib_[r].req->op].push_back(r);
+                    ++live;
+                }
+            if (live == 0) break;
+            auto &calls = who[(int)StepOp::call], &norms = who[(int)StepOp::norm];
+            if (!calls.empty() || !norms.empty()) {
+                for (int r : calls) attempt({r}, [&] { (*fib_[r].req->call)(); });
+                if (!norms.empty()) attempt(norms, [&] { launch(StepOp::norm, norms, ctx, R); });
+                for (int r : calls) resume(r);
+                for (int r : norms) resume(r);
+                continue;
+            }
+            std::vector<int> res;
+            for (StepOp k : {StepOp::cgs, StepOp::residual}) {
+                auto &w = who[(int)k];
+                if (w.empty()) continue;
+                attempt(w, [&] { launch(k, w, ctx, R); });
+                res.insert(res.end(), w.begin(), w.end());
+            }
+            if (!res.empty()) {
+                for (int r : res)
+                    if (!fib_[r].fault) attempt({r}, [&] { ctx[r]->wait(); });
+                for (int r : res) resume(r);
+                continue;
+            }
+            auto &applies = who[(int)StepOp::apply];
+            attempt(applies, [&] { launch(StepOp::apply, applies, ctx, R); });
+            for (int r : applies) resume(r);
+        }
     }
-    ~ApplyGate()
-    {
-        if (done) (void)hipEventDestroy(done);
-    }
+    const std::exception_ptr &error(int r) const { return fib_[r].err; }
 
-    void fire()
+private:
+    static constexpr size_t kStack = 256 * 1024;
+    struct Fiber {
+        ucontext_t ctx;
+        std::unique_ptr<char[]> stack;
+        std::function<void()> body;
+        const StepReq *req = nullptr;
+        std::exception_ptr fault;             // of its request, thrown in the fiber
+        std::exception_ptr err;               // what ended the solve
+        bool done = false;
+    };
+    static void entry(unsigned hi, unsigned lo)
+    {
+        Fiber *f = (Fiber *)(((uintptr_t)hi << 32) | lo);
+        try {
+            f->body();
+        } catch (...) {
+            f->err = std::current_exception();
+        }
+        f->done = true;                       // returns to uc_link: the scheduler
+    }
+    void ask(int r, const StepReq &q)
+    {
+        Fiber &f = fib_[r];
+        f.req = &q;
+        swapcontext(&f.ctx, &main_);
+        f.req = nullptr;
+        if (f.fault) {
+            std::exception_ptr e;
+            std::swap(e, f.fault);
+            std::rethrow_exception(e);
+        }
+    }
+    void resume(int r) { swapcontext(&main_, &fib_[r].ctx); }
+    // an error of a shared launch goes to every solve that asked for it
+    template <typename F>
+    void attempt(const std::vector<int> &who, F &&f)
     {
         try {
-            xtr::RhsPtrs v{};
-            for (size_t i = 0; i < subs.size(); ++i) {
-                XTR_CHECK(hipStreamWaitEvent(op->stream, subs[i].ready, 0));
-                v.x[i] = (const double2 *)subs[i].x;
-                v.y[i] = (double2 *)subs[i].y;
-                v.R[i] = subs[i].R;
-            }
-            op->apply_raw(v, (int)subs.size(), op->stream, vec32);
-            XTR_CHECK(hipEventRecord(done, op->stream));
-            for (auto &s : subs) XTR_CHECK(hipStreamWaitEvent(s.s, done, 0));
+            f();
         } catch (...) {
-            err = std::current_exception();
+            for (int r : who) fib_[r].fault = std::current_exception();
         }
-        subs.clear();
-        pending = 0;
-        ++round;
-        cv.notify_all();
+    }
+    void launch(StepOp k, const std::vector<int> &who, const std::vector<SolveCtx *> &ctx, const std::vector<const double2 *> &R)
+    {
+        const StepReq *q[xtr::kMaxRhs];
+        SolveCtx *c[xtr::kMaxRhs];
+        const double2 *m[xtr::kMaxRhs];
+        for (size_t i = 0; i < who.size(); ++i) {
+            q[i] = fib_[who[i]].req;
+            c[i] = ctx[who[i]];
+            m[i] = R[who[i]];
+        }
+        launch_steps<VT>(op_, k, (int)who.size(), q, c, m, op_->stream);
     }
 
-    void submit(const void *x, void *y, hipStream_t s, hipEvent_t ready, const double2 *R)
-    {
-        XTR_CHECK(hipEventRecord(ready, s));
-        std::unique_lock<std::mutex> lk(mu);
-        if (err) std::rethrow_exception(err);
-        subs.push_back({x, y, s, ready, R});
-        ++pending;
-        const uint64_t mine = round;
-        if (pending == active) fire();
-        else cv.wait(lk, [&] { return round != mine; });
-        if (err) std::rethrow_exception(err);
-    }
-
-    void leave()
-    {
-        std::unique_lock<std::mutex> lk(mu);
-        --active;
-        if (pending > 0 && pending == active) fire();
-    }
+    xtr_op *op_;
+    std::vector<Fiber> fib_;
+    ucontext_t main_;
 };
 
 }  // namespace
@@ -947,63 +1105,41 @@ struct ApplyGate {
 // C ABI
 // =============================================================================================
 
-// Side-by-side FGMRES solves of nrhs right-hand sides with one ApplyGate (shared applies). Right-hand
-// side r runs on its own host thread with the handle's slot r (stream, bases, scratch).
+// Side-by-side FGMRES solves of nrhs right-hand sides in step; right-hand side r uses the handle's slot r.
 template <typename VT = double2>
 static void solve_batch(xtr_op *op, const xtr_gmres_params *params, int nrhs, const void *const *b, void *const *x,
                         xtr_result_info *info, xtr_iteration_fn on_iteration, void *user, const int *model = nullptr)
 {
-    ApplyGate gate(op, nrhs, std::is_same<VT, float2>::value);
-    std::vector<Slot *> sl(nrhs, nullptr);
-    std::vector<std::exception_ptr> errs(nrhs);
-    std::mutex cb_mu;
-    struct CbUser { xtr_iteration_fn fn; void *user; std::mutex *mu; };
-    CbUser cbu{on_iteration, user, &cb_mu};
-    auto cb = [](void *u, int r, int it, double bea) {
-        auto *c = (CbUser *)u;
-        std::lock_guard<std::mutex> lk(*c->mu);
-        c->fn(c->user, r, it, bea);
-    };
+    std::vector<SolveCtx *> ctx(nrhs);
+    std::vector<const double2 *> R(nrhs, nullptr);
+    for (int r = 0; r < nrhs; ++r) {
+        ctx[r] = &op->slot(r).ctx;
+        ctx[r]->reset(op->stream);
+        ctx[r]->rhs_index = r;
+        ctx[r]->on_iter = on_iteration;
+        ctx[r]->user = user;
+        if (model) R[r] = op->model_r(model[r]);
+    }
+    // inputs written on the caller's streams must be visible to the operator's
+    XTR_CHECK(hipDeviceSynchronize());
+    // buffers grow here, on the caller's stack, and not in a fiber
+    std::vector<std::unique_ptr<Fgmres<VT>>> solves;
+    for (int r = 0; r < nrhs; ++r) {
+        std::memset(&info[r], 0, sizeof(info[r]));
+        solves.push_back(std::make_unique<Fgmres<VT>>(op->g.n(), *params, op->slot(r)));
+    }
+    Lockstep<VT> steps(op, nrhs);
     try {
-        for (int r = 0; r < nrhs; ++r) {
-            sl[r] = &op->slot(r);
-            SolveCtx &c = sl[r]->ctx;
-            c.reset(sl[r]->stream);
-            c.rhs_index = r;
-            if (on_iteration) {
-                c.on_iter = cb;
-                c.user = &cbu;
-            }
-            hipStream_t s = sl[r]->stream;
-            hipEvent_t ev = sl[r]->ready;
-            ApplyGate *gp = &gate;
-            const double2 *Rp = model ? op->model_r(model[r]) : nullptr;   // null: the handle's R
-            c.apply = [gp, s, ev, Rp](const void *xx, void *yy) { gp->submit(xx, yy, s, ev, Rp); };
-        }
-        // inputs written on the caller's default stream must be visible to the solve streams
-        XTR_CHECK(hipDeviceSynchronize());
-        std::vector<std::thread> th;
-        for (int r = 0; r < nrhs; ++r) {
-            th.emplace_back([&, r] {
-                try {
-                    std::memset(&info[r], 0, sizeof(info[r]));
-                    run_fgmres<VT>(op->g.n(), *params, *sl[r], (const VT *)b[r], (VT *)x[r], info[r]);
-                } catch (...) {
-                    errs[r] = std::current_exception();
-                }
-                gate.leave();
-            });
-        }
-        for (auto &t : th) t.join();
-        XTR_CHECK(hipStreamSynchronize(op->stream));
+        steps.run(ctx, R, [&](int r) { solves[r]->solve((const VT *)b[r], (VT *)x[r], info[r]); });
     } catch (...) {
-        for (auto *p : sl)
-            if (p) (void)hipStreamSynchronize(p->stream);
+        (void)hipStreamSynchronize(op->stream);
+        for (auto *c : ctx) c->run = nullptr;
         throw;
     }
-    for (auto *p : sl) XTR_CHECK(hipStreamSynchronize(p->stream));
-    for (auto &e : errs)
-        if (e) std::rethrow_exception(e);
+    for (auto *c : ctx) c->run = nullptr;
+    XTR_CHECK(hipStreamSynchronize(op->stream));
+    for (int r = 0; r < nrhs; ++r)
+        if (steps.error(r)) std::rethrow_exception(steps.error(r));
 }
 
 extern "C" {
@@ -1463,15 +1599,8 @@ int xtr_fgmres_solve_device(xtr_op *op, const xtr_gmres_params *params, const vo
         ctx.reset(op->stream);
         ctx.on_iter = on_iteration;
         ctx.user = user;
-        xtr_op *o = op;
-        ctx.apply = [o](const void *xx, void *yy) {
-            xtr::RhsPtrs v{};
-            v.x[0] = (const double2 *)xx;
-            v.y[0] = (double2 *)yy;
-            o->apply_raw(v, 1, o->stream);
-        };
         std::memset(info, 0, sizeof(*info));
-        run_fgmres(op->g.n(), *params, sl, (const double2 *)b, (double2 *)x, *info);
+        run_fgmres(op, *params, sl, (const double2 *)b, (double2 *)x, *info);
     });
 }
 
@@ -1553,10 +1682,13 @@ static void refined_solve(xtr_op *op, const xtr_refine_params *params, int nrhs,
             }
         }
         auto norm = [&](const double2 *v) {
-            xtr::launch_norm2(v, n, ctx.partial_r.p, ctx.stream);
-            xtr::launch_reduce_r(ctx.partial_r.p, ctx.norm_dev.p, ctx.stream, ctx.nn_host.dev);
+            xtr::StepArgs<double2> a{};
+            a.rhs[0].w = const_cast<double2 *>(v);
+            a.rhs[0].norm = ctx.n_host.dev();
+            ctx.n_host.begin(xtr::reduction_blocks(n));
+            xtr::launch_step_norm(a, 1, n, ctx.stream);
             ctx.wait();
-            return std::sqrt(ctx.nn_host.p[0]);
+            return ctx.norm(ctx.n_host, n);
         };
         std::vector<double> bn(nrhs), rn(nrhs, 0.0);
         std::vector<int> live;
@@ -2041,15 +2173,8 @@ int xtr_fgmres_solve_learned_device(xtr_op *op, const xtr_gmres_params *params, 
         Slot &sl = op->slot(0);
         SolveCtx &ctx = sl.ctx;
         ctx.reset(op->stream);
-        xtr_op *o = op;
-        ctx.apply = [o](const void *xx, void *yy) {
-            xtr::RhsPtrs v{};
-            v.x[0] = (const double2 *)xx;
-            v.y[0] = (double2 *)yy;
-            o->apply_raw(v, 1, o->stream);
-        };
         std::memset(info, 0, sizeof(*info));
-        run_fgmres(op->g.n(), *params, sl, (const double2 *)b, (double2 *)x, *info, net);
+        run_fgmres(op, *params, sl, (const double2 *)b, (double2 *)x, *info, net);
     });
 }
 
@@ -2068,15 +2193,8 @@ int xtr_fgmres_solve_harvest_device(xtr_op *op, const xtr_gmres_params *params, 
         ctx.harvest_v = (double2 *const *)v_out;
         ctx.harvest_z = (double2 *const *)z_out;
         ctx.harvest_cap = capacity;
-        xtr_op *o = op;
-        ctx.apply = [o](const void *xx, void *yy) {
-            xtr::RhsPtrs v{};
-            v.x[0] = (const double2 *)xx;
-            v.y[0] = (double2 *)yy;
-            o->apply_raw(v, 1, o->stream);
-        };
         std::memset(info, 0, sizeof(*info));
-        run_fgmres(op->g.n(), *params, sl, (const double2 *)b, (double2 *)x, *info);
+        run_fgmres(op, *params, sl, (const double2 *)b, (double2 *)x, *info);
         XTR_CHECK(hipStreamSynchronize(op->stream));
         *count = ctx.harvest_count;
     });

@@ -171,31 +171,43 @@ void launch_level_field(const double2 *G, int electric, const double2 *jq, const
 // ---- Krylov (krylov_kernels.hip) -----------------------------------------------------------
 // Vectors are complex128 (double2) or complex64 (float2, the mixed-precision correction solves);
 // every kernel accumulates in FP64.
-constexpr int kRedBlocks = 512;   // partial-sum blocks of the reductions
-// partial[k][blk] of conj(V_k) . w, k < cnt (V columns contiguous, stride n)
-void launch_block_dots(const double2 *V, int cnt, const double2 *w, int64_t n, double2 *partial, hipStream_t s);
-void launch_block_dots(const float2 *V, int cnt, const float2 *w, int64_t n, double2 *partial, hipStream_t s);
-// out[k] = sum_blk partial[k][blk]
-void launch_reduce_c(const double2 *partial, int cnt, double2 *out, hipStream_t s, double2 *host_out = nullptr);
-// w -= sum_k V_k h_k (h on device), partial norms of the new w
-void launch_cgs_update(const double2 *V, int cnt, const double2 *h, double2 *w, int64_t n, double *partial,
-                       hipStream_t s);
-void launch_cgs_update(const float2 *V, int cnt, const double2 *h, float2 *w, int64_t n, double *partial,
-                       hipStream_t s);
-// partial sums of |w|^2 ; out = sum of partials
+constexpr int kRedBlocks = 512;   // most partial sums of a reduction
+int reduction_blocks(int64_t n);  // partial sums of a Gram-Schmidt step's reductions over n elements
+
+// their sum, in the order the kernels use
+double sum_partials(const double *p, int n);
+
+// A right-hand side's vectors in the batched kernels of a Gram-Schmidt step.
+template <typename VT>
+struct StepRhs {
+    const VT *V;        // basis columns (contiguous, stride n); b of a residual
+    const VT *u;        // A x of a residual, else null
+    VT *w;              // the vector worked on
+    VT *next;           // where w / |w| (mul: (1 / |w|) w) goes, or null
+    double2 *partial;   // [cnt][reduction_blocks(n)] scratch
+    double *norm_dev;   // [reduction_blocks(n)] scratch
+    double2 *h;         // [cnt] the projections (host memory, device address)
+    double *norm;       // [reduction_blocks(n)] partial sums of |w|^2 (host memory, device address)
+    int cnt, mul;
+};
+template <typename VT>
+struct StepArgs {
+    StepRhs<VT> rhs[kMaxRhs];
+};
+// h = V^H w, w -= V h, |w|^2, next
+void launch_cgs_step(const StepArgs<double2> &a, int nrhs, int64_t n, hipStream_t s);
+void launch_cgs_step(const StepArgs<float2> &a, int nrhs, int64_t n, hipStream_t s);
+// |w|^2, with w = V - u first where u is given, and next
+void launch_step_norm(const StepArgs<double2> &a, int nrhs, int64_t n, hipStream_t s);
+void launch_step_norm(const StepArgs<float2> &a, int nrhs, int64_t n, hipStream_t s);
+
+// partial sums of |w|^2 (kRedBlocks) ; out = sum of partials
 void launch_norm2(const double2 *w, int64_t n, double *partial, hipStream_t s);
-void launch_norm2(const float2 *w, int64_t n, double *partial, hipStream_t s);
-void launch_reduce_r(const double *partial, double *out, hipStream_t s, double *host_out = nullptr);
-// dst = src / d  (v_{j+1} = w / |w|, Gmres.cs:267-268)
-void launch_div(const double2 *src, double d, double2 *dst, int64_t n, hipStream_t s);
-void launch_div(const float2 *src, double d, float2 *dst, int64_t n, hipStream_t s);
-// dst = a * src  (V_0 = (1/beta) w, Gmres.cs:117; and the complex64 copy of a scaled residual)
-void launch_mul(const double2 *src, double a, double2 *dst, int64_t n, hipStream_t s);
-void launch_mul(const float2 *src, double a, float2 *dst, int64_t n, hipStream_t s);
+void launch_reduce_r(const double *partial, double *out, hipStream_t s);
+// dst = a * src (the complex64 copy of a scaled residual)
 void launch_mul(const double2 *src, double a, float2 *dst, int64_t n, hipStream_t s);
 // dst = a - b
 void launch_sub(const double2 *a, const double2 *b, double2 *dst, int64_t n, hipStream_t s);
-void launch_sub(const float2 *a, const float2 *b, float2 *dst, int64_t n, hipStream_t s);
 // x += sum_k B_k y_k  (ConstructCurrentSolution, y passed by value)
 struct Coef32 { double2 c[32]; };
 void launch_update_solution(const double2 *B, int cnt, const Coef32 &y, double2 *x, int64_t n, hipStream_t s);
