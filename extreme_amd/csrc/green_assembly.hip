@@ -932,7 +932,7 @@ void build_green_atoa(const GreenInput &in, GreenScratch &work, double2 *G, bool
         }
     }
     if (folded) launch_fft2_mirror(G, g, tw_x, tw_y, s);
-    else launch_fft2_plain(G, 2 * g.nx, 2 * g.ny, g.gblk(), tw_x, tw_y, -1, s);
+    else launch_fft2_plain(G, 2 * g.nx, 2 * g.ny, g.gblk(), tw_x, tw_y, s);
     XTR_CHECK(hipStreamSynchronize(s));   // the host pack is freed on return
 }
 
@@ -1081,13 +1081,15 @@ struct AoArgs {
     const double2 *segA, *segB;   // [seg][comp][tr]
     const double *radii;
     double2 *G;                   // [2Nx][2Ny][components][nz], components as in atoo_components
+    int folded;                   // [Nx+1][Ny+1][components][nz], offsets i, j >= 0 only
 };
 
-// One wave per lateral offset (i, j) in (-Nx, Nx) x (-Ny, Ny), lanes the transmitter layers: the four edge
+// One wave per lateral offset (i, j) in (-Nx, Nx) x (-Ny, Ny), or its non-negative quadrant where the tensor is
+// folded (a level that is not shifted), lanes the transmitter layers: the four edge
 // integrals of RunAlongX / RunAlongY (GreenTensorCalculator.cs:192-281), written at TransformI/J
 // (AtoOLevelGreenTensorCalculator.cs:106-117). The wave forms its offset's weights itself (CellWeights), 8 segments
-// at a time, a thread for each (segment, stretch). At 128 x 128 x 32: 0.26 and 0.22 ms; 0.64 ms each with every
-// thread working out the geometry.
+// at a time, a thread for each (segment, stretch). At 128 x 128 x 32, all offsets: 0.26 and 0.22 ms (0.64 ms each
+// with every thread working out the geometry); the quadrant: 0.12 and 0.11 ms.
 constexpr int kAoWaves = 4, kAoSegs = 8;
 
 template <int ELECTRIC>
@@ -1096,10 +1098,10 @@ __global__ __launch_bounds__(64 * kAoWaves) void atoo_lateral_kernel(AoArgs a)
     __shared__ CellWeights<kAoSegs> all[kAoWaves];
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     CellWeights<kAoSegs> &cw = all[wave];
-    const int ncy = 2 * a.ny - 1, cells = (2 * a.nx - 1) * ncy;
+    const int ncy = a.folded ? a.ny : 2 * a.ny - 1, cells = (a.folded ? a.nx : 2 * a.nx - 1) * ncy;
     const int cell = blockIdx.x * kAoWaves + wave;
     if (cell >= cells) return;                                  // waves do not meet at a barrier
-    const int i = cell / ncy - (a.nx - 1), j = cell % ncy - (a.ny - 1);
+    const int i = cell / ncy - (a.folded ? 0 : a.nx - 1), j = cell % ncy - (a.folded ? 0 : a.ny - 1);
     // LDS writes of this wave become visible to it in order; the fence only keeps the compiler from moving them
     auto sync = [] { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); __builtin_amdgcn_wave_barrier(); };
     cw.ends(lane, a.radii, a.nr, a.dx * (i - 0.5) - a.xs, a.dx * (i + 0.5) - a.xs, a.dy * (j - 0.5) - a.ys,
@@ -1156,7 +1158,7 @@ __global__ __launch_bounds__(64 * kAoWaves) void atoo_lateral_kernel(AoArgs a)
             sync();                                             // the weights are read
         }
         if (tr < a.nz) {
-            double2 *dst = a.G + (ti * 2 * a.ny + tj) * (int64_t)(no * a.nz) + tr;
+            double2 *dst = a.G + (ti * (a.folded ? a.ny + 1 : 2 * a.ny) + tj) * (int64_t)(no * a.nz) + tr;
 #pragma unroll
             for (int t = 0; t < no; ++t) dst[(int64_t)t * a.nz] = G[t];
         }
@@ -1175,7 +1177,7 @@ int atoo_components(int electric, int *slot)
 }
 
 void build_green_atoo_level(const GreenInput &in, GreenScratch &work, double level_z, double shift_x, double shift_y,
-                            int electric, double2 *G, const double2 *tw_x, const double2 *tw_y, hipStream_t s)
+                            int electric, bool folded, double2 *G, const double2 *tw_x, const double2 *tw_y, hipStream_t s)
 {
     const Geom &g = in.g;
     const int nz = g.nz;
@@ -1253,12 +1255,20 @@ void build_green_atoo_level(const GreenInput &in, GreenScratch &work, double lev
     a.segB = segB;
     a.radii = d.radii;
     a.G = G;
-    XTR_CHECK(hipMemsetAsync(G, 0, (size_t)g.L() * ntc * nz * sizeof(double2), s));
-    const dim3 grid((unsigned)ceil_div((2 * g.nx - 1) * (2 * g.ny - 1), kAoWaves)), nt(64 * kAoWaves);
+    a.folded = folded ? 1 : 0;
+    if (!folded) XTR_CHECK(hipMemsetAsync(G, 0, (size_t)g.L() * ntc * nz * sizeof(double2), s));
+    const int cells = folded ? g.nx * g.ny : (2 * g.nx - 1) * (2 * g.ny - 1);
+    const dim3 grid((unsigned)ceil_div(cells, kAoWaves)), nt(64 * kAoWaves);
     if (electric) hipLaunchKernelGGL(atoo_lateral_kernel<1>, grid, nt, 0, s, a);
     else hipLaunchKernelGGL(atoo_lateral_kernel<0>, grid, nt, 0, s, a);
     XTR_LAUNCH_CHECK("atoo_lateral_kernel");
-    launch_fft2_plain(G, 2 * g.nx, 2 * g.ny, (int64_t)ntc * nz, tw_x, tw_y, -1, s);
+    if (folded) {
+        unsigned odd[2];
+        level_parity(electric, odd);
+        launch_fft2_mirror_level(G, g, ntc, odd, tw_x, tw_y, s);
+    } else {
+        launch_fft2_plain(G, 2 * g.nx, 2 * g.ny, (int64_t)ntc * nz, tw_x, tw_y, s);
+    }
     XTR_CHECK(hipStreamSynchronize(s));   // the host pack is freed on return
 }
 

@@ -178,7 +178,7 @@ struct xtr_op {
     DevBuf<double2> stage_x, stage_y;   // host-pointer apply staging
     xtr::GreenScratch green_work;  // scratch of the tensor assemblies
     DevBuf<double2> Go[2];        // AtoO level tensors [L][ncomp][nz]: [0] magnetic, [1] electric
-    bool go_ready[2] = {false, false};
+    bool go_ready[2] = {false, false}, go_folded[2] = {false, false};
     DevBuf<double2> lvl_spec, lvl_small;   // level-field scratch: L * 3nz and L * 3
 
     // Per-stage timing: one set of six events per apply while profiling is on, summed on demand.
@@ -1800,10 +1800,13 @@ int xtr_op_build_green_atoo(xtr_op *op, double level_z, double x_shift, double y
         const int ncomp = xtr::atoo_components(e, slot);
         op->go_ready[e] = false;
         require(std::isfinite(x_shift) && std::isfinite(y_shift), "level shift must be finite");
-        const size_t need = (size_t)(op->g.L() * ncomp * op->g.nz);
+        // without a shift the offsets (i, j) and (-i, j) mirror each other, as the anomaly's own do
+        const bool fold = x_shift == 0 && y_shift == 0 && green_fold_allowed();
+        const size_t need = (size_t)((fold ? op->g.Lq() : op->g.L()) * ncomp * op->g.nz);
         if (op->Go[e].count != need) op->Go[e].alloc(need);
-        xtr::build_green_atoo_level(green_input(op), op->green_work, level_z, x_shift, y_shift, e, op->Go[e].p, op->tw64_x.p,
-                                    op->tw64_y.p, op->stream);
+        xtr::build_green_atoo_level(green_input(op), op->green_work, level_z, x_shift, y_shift, e, fold, op->Go[e].p,
+                                    op->tw64_x.p, op->tw64_y.p, op->stream);
+        op->go_folded[e] = fold;
         op->go_ready[e] = true;
     });
 }
@@ -1817,13 +1820,21 @@ int xtr_op_get_green_atoo(xtr_op *op, int electric, xtr_complex *const *comps)
         int slot[9];
         const int ncomp = xtr::atoo_components(e, slot);
         const int64_t L = op->g.L(), nz = op->g.nz;
-        std::vector<double2> h((size_t)(L * ncomp * nz));
+        std::vector<double2> h(op->Go[e].count);
         XTR_CHECK(hipMemcpy(h.data(), op->Go[e].p, h.size() * sizeof(double2), hipMemcpyDeviceToHost));
+        unsigned odd[2];
+        xtr::level_parity(e, odd);
         for (int t = 0; t < 9; ++t) {
             if (!comps[t] || slot[t] < 0) continue;
             auto *dst = reinterpret_cast<double2 *>(comps[t]);
-            for (int64_t l = 0; l < L; ++l)
-                std::memcpy(dst + l * nz, h.data() + (l * ncomp + slot[t]) * nz, nz * sizeof(double2));
+            for (int64_t l = 0; l < L; ++l) {
+                xtr::FoldPos p{l, 0, 0};
+                if (op->go_folded[e]) p = xtr::fold_pos(l, op->g.nx, op->g.ny);
+                const double2 *src = h.data() + (p.b * ncomp + slot[t]) * nz;
+                const bool neg = (p.mx && odd[0] >> slot[t] & 1) != (p.my && odd[1] >> slot[t] & 1);
+                for (int64_t k = 0; k < nz; ++k)
+                    dst[l * nz + k] = neg ? make_double2(-src[k].x, -src[k].y) : src[k];
+            }
         }
     });
 }
@@ -1896,7 +1907,7 @@ int xtr_op_level_field_noalloc_device(xtr_op *op, int electric, const void *jq, 
         require(dev == op->device, "the handle was created on another device than the current one");
         double2 *ptr = scratch_on_device(dev);
         XTR_CHECK(hipDeviceSynchronize());   // jQ may have been written on another stream
-        xtr::launch_level_field(op->Go[e].p, e, (const double2 *)jq, g, ptr, ptr + g.M(), op->tw64_x.p, op->tw64_y.p,
+        xtr::launch_level_field(op->Go[e].p, e, op->go_folded[e], (const double2 *)jq, g, ptr, ptr + g.M(), op->tw64_x.p, op->tw64_y.p,
                                 (double2 *)field, op->stream);
         XTR_CHECK(hipStreamSynchronize(op->stream));
     });
@@ -1912,7 +1923,7 @@ int xtr_op_level_field_device(xtr_op *op, int electric, const void *jq, void *fi
         if (op->lvl_spec.count < (size_t)g.M()) op->lvl_spec.alloc((size_t)g.M());
         if (op->lvl_small.count < (size_t)(3 * g.L())) op->lvl_small.alloc((size_t)(3 * g.L()));
         XTR_CHECK(hipDeviceSynchronize());   // jQ may have been written on another stream
-        xtr::launch_level_field(op->Go[e].p, e, (const double2 *)jq, g, op->lvl_spec.p, op->lvl_small.p, op->tw64_x.p,
+        xtr::launch_level_field(op->Go[e].p, e, op->go_folded[e], (const double2 *)jq, g, op->lvl_spec.p, op->lvl_small.p, op->tw64_x.p,
                                 op->tw64_y.p, (double2 *)field, op->stream);
         XTR_CHECK(hipStreamSynchronize(op->stream));
     });

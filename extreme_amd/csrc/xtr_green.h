@@ -100,9 +100,10 @@ void build_green_atoa(const GreenInput &in, GreenScratch &work, double2 *G, bool
 // AtoO level tensor for the observation level at depth level_z whose sites are the cell centres
 // shifted by (shift_x, shift_y) metres: device layout [L][component][nz] with components, in order,
 // xx yy zz xy xz yz zx zy (electric = 1) or xx xy yx xz yz zx zy (electric = 0), FFT'd; G holds
-// L * ncomp * nz complex128.
+// L * ncomp * nz complex128. folded (a level that is not shifted): only the (Nx+1)(Ny+1) blocks kx <= Nx, ky <= Ny;
+// the others follow with the signs of level_parity.
 int atoo_components(int electric, int *slot /* [9]: xx yy zz xy yx xz yz zx zy -> compact or -1 */);
 void build_green_atoo_level(const GreenInput &in, GreenScratch &work, double level_z, double shift_x, double shift_y,
-                            int electric, double2 *G, const double2 *tw_x, const double2 *tw_y, hipStream_t s);
+                            int electric, bool folded, double2 *G, const double2 *tw_x, const double2 *tw_y, hipStream_t s);
 
 }  // namespace xtr

@@ -138,13 +138,21 @@ int device_cus();            // compute units of the current device
 void launch_inv_x(const ApplyArgs &a, hipStream_t s);
 void launch_inv_y(const ApplyArgs &a, hipStream_t s);
 
-// In-place forward 2-D FFT of a [2nx][2ny][ncols] array (Green tensor), FP64.
-void launch_fft2_plain(double2 *data, int n1, int n2, int64_t ncols, const double2 *tw1, const double2 *tw2,
-                       int sign, hipStream_t s);
+// In-place forward 2-D FFT of an [n1][n2][ncols] array (an assembled tensor), FP64.
+void launch_fft2_plain(double2 *data, int n1, int n2, int64_t ncols, const double2 *tw1, const double2 *tw2, hipStream_t s);
 // The same for a Green tensor held folded, [Nx+1][Ny+1][gblk], in place: points (i, j), i < Nx and j < Ny,
 // hold the tensor at those lateral offsets on entry, and every block the spectrum on return; the negative
 // offsets follow from the mirror parities.
 void launch_fft2_mirror(double2 *folded, const Geom &g, const double2 *tw_x, const double2 *tw_y, hipStream_t s);
+// The same for a level tensor [Nx+1][Ny+1][ncomp][nz]; bit c of odd[0] (odd[1]): component c is odd in x (y).
+void launch_fft2_mirror_level(double2 *folded, const Geom &g, int ncomp, const unsigned *odd, const double2 *tw_x,
+                              const double2 *tw_y, hipStream_t s);
+// Forward FFT of src [Nx][Ny][C], zero-padded, into spec [2Nx][2Ny][C]; backward FFT of spec (which it works in),
+// cropped and scaled, into dst [Nx][Ny][C].
+void launch_fft2_padded(const double2 *src, double2 *spec, const Geom &g, int C, const double2 *tw_x, const double2 *tw_y,
+                        hipStream_t s);
+void launch_fft2_cropped(double2 *spec, double2 *dst, const Geom &g, int C, double scale, const double2 *tw_x,
+                         const double2 *tw_y, hipStream_t s);
 bool fft_length_supported(int p);
 
 // Reorders the Green tensor between the reference layout (six component arrays) and the
@@ -161,12 +169,20 @@ void launch_to_f32(const double2 *src, float2 *dst, int64_t n, hipStream_t s);
 void launch_probe_stream(const void *src, void *dst, int64_t blocks, int read_kb, int write_kb, hipStream_t s);
 
 // Observation level (obs_kernels.hip): jQ from chi (operator prepared as A: R and f of that type),
-// and the anomalous field at a level from jQ with the AtoO tensor G ([L][ncomp][nz]); spec holds
-// L * 3nz and small L * 3 complex128 of scratch; field is [Nx][Ny][3].
+// and the anomalous field at a level from jQ with the AtoO tensor G ([L][ncomp][nz], or folded the
+// (Nx+1)(Ny+1) blocks kx <= Nx, ky <= Ny); spec holds L * 3nz and small L * 3 complex128 of scratch; field
+// is [Nx][Ny][3].
 void launch_jq(const double2 *chi, const double2 *js, const double2 *R, const double *f, const Geom &g, double2 *jq,
                hipStream_t s);
-void launch_level_field(const double2 *G, int electric, const double2 *jq, const Geom &g, double2 *spec,
+void launch_level_field(const double2 *G, int electric, int folded, const double2 *jq, const Geom &g, double2 *spec,
                         double2 *small, const double2 *tw_x, const double2 *tw_y, double2 *field, hipStream_t s);
+// Components of a level tensor that are odd in x (odd[0]) and in y (odd[1]), as bit masks in their order
+inline void level_parity(int electric, unsigned *odd)
+{
+    // electric xx yy zz xy xz yz zx zy; magnetic xx xy yx xz yz zx zy
+    odd[0] = electric ? 1u << 3 | 1u << 4 | 1u << 6 : 1u << 0 | 1u << 4 | 1u << 6;
+    odd[1] = electric ? 1u << 3 | 1u << 5 | 1u << 7 : 1u << 0 | 1u << 3 | 1u << 5;
+}
 
 // ---- Krylov (krylov_kernels.hip) -----------------------------------------------------------
 // Vectors are complex128 (double2) or complex64 (float2, the mixed-precision correction solves);
