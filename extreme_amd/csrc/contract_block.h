@@ -33,7 +33,7 @@ namespace xtr {
 // Measured, time of the contraction per apply, against the kernels it replaced (vector FMAs or MFMA on a block
 // expanded through registers up to nz = 31, one workgroup per wavenumber from 33, a one-region MFMA kernel for
 // 32): 32 x 32 x 8, 1 right-hand side 11.3 -> 8.3 us; 48 x 96 x 24, 2: 150 -> 60 us (264 MB, 4.4 TB/s; the
-// copies without arithmetic 47); 40 x 40 x 40, 2: 209 -> 58 us (copies 43); 64 x 64 x 16, 8: 220 -> 83 us
+// copies without arithmetic 47); 40 x 40 x 40, 2: 209 -> 58 us (copies 43); 64 x 64 x 16, 8: 220 -> 77 us
 // (copies 56, arithmetic 65 to 80); nz = 32: 64 x 64, 1: 85 -> 79 us, 4: 167 -> 141 us, 128 x 128, 2: 301 us both.
 // What is left above the copies is the last, partly filled round of blocks, and MFMA work for padding
 // (nz = 24: 80 of 72 rows).
@@ -360,12 +360,18 @@ __global__ __launch_bounds__((64 * BlockCfg<T, NZ, NR>::W)) void contract_block_
     static_assert(K::N1 / K::W + K::NU / K::W + 2 + K::STORES < 64 && K::N2 / K::W + 1 + K::STORES < 64, "vmcnt range");
     __shared__ __attribute__((aligned(16))) unsigned char smem[K::LDS];
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    p.buf += (int64_t)(blockIdx.y * NR) * p.M;                         // this workgroup's right-hand sides
+    p.nrhs -= blockIdx.y * NR;
     if (wave < K::TXY) block_run<T, NZ, NR, false>(p, smem, wave, lane);
     else block_run<T, NZ, NR, true>(p, smem, wave, lane);
 }
 
+// The right-hand sides in groups of NR, a row of workgroups (blockIdx.y) each: one launch, so that a group fills
+// the CUs that the last blocks of another leave. In launches of up to 8, one after the other, 8 right-hand sides
+// took 64 instead of 54 us at 64 x 64 x 12, 84 instead of 77 us at nz = 16, 200 instead of 166 us at nz = 24, and
+// at 48 x 40 x 40 (launches of 2) 250 instead of 211 us.
 template <typename T, int NZ, int NR>
-void launch_block(const ApplyArgs &a, int h0, int nh, hipStream_t s)
+void launch_block(const ApplyArgs &a, hipStream_t s)
 {
     using K = BlockCfg<T, NZ, NR>;
     // as many workgroups as are resident at once (registers and LDS): more would run in rounds
@@ -375,14 +381,15 @@ void launch_block(const ApplyArgs &a, int h0, int nh, hipStream_t s)
             &nb, (const void *)contract_block_kernel<T, NZ, NR>, 64 * K::W, 0)));
         return std::max(1, nb);
     }();
-    BlockArgs<T> p{(const cplx<T> *)a.G, (cplx<T> *)a.buf + h0 * a.g.M(), a.g.M(), (int)a.g.Lq(), nh, a.g.nx, a.g.ny};
-    const unsigned grid = (unsigned)std::min<int64_t>(p.Lq, (int64_t)resident * device_cus());
-    hipLaunchKernelGGL((contract_block_kernel<T, NZ, NR>), dim3(grid), dim3(64 * K::W), 0, s, p);
+    BlockArgs<T> p{(const cplx<T> *)a.G, (cplx<T> *)a.buf, a.g.M(), (int)a.g.Lq(), a.nrhs, a.g.nx, a.g.ny};
+    const unsigned groups = (unsigned)ceil_div(a.nrhs, NR);
+    const unsigned grid = (unsigned)std::min<int64_t>(p.Lq, ceil_div((int64_t)resident * device_cus(), groups));
+    hipLaunchKernelGGL((contract_block_kernel<T, NZ, NR>), dim3(grid, groups), dim3(64 * K::W), 0, s, p);
     XTR_LAUNCH_CHECK("contract_block_kernel");
 }
 
-// Depths LO..HI; false for another depth or one whose block does not fit. Right-hand sides in launches of up
-// to 8, 4 or 2, as many as fit (each launch reads the tensor once).
+// Depths LO..HI; false for another depth or one whose block does not fit. One right-hand side or two by
+// themselves; more in groups of 4 or 2 (a group reads the tensor once).
 template <typename T, int LO, int HI>
 bool contract_block_range(const ApplyArgs &a, hipStream_t s)
 {
@@ -393,16 +400,13 @@ bool contract_block_range(const ApplyArgs &a, hipStream_t s)
         if constexpr (!BlockCfg<T, LO, 1>::ok) {
             return false;
         } else {
-            constexpr int most = BlockCfg<T, LO, 8>::ok ? 8 : BlockCfg<T, LO, 4>::ok ? 4 : BlockCfg<T, LO, 2>::ok ? 2 : 1;
-            for (int h0 = 0; h0 < a.nrhs; h0 += most) {
-                const int nh = std::min(most, a.nrhs - h0);
-                if (nh == 1) { launch_block<T, LO, 1>(a, h0, nh, s); continue; }
-                if constexpr (most >= 2)
-                    if (nh == 2) { launch_block<T, LO, 2>(a, h0, nh, s); continue; }
-                if constexpr (most >= 4)
-                    if (nh <= 4) { launch_block<T, LO, 4>(a, h0, nh, s); continue; }
-                if constexpr (most >= 8) launch_block<T, LO, 8>(a, h0, nh, s);
-            }
+            // Groups of 2 where they leave room for more workgroups on a CU than groups of 4 (3 or 4 instead of 2
+            // to 3, by registers and LDS): 8 right-hand sides at 64 x 64, groups of 2 and of 4: nz = 16 77 and
+            // 82 us, 20: 130 and 155, 24: 166 and 188; outside these depths 12: 60 and 54, 32: 287 and 266.
+            constexpr int most = BlockCfg<T, LO, 4>::ok && (LO < 16 || LO > 25) ? 4 : BlockCfg<T, LO, 2>::ok ? 2 : 1;
+            if (a.nrhs == 1) launch_block<T, LO, 1>(a, s);
+            else if (a.nrhs == 2 && BlockCfg<T, LO, 2>::ok) launch_block<T, LO, BlockCfg<T, LO, 2>::ok ? 2 : 1>(a, s);
+            else launch_block<T, LO, most>(a, s);
             return true;
         }
     }
