@@ -93,57 +93,66 @@ struct LayerModel {
     double omega;
 };
 
-__global__ __launch_bounds__(128) void layer_aux_kernel(const LayerModel *lmp, int nitems, int nlam_max, const int *nlam, const double *lam,
+// Bound by the chain of complex divisions, roots and exponentials through the layers: a quarter of the grid
+// (blockIdx.z) runs each of the four recursions, with its layers' roots and exponentials in registers:
+// 9 us for 5 layers where one thread with all four in scratch arrays took 18.
+__global__ __launch_bounds__(64) void layer_aux_kernel(const LayerModel *lmp, int nitems, int nlam_max, const int *nlam, const double *lam,
                                  double2 *eta, double2 *ex, double2 *p1, double2 *q1, double2 *ps, double2 *qs)
 {
     const int m = blockIdx.x * blockDim.x + threadIdx.x;
     const int it = blockIdx.y;
     if (it >= nitems || m >= nlam[it]) return;
     const LayerModel &lm = *lmp;
-    const int nl = lm.nl;
+    const int nl = lm.nl, n = nl - 1;
     const double l = lam[(int64_t)it * nlam_max + m];
     const int64_t base = ((int64_t)it * nlam_max + m) * nl;
-    double2 E[kMaxLayers], X[kMaxLayers];
-    for (int k = 0; k < nl; ++k) {
-        // value = i omega * zeta * Mu0; eta = sqrt(lambda^2 - value)  (CalcEta, green_scalar.c:30-34)
-        const double2 value = (c_(0, lm.omega) * lm.zeta[k]) * c_(kMu0);
-        E[k] = csqrt_d(c_(l * l) - value);
-        X[k] = cexp_d((-2 * lm.thick[k]) * E[k]);    // CalcExp (green_scalar.c:36-41)
-        eta[base + k] = E[k];
-        ex[base + k] = X[k];
-    }
-    // P: p[1] from the top interface, then downwards (CalculatePBelow1, PlanCalculatorFast.cs:266-280)
-    double2 P1[kMaxLayers], PS[kMaxLayers], Q1[kMaxLayers], QS[kMaxLayers];
-    for (int k = 0; k < nl; ++k) P1[k] = PS[k] = Q1[k] = QS[k] = c_(0);
-    P1[1] = (E[1] - E[0]) / (E[1] + E[0]);
-    PS[1] = (lm.zeta[0] * E[1] - lm.zeta[1] * E[0]) / (lm.zeta[0] * E[1] + lm.zeta[1] * E[0]);
-    for (int k = 1; k < nl - 1; ++k) {
-        double2 pe = P1[k] * X[k];
-        double2 part = (c_(1) * (E[k] / E[k + 1])) * ((pe - c_(1)) / (pe + c_(1)));
-        P1[k + 1] = (c_(1) + part) / (c_(1) - part);
-        pe = PS[k] * X[k];
-        part = ((lm.zeta[k + 1] / lm.zeta[k]) * (E[k] / E[k + 1])) * ((pe - c_(1)) / (pe + c_(1)));
-        PS[k + 1] = (c_(1) + part) / (c_(1) - part);
-    }
-    // Q: q[n] = 0 at the bottom, then upwards (CalculateQ, PlanCalculatorFast.cs:292-318)
-    const int n = nl - 1;
-    double2 part = c_(1) * (E[n] / E[n - 1]);
-    Q1[n - 1] = (c_(1) - part) / (c_(1) + part);
-    part = (lm.zeta[n - 1] / lm.zeta[n]) * (E[n] / E[n - 1]);
-    QS[n - 1] = (c_(1) - part) / (c_(1) + part);
-    for (int k = n - 1; k > 1; --k) {
-        double2 qe = Q1[k] * X[k];
-        part = (c_(1) * (E[k] / E[k - 1])) * ((qe - c_(1)) / (qe + c_(1)));
-        Q1[k - 1] = (c_(1) + part) / (c_(1) - part);
-        qe = QS[k] * X[k];
-        part = ((lm.zeta[k - 1] / lm.zeta[k]) * (E[k] / E[k - 1])) * ((qe - c_(1)) / (qe + c_(1)));
-        QS[k - 1] = (c_(1) + part) / (c_(1) - part);
-    }
-    for (int k = 0; k < nl; ++k) {
-        p1[base + k] = P1[k];
-        q1[base + k] = Q1[k];
-        ps[base + k] = PS[k];
-        qs[base + k] = QS[k];
+    // value = i omega * zeta * Mu0; eta = sqrt(lambda^2 - value)  (CalcEta, green_scalar.c:30-34)
+    auto root = [&](int k) { return csqrt_d(c_(l * l) - (c_(0, lm.omega) * lm.zeta[k]) * c_(kMu0)); };
+    auto expo = [&](int k, double2 E) { return cexp_d((-2 * lm.thick[k]) * E); };    // CalcExp (green_scalar.c:36-41)
+    // the sigma recursions carry the layers' zeta, the others 1
+    const bool sig = blockIdx.z & 1;
+    auto ratio = [&](int k, int j) { return sig ? lm.zeta[k] / lm.zeta[j] : c_(1); };
+    if (blockIdx.z < 2) {
+        // P: p[1] from the top interface, then downwards (CalculatePBelow1, PlanCalculatorFast.cs:266-280)
+        double2 *out = (sig ? ps : p1) + base;
+        double2 e0 = root(0), e1 = root(1);
+        double2 v = sig ? (lm.zeta[0] * e1 - lm.zeta[1] * e0) / (lm.zeta[0] * e1 + lm.zeta[1] * e0) : (e1 - e0) / (e1 + e0);
+        out[0] = c_(0);
+        out[1] = v;
+        if (!sig) {
+            eta[base] = e0;
+            eta[base + 1] = e1;
+        }
+        for (int k = 1; k < nl - 1; ++k) {
+            e0 = e1;
+            e1 = root(k + 1);
+            const double2 pe = v * expo(k, e0);
+            const double2 part = (ratio(k + 1, k) * (e0 / e1)) * ((pe - c_(1)) / (pe + c_(1)));
+            v = (c_(1) + part) / (c_(1) - part);
+            out[k + 1] = v;
+            if (!sig) eta[base + k + 1] = e1;
+        }
+    } else {
+        // Q: q[n] = 0 at the bottom, then upwards (CalculateQ, PlanCalculatorFast.cs:292-318)
+        double2 *out = (sig ? qs : q1) + base;
+        double2 e1 = root(n), e0 = root(n - 1);                      // of layers k, k - 1
+        const double2 first = ratio(n - 1, n) * (e1 / e0);
+        double2 v = (c_(1) - first) / (c_(1) + first);
+        out[n] = c_(0);
+        if (!sig) ex[base + n] = expo(n, e1);
+        if (n > 1) out[0] = c_(0);
+        out[n - 1] = v;
+        for (int k = n - 1; k >= 0; --k) {
+            e1 = e0;
+            const double2 X = expo(k, e1);
+            if (!sig) ex[base + k] = X;
+            if (k > 0) e0 = root(k - 1);
+            if (k <= 1) continue;
+            const double2 qe = v * X;
+            const double2 part = (ratio(k - 1, k) * (e1 / e0)) * ((qe - c_(1)) / (qe + c_(1)));
+            v = (c_(1) + part) / (c_(1) - part);
+            out[k - 1] = v;
+        }
     }
 }
 
@@ -286,39 +295,41 @@ struct HankelArgs {
     double sgn[5], den;
     double2 *I;
 };
-constexpr int kHTiles = 8, kHPad = 16 * kHTiles - 1;
-constexpr int kHSteps = (kTaps - 1 + 16 * kHTiles + 15) / 16 * 4;             // k-steps of a full group
-constexpr int kHTable = kHPad + 4 * kHSteps;
-
-__global__ __launch_bounds__(256) void hankel_kernel(HankelArgs a)
+// TILES radius tiles a wave. Few rows leave most of the chip idle and a wave with 8 tiles is a chain of 2000 MFMAs:
+// then a wave takes 2 tiles, and `groups` workgroups share the radii (the rows are read again, from L2):
+// the 32 rows of a level at 128 x 128 x 32 take 21 us instead of 47, the 36 and 64 of 32 x 32 x 8 20 instead of 37.
+template <int TILES>
+__global__ __launch_bounds__(256) void hankel_kernel(HankelArgs a, int groups)
 {
-    __shared__ double h[kHTable];
+    constexpr int PAD = 16 * TILES - 1, STEPS = (kTaps - 1 + 16 * TILES + 15) / 16 * 4;   // k-steps of a full group
+    constexpr int TABLE = PAD + 4 * STEPS;
+    __shared__ double h[TABLE];
     const int it = blockIdx.y, c = blockIdx.z;
     const double *hank = (a.j0 >> c) & 1 ? a.h0 : a.h1;
-    for (int x = threadIdx.x; x < kHTable; x += blockDim.x) {
-        const int j = x - kHPad;
+    for (int x = threadIdx.x; x < TABLE; x += blockDim.x) {
+        const int j = x - PAD;
         h[x] = j >= 0 && j < kTaps ? hank[kTaps - 1 - j] : 0.0;
     }
     __syncthreads();
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-    const int p0 = (blockIdx.x * 4 + wave) * 8;
+    const int grp = blockIdx.x % groups, p0 = ((int)blockIdx.x / groups * 4 + wave) * 8;
     if (p0 >= a.np) return;
     const int n = lane & 15, kl = lane >> 4, p = p0 + (n >> 1), part = n & 1;
     const int nlam = a.nlam[it], nrho = nlam - kTaps;
     const double *u = reinterpret_cast<const double *>(
                           a.U + (((int64_t)min(p, a.np - 1) * a.nitems + it) * a.ncomp + c) * a.nlam_max) + part;
-    const double *hl = h + kHPad + kl - n;                             // H[i = n][k = kl], plus 4 step - 16 tile
-    for (int ix0 = 0; ix0 < nrho; ix0 += 16 * kHTiles) {
-        const int tiles = min(kHTiles, (nrho - ix0 + 15) / 16);
+    const double *hl = h + PAD + kl - n;                             // H[i = n][k = kl], plus 4 step - 16 tile
+    for (int ix0 = 16 * TILES * grp; ix0 < nrho; ix0 += 16 * TILES * groups) {
+        const int tiles = min(TILES, (nrho - ix0 + 15) / 16);
         const int chunks = (kTaps - 1 + 16 * tiles + 15) / 16;         // of 4 k-steps
         auto get = [&](int step) __attribute__((always_inline)) {      // past the row's end: no radius uses it
             const int k = ix0 + 4 * step + kl;
             const double v = u[2 * min(k, nlam - 1)];
             return k < nlam ? v : 0.0;
         };
-        mfma_d4 acc[kHTiles];
+        mfma_d4 acc[TILES];
 #pragma unroll
-        for (int t = 0; t < kHTiles; ++t) acc[t] = mfma_d4{0, 0, 0, 0};
+        for (int t = 0; t < TILES; ++t) acc[t] = mfma_d4{0, 0, 0, 0};
         double bn[4];
 #pragma unroll
         for (int q = 0; q < 4; ++q) bn[q] = get(q);
@@ -330,7 +341,7 @@ __global__ __launch_bounds__(256) void hankel_kernel(HankelArgs a)
             for (int q = 0; q < 4; ++q) bn[q] = get(4 * (ch + 1) + q);
             const double *hc = hl + 16 * ch;
 #pragma unroll
-            for (int t = 0; t < kHTiles; ++t) {
+            for (int t = 0; t < TILES; ++t) {
                 // radii 16 t .. 16 t + 15 use lambdas 16 t .. 16 t + 15 + 430 of this group
                 if (t < tiles && t <= ch && 16 * ch <= 16 * t + 15 + kTaps - 1) {
 #pragma unroll
@@ -339,7 +350,7 @@ __global__ __launch_bounds__(256) void hankel_kernel(HankelArgs a)
             }
         }
 #pragma unroll
-        for (int t = 0; t < kHTiles; ++t)
+        for (int t = 0; t < TILES; ++t)
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 const int ix = ix0 + 16 * t + mfma_row<double>(lane, r);
@@ -354,7 +365,14 @@ __global__ __launch_bounds__(256) void hankel_kernel(HankelArgs a)
 
 void launch_hankel(const HankelArgs &a, hipStream_t s)
 {
-    hipLaunchKernelGGL(hankel_kernel, dim3((unsigned)ceil_div(a.np, 32), a.nitems, a.ncomp), dim3(256), 0, s, a);
+    const int64_t rows = ceil_div(a.np, 32);
+    // fewer waves than SIMDs
+    if (4 * rows * a.nitems * a.ncomp < 4 * device_cus()) {
+        const int groups = (int)ceil_div(a.nrho_max, 32);
+        hipLaunchKernelGGL(hankel_kernel<2>, dim3((unsigned)(rows * groups), a.nitems, a.ncomp), dim3(256), 0, s, a, groups);
+    } else {
+        hipLaunchKernelGGL(hankel_kernel<8>, dim3((unsigned)rows, a.nitems, a.ncomp), dim3(256), 0, s, a, 1);
+    }
     XTR_LAUNCH_CHECK("hankel_kernel");
 }
 
@@ -419,6 +437,7 @@ __device__ inline Factors factors(double s, double u, double rs, double ru, doub
 struct LatArgs {
     int nx, ny, nz, npairs, nr;
     int p0;                       // first pair of this chunk
+    int width;                    // threads, and pairs, of a group
     int folded;                   // G holds blocks [Nx+1][Ny+1], else [2Nx][2Ny]
     double dx, dy;
     const double2 *segA, *segB;   // [seg][comp][pair]
@@ -546,18 +565,23 @@ __device__ __forceinline__ double2 wab(const double (&w)[WN], int c, double2 q, 
     return make_double2(fma(w[c], A.x, fma(w[c + 1], B.x, q.x)), fma(w[c], A.y, fma(w[c + 1], B.y, q.y)));
 }
 
-// One workgroup per cell and a share of the pairs. Bound by the L2 reads of the segments' coefficients (96 bytes
-// a pair and segment). At 128 x 128 x 32: 0.73 ms for both sets; 3.6 ms with every thread working out the edges'
+// One workgroup per cell and a share of the pairs; groups of `width` threads share the segments between them, and
+// their sums meet in LDS. Bound by the L2 reads of the segments' coefficients (96 bytes a pair and segment) on a
+// large grid, and on a small one by the chain of the cells next to the source, which cross up to 200 segments. At
+// 128 x 128 x 32, 256 pairs a group: 0.73 ms for both sets; 3.6 ms with every thread working out the edges'
 // geometry for its own pair, 1.16 ms with the geometry shared but one pass over the segments per edge.
+// 32 x 32 x 8 (64 and 36 pairs), 4 groups of 64: 38 us a set instead of 101 with one.
 constexpr int kCellSegs = 32;
 
-template <int ASYM>
+template <int ASYM, bool GROUPS>
 __global__ __launch_bounds__(256) void lateral_kernel(LatArgs a)
 {
     __shared__ CellWeights<kCellSegs> cw;
     const int64_t cell = blockIdx.x;
     const int i = (int)(cell / a.ny), j = (int)(cell % a.ny);
-    const int p = blockIdx.y * blockDim.x + threadIdx.x, np = a.npairs;
+    const int grp = GROUPS ? threadIdx.x / a.width : 0, tp = threadIdx.x - grp * a.width;
+    const int groups = GROUPS ? blockDim.x / a.width : 1;
+    const int p = blockIdx.y * a.width + tp, np = a.npairs;
     cw.ends(threadIdx.x, a.radii, a.nr, a.dx * (i - 0.5), a.dx * (i + 0.5), a.dy * (j - 0.5), a.dy * (j + 0.5));
     __syncthreads();
     int lo, hi;
@@ -575,7 +599,7 @@ __global__ __launch_bounds__(256) void lateral_kernel(LatArgs a)
         __syncthreads();
         if (p < np)
 #pragma unroll 2
-            for (int k = 0; k < n; ++k) {
+            for (int k = grp; k < n; k += groups) {
                 const double (&wx)[WN] = cw.w[k][0], (&wy)[WN] = cw.w[k][1];
                 const int64_t o = (int64_t)(seg0 + k) * (ASYM ? 1 : 3) * np + p;
                 if constexpr (ASYM) {      // edges along y give xz, along x yz (AddToQBuff..., D1)
@@ -594,7 +618,23 @@ __global__ __launch_bounds__(256) void lateral_kernel(LatArgs a)
             }
         __syncthreads();                                       // the weights are read
     }
-    if (p >= np) return;
+    if constexpr (GROUPS) {
+        static_assert(sizeof(cw.f) >= 2 * 256 * sizeof(double2), "two components of 256 threads");
+        double2 *red = reinterpret_cast<double2 *>(cw.f);
+#pragma unroll
+        for (int t = 0; t < nq; t += 2) {
+            if (t) __syncthreads();
+            red[threadIdx.x] = G[t];
+            red[256 + threadIdx.x] = G[t + 1];
+            __syncthreads();
+            if (grp == 0)
+                for (int o = a.width; o < (int)blockDim.x; o += a.width) {
+                    G[t] = cadd<double>(G[t], red[o + tp]);
+                    G[t + 1] = cadd<double>(G[t + 1], red[256 + o + tp]);
+                }
+        }
+    }
+    if (p >= np || grp > 0) return;
     // write G(i,j) and, into a full tensor, its mirror images (GreenTensorFftPopulator.cs:88-148); of a folded
     // one the FFT forms the images from the parities as it reads
     const int64_t nx2 = 2LL * a.nx, ny2 = a.folded ? a.ny + 1 : 2LL * a.ny;
@@ -793,8 +833,8 @@ struct PlanHost {
         d.lm = (const LayerModel *)(base + at[6]);
         double2 **aux[6] = {&d.eta, &d.ex, &d.p1, &d.q1, &d.ps, &d.qs};
         for (auto *a : aux) *a = work.take<double2>(auxn);
-        dim3 grid((unsigned)ceil_div(nlam_max, 128), nitems);
-        hipLaunchKernelGGL(layer_aux_kernel, grid, dim3(128), 0, s, d.lm, nitems, nlam_max, d.nlam, d.lam, d.eta, d.ex,
+        dim3 grid((unsigned)ceil_div(nlam_max, 64), nitems, 4);
+        hipLaunchKernelGGL(layer_aux_kernel, grid, dim3(64), 0, s, d.lm, nitems, nlam_max, d.nlam, d.lam, d.eta, d.ex,
                            d.p1, d.q1, d.ps, d.qs);
         XTR_LAUNCH_CHECK("layer_aux_kernel");
         return d;
@@ -924,10 +964,21 @@ void build_green_atoa(const GreenInput &in, GreenScratch &work, double2 *G, bool
                 for (int t = 0; t < 3; ++t) { la.xs[t] = 1; la.ys[t] = 1; }
                 la.xs[3] = -1; la.ys[3] = -1;
             }
-            const int wgs = (int)ceil_div(np, 256);                  // of a cell, with equal shares of the pairs
-            const dim3 grid((unsigned)((int64_t)g.nx * g.ny), wgs), nt((unsigned)(ceil_div(ceil_div(np, wgs), 64) * 64));
-            if (asym) hipLaunchKernelGGL(lateral_kernel<1>, grid, nt, 0, s, la);
-            else hipLaunchKernelGGL(lateral_kernel<0>, grid, nt, 0, s, la);
+            const int64_t cells = (int64_t)g.nx * g.ny;
+            int wgs = (int)ceil_div(np, 256);                        // of a cell, with equal shares of the pairs
+            la.width = (int)(ceil_div(ceil_div(np, wgs), 64) * 64);
+            int threads = la.width;
+            // Few pairs, or too few cells for 4 workgroups a CU: 256 threads in groups of as many as the pairs take,
+            // and fewer until the cells fill the chip.
+            if (la.width <= 128 || cells * wgs < 4 * device_cus()) {
+                threads = la.width = 256;
+                while (la.width > 16 && (la.width / 2 >= np || cells * ceil_div(np, la.width) < 4 * device_cus())) la.width /= 2;
+                wgs = (int)ceil_div(np, la.width);
+            }
+            const dim3 grid((unsigned)cells, wgs), nt((unsigned)threads);
+            auto run = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, nt, 0, s, la); };
+            if (threads > la.width) asym ? run(lateral_kernel<1, true>) : run(lateral_kernel<0, true>);
+            else asym ? run(lateral_kernel<1, false>) : run(lateral_kernel<0, false>);
             XTR_LAUNCH_CHECK("lateral_kernel");
         }
     }
@@ -1082,87 +1133,143 @@ struct AoArgs {
     const double *radii;
     double2 *G;                   // [2Nx][2Ny][components][nz], components as in atoo_components
     int folded;                   // [Nx+1][Ny+1][components][nz], offsets i, j >= 0 only
+    int width;                    // lanes of a group: a power of 2, the layers or 64
+    int i0, i1, j0, j1;           // the offsets near the receiver, [i0, i1) x [j0, j1)
 };
 
-// One wave per lateral offset (i, j) in (-Nx, Nx) x (-Ny, Ny), or its non-negative quadrant where the tensor is
-// folded (a level that is not shifted), lanes the transmitter layers: the four edge
-// integrals of RunAlongX / RunAlongY (GreenTensorCalculator.cs:192-281), written at TransformI/J
-// (AtoOLevelGreenTensorCalculator.cs:106-117). The wave forms its offset's weights itself (CellWeights), 8 segments
-// at a time, a thread for each (segment, stretch). At 128 x 128 x 32, all offsets: 0.26 and 0.22 ms (0.64 ms each
-// with every thread working out the geometry); the quadrant: 0.12 and 0.11 ms.
-constexpr int kAoWaves = 4, kAoSegs = 8;
+// The four edge integrals of RunAlongX / RunAlongY (GreenTensorCalculator.cs:192-281) for each lateral offset (i, j)
+// in (-Nx, Nx) x (-Ny, Ny), or its non-negative quadrant where the tensor is folded (a level that is not shifted),
+// written at TransformI/J (AtoOLevelGreenTensorCalculator.cs:106-117). A team of waves owns an offset: it forms its
+// weights (CellWeights), 8 segments a wave at a time, a thread for each (segment, stretch), and sums over the
+// segments in groups of `width` lanes, lane = transmitter layer, each group its own segments.
+// Bound by the chain over the segments of the offsets next to the receiver, up to 200 of some 1500 where one 8 cells
+// away crosses 22: those within kAoNear cells are shared by the 4 waves of a workgroup, which come first; the others
+// take a wave each. 128 x 128 x 32, folded: 60 (electric) and 50 us; 120 and 114 with a wave for every offset, and
+// there 0.64 ms each over all offsets with every thread working out the geometry, 0.26 and 0.22 with weights.
+constexpr int kAoWaves = 4, kAoSegs = 8, kAoNear = 8;
 
-template <int ELECTRIC>
-__global__ __launch_bounds__(64 * kAoWaves) void atoo_lateral_kernel(AoArgs a)
+// Sums of one offset for the layers tr0 .. tr0 + width - 1, complete in the first `width` lanes of the team's first wave
+template <int ELECTRIC, int TEAM, typename Sync>
+__device__ __forceinline__ void ao_sums(const AoArgs &a, CellWeights<kAoSegs * TEAM> &cw, int tid, int lo, int hi, int tr0,
+                                        double2 *G, const Sync &sync)
 {
-    __shared__ CellWeights<kAoSegs> all[kAoWaves];
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-    CellWeights<kAoSegs> &cw = all[wave];
-    const int ncy = a.folded ? a.ny : 2 * a.ny - 1, cells = (a.folded ? a.nx : 2 * a.nx - 1) * ncy;
-    const int cell = blockIdx.x * kAoWaves + wave;
-    if (cell >= cells) return;                                  // waves do not meet at a barrier
-    const int i = cell / ncy - (a.folded ? 0 : a.nx - 1), j = cell % ncy - (a.folded ? 0 : a.ny - 1);
-    // LDS writes of this wave become visible to it in order; the fence only keeps the compiler from moving them
-    auto sync = [] { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); __builtin_amdgcn_wave_barrier(); };
-    cw.ends(lane, a.radii, a.nr, a.dx * (i - 0.5) - a.xs, a.dx * (i + 0.5) - a.xs, a.dy * (j - 0.5) - a.ys,
+    constexpr int nc = ELECTRIC ? 5 : 4, no = ELECTRIC ? 8 : 7, SEGS = kAoSegs * TEAM;
+    const int lane = tid & 63, tr = tr0 + (lane & (a.width - 1)), grp = tid / a.width, groups = 64 * TEAM / a.width;
+#pragma unroll
+    for (int t = 0; t < no; ++t) G[t] = c_(0);
+    for (int seg0 = lo; seg0 <= hi; seg0 += SEGS) {
+        const int n = min(SEGS, hi - seg0 + 1);
+        cw.factors_of(tid, 64 * TEAM, a.radii, seg0, n);
+        sync();
+        cw.sum(tid, 64 * TEAM, n);
+        sync();
+        if (tr < a.nz)
+            for (int k = grp; k < n; k += groups) {
+                const double (&wx)[WN] = cw.w[k][0], (&wy)[WN] = cw.w[k][1];
+                const double2 *A = a.segA + (int64_t)(seg0 + k) * nc * a.nz + tr;
+                const double2 *B = a.segB + (int64_t)(seg0 + k) * nc * a.nz + tr;
+                double2 sa[nc], sb[nc];                         // I1 .. I5 (I4)
+#pragma unroll
+                for (int c = 0; c < nc; ++c) {
+                    sa[c] = A[(int64_t)c * a.nz];
+                    sb[c] = B[(int64_t)c * a.nz];
+                }
+                // AddToQBuffAlong{X,Y}{Electric,Magnetic} (GreenTensorCalculator.cs:505-560) with the signs of the
+                // QSigns tables (QSign.cs:31-38)
+                const double nxw[WN] = {0, 0, -wx[W2A], -wx[W2B], 0, 0}, nyw[WN] = {0, 0, -wy[W2A], -wy[W2B], 0, 0};
+                if constexpr (ELECTRIC) {                       // xx yy zz xy xz yz zx zy
+                    G[0] = wab(nyw, W2A, wab(wx, W2A, G[0], sa[0], sb[0]), sa[1], sb[1]);
+                    G[1] = wab(nxw, W2A, wab(wy, W2A, G[1], sa[0], sb[0]), sa[1], sb[1]);
+                    G[2] = wab(nyw, W2A, wab(nxw, W2A, G[2], sa[4], sb[4]), sa[4], sb[4]);
+                    G[3] = wab(wy, W3A, wab(wx, W3A, G[3], sa[1], sb[1]), sa[0], sb[0]);
+                    G[4] = wab(wy, W1A, G[4], sa[2], sb[2]);
+                    G[5] = wab(wx, W1A, G[5], sa[2], sb[2]);
+                    G[6] = wab(wy, W1A, G[6], sa[3], sb[3]);
+                    G[7] = wab(wx, W1A, G[7], sa[3], sb[3]);
+                } else {                                        // xx xy yx xz yz zx zy
+                    G[0] = wab(wy, W3A, wab(wx, W3A, G[0], sa[1], sb[1]), sa[0], sb[0]);
+                    G[1] = wab(wy, W2A, wab(nxw, W2A, G[1], sa[1], sb[1]), sa[0], sb[0]);
+                    G[2] = wab(nyw, W2A, wab(wx, W2A, G[2], sa[0], sb[0]), sa[1], sb[1]);
+                    G[3] = wab(wx, W1A, G[3], sa[2], sb[2]);
+                    G[4] = wab(wy, W1A, G[4], sa[2], sb[2]);
+                    G[5] = wab(wx, W1A, G[5], sa[3], sb[3]);
+                    G[6] = wab(wy, W1A, G[6], sa[3], sb[3]);
+                }
+            }
+        sync();                                                 // the weights are read
+    }
+#pragma unroll
+    for (int t = 0; t < no; ++t)
+        for (int off = a.width; off < 64; off <<= 1) {
+            G[t].x += __shfl_xor(G[t].x, off, 64);
+            G[t].y += __shfl_xor(G[t].y, off, 64);
+        }
+    if constexpr (TEAM > 1) {
+        static_assert(sizeof(cw.f) >= (TEAM - 1) * 4 * 64 * sizeof(double2), "four components of the other waves");
+        double2 *red = reinterpret_cast<double2 *>(cw.f);
+#pragma unroll
+        for (int t0 = 0; t0 < no; t0 += 4) {
+            const int wave = tid >> 6;
+            if (wave > 0)
+#pragma unroll
+                for (int t = t0; t < t0 + 4 && t < no; ++t) red[((wave - 1) * 4 + t - t0) * 64 + lane] = G[t];
+            sync();
+            if (wave == 0)
+#pragma unroll
+                for (int t = t0; t < t0 + 4 && t < no; ++t)
+#pragma unroll
+                    for (int w = 0; w < TEAM - 1; ++w) G[t] = cadd<double>(G[t], red[(w * 4 + t - t0) * 64 + lane]);
+            sync();
+        }
+    }
+}
+
+template <int ELECTRIC, int TEAM, typename Sync>
+__device__ __forceinline__ void ao_offset(const AoArgs &a, CellWeights<kAoSegs * TEAM> &cw, int tid, int i, int j,
+                                          const Sync &sync)
+{
+    constexpr int no = ELECTRIC ? 8 : 7;
+    cw.ends(tid, a.radii, a.nr, a.dx * (i - 0.5) - a.xs, a.dx * (i + 0.5) - a.xs, a.dy * (j - 0.5) - a.ys,
             a.dy * (j + 0.5) - a.ys);
     sync();
     int lo, hi;
     cw.range(lo, hi);
-    constexpr int nc = ELECTRIC ? 5 : 4, no = ELECTRIC ? 8 : 7;
     const int64_t ti = i < 0 ? 2 * a.nx + i : i, tj = j < 0 ? 2 * a.ny + j : j;
-    for (int tr0 = 0; tr0 < a.nz; tr0 += 64) {
-        const int tr = tr0 + lane;
+    for (int tr0 = 0; tr0 < a.nz; tr0 += a.width) {
         double2 G[no];
-#pragma unroll
-        for (int t = 0; t < no; ++t) G[t] = c_(0);
-        for (int seg0 = lo; seg0 <= hi; seg0 += kAoSegs) {
-            const int n = min(kAoSegs, hi - seg0 + 1);
-            cw.factors_of(lane, 64, a.radii, seg0, n);
-            sync();
-            cw.sum(lane, 64, n);
-            sync();
-            if (tr < a.nz)
-                for (int k = 0; k < n; ++k) {
-                    const double (&wx)[WN] = cw.w[k][0], (&wy)[WN] = cw.w[k][1];
-                    const double2 *A = a.segA + (int64_t)(seg0 + k) * nc * a.nz + tr;
-                    const double2 *B = a.segB + (int64_t)(seg0 + k) * nc * a.nz + tr;
-                    double2 sa[nc], sb[nc];                     // I1 .. I5 (I4)
-#pragma unroll
-                    for (int c = 0; c < nc; ++c) {
-                        sa[c] = A[(int64_t)c * a.nz];
-                        sb[c] = B[(int64_t)c * a.nz];
-                    }
-                    // AddToQBuffAlong{X,Y}{Electric,Magnetic} (GreenTensorCalculator.cs:505-560) with the signs of the
-                    // QSigns tables (QSign.cs:31-38)
-                    const double nxw[WN] = {0, 0, -wx[W2A], -wx[W2B], 0, 0}, nyw[WN] = {0, 0, -wy[W2A], -wy[W2B], 0, 0};
-                    if constexpr (ELECTRIC) {                   // xx yy zz xy xz yz zx zy
-                        G[0] = wab(nyw, W2A, wab(wx, W2A, G[0], sa[0], sb[0]), sa[1], sb[1]);
-                        G[1] = wab(nxw, W2A, wab(wy, W2A, G[1], sa[0], sb[0]), sa[1], sb[1]);
-                        G[2] = wab(nyw, W2A, wab(nxw, W2A, G[2], sa[4], sb[4]), sa[4], sb[4]);
-                        G[3] = wab(wy, W3A, wab(wx, W3A, G[3], sa[1], sb[1]), sa[0], sb[0]);
-                        G[4] = wab(wy, W1A, G[4], sa[2], sb[2]);
-                        G[5] = wab(wx, W1A, G[5], sa[2], sb[2]);
-                        G[6] = wab(wy, W1A, G[6], sa[3], sb[3]);
-                        G[7] = wab(wx, W1A, G[7], sa[3], sb[3]);
-                    } else {                                    // xx xy yx xz yz zx zy
-                        G[0] = wab(wy, W3A, wab(wx, W3A, G[0], sa[1], sb[1]), sa[0], sb[0]);
-                        G[1] = wab(wy, W2A, wab(nxw, W2A, G[1], sa[1], sb[1]), sa[0], sb[0]);
-                        G[2] = wab(nyw, W2A, wab(wx, W2A, G[2], sa[0], sb[0]), sa[1], sb[1]);
-                        G[3] = wab(wx, W1A, G[3], sa[2], sb[2]);
-                        G[4] = wab(wy, W1A, G[4], sa[2], sb[2]);
-                        G[5] = wab(wx, W1A, G[5], sa[3], sb[3]);
-                        G[6] = wab(wy, W1A, G[6], sa[3], sb[3]);
-                    }
-                }
-            sync();                                             // the weights are read
-        }
-        if (tr < a.nz) {
-            double2 *dst = a.G + (ti * (a.folded ? a.ny + 1 : 2 * a.ny) + tj) * (int64_t)(no * a.nz) + tr;
+        ao_sums<ELECTRIC, TEAM>(a, cw, tid, lo, hi, tr0, G, sync);
+        if (tid < a.width && tr0 + tid < a.nz) {
+            double2 *dst = a.G + (ti * (a.folded ? a.ny + 1 : 2 * a.ny) + tj) * (int64_t)(no * a.nz) + tr0 + tid;
 #pragma unroll
             for (int t = 0; t < no; ++t) dst[(int64_t)t * a.nz] = G[t];
         }
     }
+}
+
+template <int ELECTRIC>
+__global__ __launch_bounds__(64 * kAoWaves) void atoo_lateral_kernel(AoArgs a)
+{
+    __shared__ union Weights {
+        CellWeights<kAoSegs> one[kAoWaves];
+        CellWeights<kAoSegs * kAoWaves> team;
+    } cw;
+    const int nny = a.j1 - a.j0, near = (a.i1 - a.i0) * nny;     // offsets [i0, i1) x [j0, j1)
+    if ((int)blockIdx.x < near) {
+        ao_offset<ELECTRIC, kAoWaves>(a, cw.team, threadIdx.x, a.i0 + blockIdx.x / nny, a.j0 + blockIdx.x % nny,
+                                      [] { __syncthreads(); });
+        return;
+    }
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int ncy = a.folded ? a.ny : 2 * a.ny - 1, cells = (a.folded ? a.nx : 2 * a.nx - 1) * ncy;
+    const int cell = ((int)blockIdx.x - near) * kAoWaves + wave;
+    if (cell >= cells) return;                                  // waves do not meet at a barrier
+    const int i = cell / ncy - (a.folded ? 0 : a.nx - 1), j = cell % ncy - (a.folded ? 0 : a.ny - 1);
+    if (i >= a.i0 && i < a.i1 && j >= a.j0 && j < a.j1) return;
+    // LDS writes of this wave become visible to it in order; the fence only keeps the compiler from moving them
+    ao_offset<ELECTRIC, 1>(a, cw.one[wave], lane, i, j, [] {
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+    });
 }
 
 }  // namespace
@@ -1258,7 +1365,17 @@ void build_green_atoo_level(const GreenInput &in, GreenScratch &work, double lev
     a.folded = folded ? 1 : 0;
     if (!folded) XTR_CHECK(hipMemsetAsync(G, 0, (size_t)g.L() * ntc * nz * sizeof(double2), s));
     const int cells = folded ? g.nx * g.ny : (2 * g.nx - 1) * (2 * g.ny - 1);
-    const dim3 grid((unsigned)ceil_div(cells, kAoWaves)), nt(64 * kAoWaves);
+    for (a.width = 8; a.width < nz && a.width < 64;) a.width *= 2;
+    // within kAoNear cells of the receiver, as far as the offsets go (i1 = i0 where none is)
+    auto window = [&](double shift, double d, int n, int &from, int &to) {
+        const double c = std::fmin(std::fmax(std::nearbyint(shift / d), -2.0 * n), 2.0 * n);
+        const int first = folded ? 0 : 1 - n;
+        from = std::min(std::max((int)c - kAoNear + 1, first), n);
+        to = std::max(std::min((int)c + kAoNear, n), from);
+    };
+    window(a.xs, a.dx, g.nx, a.i0, a.i1);
+    window(a.ys, a.dy, g.ny, a.j0, a.j1);
+    const dim3 grid((unsigned)((a.i1 - a.i0) * (a.j1 - a.j0) + ceil_div(cells, kAoWaves))), nt(64 * kAoWaves);
     if (electric) hipLaunchKernelGGL(atoo_lateral_kernel<1>, grid, nt, 0, s, a);
     else hipLaunchKernelGGL(atoo_lateral_kernel<0>, grid, nt, 0, s, a);
     XTR_LAUNCH_CHECK("atoo_lateral_kernel");
