@@ -20,6 +20,7 @@ ARCH = "gfx950"
 
 SOURCES = ["op_fft_forward.hip", "op_fft_inverse.hip", "op_kernels.hip", "tensor_fft.hip",
            "krylov_kernels.hip", "green_assembly.hip", "obs_kernels.hip", "learned_kernels.hip", "probe_kernels.hip", "xtr_api.cpp"]
+SOURCES += ["contract_direct.hip"]
 SOURCES += [f"contract_block_{t}_{r}.hip" for t in ("c128", "c64") for r in "abcd"]
 
 COMMON = ["-O3", "-fPIC", "-std=c++17", f"--offload-arch={ARCH}",

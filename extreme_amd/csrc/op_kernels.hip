@@ -977,11 +977,17 @@ static bool contract_fold64(const ApplyArgs &a, hipStream_t s)
     return true;
 }
 
-// Folded tensor, a block that fits in LDS (contract_block.h); 1-8 right-hand sides.
+// Folded tensor, a block that fits in LDS (contract_block.h), or a wave per block (contract_direct.hip) where the
+// blocks are small and enough of them fill the chip; 1-8 right-hand sides.
 static bool contract_block(const ApplyArgs &a, hipStream_t s)
 {
     // byte offsets within one right-hand side's spectrum are 32-bit
     if (!a.folded || a.nrhs < 1 || a.nrhs > kMaxRhs || contract_force_generic() || a.g.M() * 16 > 0xffffffffLL) return false;
+    // Up to 10 layers; a wave per block needs 6 blocks a CU (2 up to 5 layers, one row tile). Times of the block
+    // kernel over those of the wave's, 1 to 8 right-hand sides, complex128: nz = 8 at 120 x 100 1.04-1.14, 64 x 64
+    // 0.99-1.19, 32 x 32 0.92-1.05, 16 x 16 0.79-1.10; nz = 5 1.44-1.78, 1.36-1.47, 1.12-1.32, 0.98-1.16. Past 10
+    // layers 48 x 40 x 12 0.95-1.17, 64 x 64 x 16 0.70-0.97.
+    if (a.g.nz <= kDirectMostLayers && a.g.Lq() >= (a.g.nz <= 5 ? 2 : 6) * device_cus() && contract_direct(a, s)) return true;
     using Range = bool (*)(const ApplyArgs &, hipStream_t);
     static const Range c128[] = {contract_block_c128_a, contract_block_c128_b, contract_block_c128_c, contract_block_c128_d};
     static const Range c64[] = {contract_block_c64_a, contract_block_c64_b, contract_block_c64_c, contract_block_c64_d};

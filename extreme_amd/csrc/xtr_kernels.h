@@ -134,6 +134,9 @@ bool contract_block_c64_a(const ApplyArgs &a, hipStream_t s);
 bool contract_block_c64_b(const ApplyArgs &a, hipStream_t s);
 bool contract_block_c64_c(const ApplyArgs &a, hipStream_t s);
 bool contract_block_c64_d(const ApplyArgs &a, hipStream_t s);
+// the same for up to kDirectMostLayers layers, a wave per block (contract_direct.hip)
+constexpr int kDirectMostLayers = 10;
+bool contract_direct(const ApplyArgs &a, hipStream_t s);
 int device_cus();            // compute units of the current device
 void launch_inv_x(const ApplyArgs &a, hipStream_t s);
 void launch_inv_y(const ApplyArgs &a, hipStream_t s);
