@@ -39,21 +39,20 @@ struct IoFwdY {
     int nx, ny, nz;
     __device__ cplx<T> load(int rhs, int64_t c, int p) const
     {
-        const int64_t C = 3LL * nz;
-        if (c >= nx * C || p >= ny) return mk<T>(0, 0);
-        const int64_t i = c / C, col = c % C;
-        const int k = (int)(col % nz);
-        const int64_t ij = i * ny + p;
+        const unsigned C = 3u * nz;
+        if (c >= (int64_t)nx * C || p >= ny) return mk<T>(0, 0);
+        const unsigned i = (unsigned)c / C, col = (unsigned)c - i * C, k = col % (unsigned)nz;
+        const int64_t ij = (int64_t)i * ny + p;
         const cplx<V> *x = reinterpret_cast<const cplx<V> *>(v.x[rhs]);
         double2 rx = cmul<double>(v.R[rhs][ij * nz + k], widen(x[ij * C + col]));
         return from_d<T>(cscale<double>(rx, f[k]));
     }
     __device__ void store(int rhs, int64_t c, int p, cplx<T> val) const
     {
-        const int64_t C = 3LL * nz;
-        if (c >= nx * C) return;
-        const int64_t i = c / C, col = c % C;
-        buf[rhs * M + (i * 2 * ny + p) * C + col] = val;
+        const unsigned C = 3u * nz;
+        if (c >= (int64_t)nx * C) return;
+        const unsigned i = (unsigned)c / C, col = (unsigned)c - i * C;
+        buf[rhs * M + ((int64_t)i * 2 * ny + p) * C + col] = val;
     }
 };
 

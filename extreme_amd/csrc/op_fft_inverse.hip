@@ -38,18 +38,17 @@ struct IoInvY {
     int nx, ny, nz, type;
     __device__ cplx<T> load(int rhs, int64_t c, int p) const
     {
-        const int64_t C = 3LL * nz;
-        if (c >= nx * C) return mk<T>(0, 0);
-        const int64_t i = c / C, col = c % C;
-        return buf[rhs * M + (i * 2 * ny + p) * C + col];
+        const unsigned C = 3u * nz;
+        if (c >= (int64_t)nx * C) return mk<T>(0, 0);
+        const unsigned i = (unsigned)c / C, col = (unsigned)c - i * C;
+        return buf[rhs * M + ((int64_t)i * 2 * ny + p) * C + col];
     }
     __device__ void store(int rhs, int64_t c, int p, cplx<T> val) const
     {
-        const int64_t C = 3LL * nz;
-        if (c >= nx * C || p >= ny) return;
-        const int64_t i = c / C, col = c % C;
-        const int k = (int)(col % nz);
-        const int64_t ij = i * ny + p, t = ij * C + col;
+        const unsigned C = 3u * nz;
+        if (c >= (int64_t)nx * C || p >= ny) return;
+        const unsigned i = (unsigned)c / C, col = (unsigned)c - i * C, k = col % (unsigned)nz;
+        const int64_t ij = (int64_t)i * ny + p, t = ij * C + col;
         double2 conv;
         if constexpr (sizeof(T) == 8) conv = cscale<double>(val, b[k]);
         else conv = cscale<double>(to_d(val), b[k]);

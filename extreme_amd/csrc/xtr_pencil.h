@@ -160,7 +160,8 @@ __device__ inline void fft_stage(cplx<T> *s, const cplx<T> *tw, int tid)
 // ---- load/store policies -------------------------------------------------------------------
 
 // Generic strided pencils of one array per right-hand side. Column c lives at
-// (c / cpr) * row_stride + (c % cpr); point p at + p * pstride.
+// (c / cpr) * row_stride + (c % cpr); point p at + p * pstride. Columns fit 32 bits (a division of 64 takes
+// several times the instructions).
 template <typename T>
 struct IoPlain {
     cplx<T> *buf;
@@ -169,7 +170,8 @@ struct IoPlain {
     int n_in, n_out;
     __device__ int64_t addr(int rhs, int64_t c, int p) const
     {
-        return rhs * rhs_stride + (c / cpr) * row_stride + (c % cpr) + (int64_t)p * pstride;
+        const unsigned col = (unsigned)c, per = (unsigned)cpr, row = col / per;
+        return rhs * rhs_stride + row * row_stride + (col - row * per) + (int64_t)p * pstride;
     }
     __device__ cplx<T> load(int rhs, int64_t c, int p) const
     {
