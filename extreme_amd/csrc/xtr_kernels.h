@@ -137,6 +137,9 @@ bool contract_block_c64_d(const ApplyArgs &a, hipStream_t s);
 // the same for up to kDirectMostLayers layers, a wave per block (contract_direct.hip)
 constexpr int kDirectMostLayers = 10;
 bool contract_direct(const ApplyArgs &a, hipStream_t s);
+// and for up to kRowsMost rows (3nz), a wave per 16 rows (contract_direct.hip)
+constexpr int kRowsMost = 256;
+bool contract_rows(const ApplyArgs &a, hipStream_t s);
 int device_cus();            // compute units of the current device
 void launch_inv_x(const ApplyArgs &a, hipStream_t s);
 void launch_inv_y(const ApplyArgs &a, hipStream_t s);
