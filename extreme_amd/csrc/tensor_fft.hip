@@ -17,8 +17,8 @@ void launch_fft2_plain(double2 *data, int n1, int n2, int64_t ncols, const doubl
     IoTensor y{{data, 0, (int64_t)n1 * ncols, ncols, (int64_t)n2 * ncols, ncols, n2, n2}};
     // along n1: columns (i2, c) flattened, pencil stride n2*ncols
     IoTensor x{{data, 0, (int64_t)n2 * ncols, (int64_t)n2 * ncols, 0, (int64_t)n2 * ncols, n1, n1}};
-    launch_pencil<double, -1, IoTensor, false>(n2, y, (int64_t)n1 * ncols, 1, tw2, s, tile_of(n2));
-    launch_pencil<double, -1, IoTensor, false>(n1, x, (int64_t)n2 * ncols, 1, tw1, s, tile_of(n1));
+    launch_pencil<double, -1, IoTensor, TILES_TWO>(n2, y, (int64_t)n1 * ncols, 1, tw2, s, tile_of(n2));
+    launch_pencil<double, -1, IoTensor, TILES_TWO>(n1, x, (int64_t)n2 * ncols, 1, tw1, s, tile_of(n1));
 }
 
 // Pencils of a folded Green tensor in its own buffer [Nx+1][Ny+1][gblk]: points p < half hold the values at
@@ -72,6 +72,11 @@ struct LevelParity {
     __device__ double sign(int o, int axis) const { return (axis == 0 ? odd[0] : odd[1]) >> (o / nz) & 1 ? -1.0 : 1.0; }
 };
 
+// Half the columns of the default tile, so more workgroups a CU, or register pencils, a pass at nz = 32 (16, 16 and
+// 8 from 192 points): 96 points 74 us (default tile 77), 128 135 (165; registers 148), 192 74 (80), 256 153 (174;
+// registers 174), 512 196 (283; registers 147); at 64 points 34, 32 and 32.
+static int mirror_tile(int p) { return p == 64 || p == 512 ? FFT_TILE_REG : p > 64 ? FFT_TILE_NARROW : FFT_TILE_DEFAULT; }
+
 template <class Parity>
 static void fft2_mirror(double2 *folded, int nx, int ny, int64_t gb, const Parity &par, const double2 *tw_x,
                         const double2 *tw_y, hipStream_t s)
@@ -80,8 +85,8 @@ static void fft2_mirror(double2 *folded, int nx, int ny, int64_t gb, const Parit
     const int64_t row = (ny + 1) * gb;
     const Io y{{folded, 0, nx * gb, gb, row, gb, 0, 0}, par, (int)gb, ny, 1};
     const Io x{{folded, 0, row, row, 0, row, 0, 0}, par, (int)gb, nx, 0};
-    launch_pencil<double, -1, Io, false>(2 * ny, y, nx * gb, 1, tw_y, s, tile_of(2 * ny));
-    launch_pencil<double, -1, Io, false>(2 * nx, x, row, 1, tw_x, s, tile_of(2 * nx));
+    launch_pencil<double, -1, Io, TILES_NARROW>(2 * ny, y, nx * gb, 1, tw_y, s, mirror_tile(2 * ny));
+    launch_pencil<double, -1, Io, TILES_NARROW>(2 * nx, x, row, 1, tw_x, s, mirror_tile(2 * nx));
 }
 
 void launch_fft2_mirror(double2 *folded, const Geom &g, const double2 *tw_x, const double2 *tw_y, hipStream_t s)
@@ -121,8 +126,8 @@ void launch_fft2_padded(const double2 *src, double2 *spec, const Geom &g, int C,
     const int64_t nc = 2LL * g.ny * C;
     const IoPadY y{src, spec, g.nx, g.ny, C};
     const IoTensor x{{spec, 0, nc, nc, 0, nc, g.nx, 2 * g.nx}};
-    launch_pencil<double, -1, IoPadY, false>(2 * g.ny, y, (int64_t)g.nx * C, 1, tw_y, s, tile_of(2 * g.ny));
-    launch_pencil<double, -1, IoTensor, false>(2 * g.nx, x, nc, 1, tw_x, s, tile_of(2 * g.nx));
+    launch_pencil<double, -1, IoPadY, TILES_TWO>(2 * g.ny, y, (int64_t)g.nx * C, 1, tw_y, s, tile_of(2 * g.ny));
+    launch_pencil<double, -1, IoTensor, TILES_TWO>(2 * g.nx, x, nc, 1, tw_x, s, tile_of(2 * g.nx));
 }
 
 // Backward transform of spec [2Nx][2Ny][C], cropped to [Nx][Ny][C] and scaled (ToOCalculator.cs:38-42, 159-172):
@@ -152,8 +157,8 @@ void launch_fft2_cropped(double2 *spec, double2 *dst, const Geom &g, int C, doub
     const int64_t nc = 2LL * g.ny * C;
     const IoTensor x{{spec, 0, nc, nc, 0, nc, 2 * g.nx, g.nx}};
     const IoCropY y{spec, dst, g.nx, g.ny, C, scale};
-    launch_pencil<double, +1, IoTensor, false>(2 * g.nx, x, nc, 1, tw_x, s, tile_of(2 * g.nx));
-    launch_pencil<double, +1, IoCropY, false>(2 * g.ny, y, (int64_t)g.nx * C, 1, tw_y, s, tile_of(2 * g.ny));
+    launch_pencil<double, +1, IoTensor, TILES_TWO>(2 * g.nx, x, nc, 1, tw_x, s, tile_of(2 * g.nx));
+    launch_pencil<double, +1, IoCropY, TILES_TWO>(2 * g.ny, y, (int64_t)g.nx * C, 1, tw_y, s, tile_of(2 * g.ny));
 }
 
 }  // namespace xtr

@@ -364,9 +364,10 @@ constexpr int reg_cols_of(int tile)
     return P * 2 * d * (int)sizeof(cplx<T>) <= 65536 ? 2 * d : d / 2;
 }
 
-// TUNED: every tile (the apply's passes, which measure them); otherwise the default and the register
-// pencil of the default column count.
-template <typename T, int DIR, class IO, bool TUNED = true>
+// TILES_ALL: every tile (the apply's passes, which measure them); otherwise the default, the register pencil of the
+// default column count and, with TILES_NARROW, the narrow tile.
+enum { TILES_TWO, TILES_NARROW, TILES_ALL };
+template <typename T, int DIR, class IO, int TILES = TILES_ALL>
 void launch_pencil(int P, const IO &io, int64_t ncols, int nrhs, const void *tw, hipStream_t s, int tile)
 {
     auto go = [&](auto pc) {
@@ -389,7 +390,7 @@ void launch_pencil(int P, const IO &io, int64_t ncols, int nrhs, const void *tw,
                     hipLaunchKernelGGL((pencil_fft_reg_kernel<T, PP, TC, DIR, IO, NT>), grid, dim3(NT), 0, s, io,
                                        (const cplx<T> *)tw);
                 };
-                if constexpr (TUNED) {
+                if constexpr (TILES == TILES_ALL) {
                     if (tile == FFT_TILE_REG_ALT) {
                         reg(std::integral_constant<int, reg_cols_of<T, PP>(FFT_TILE_REG_ALT)>{});
                         return;
@@ -399,9 +400,11 @@ void launch_pencil(int P, const IO &io, int64_t ncols, int nrhs, const void *tw,
                 return;
             }
         }
-        if constexpr (TUNED) {
-            if (tile == FFT_TILE_WIDE && TW != TD) return run(std::integral_constant<int, TW>{}, T256{});
+        if constexpr (TILES >= TILES_NARROW) {
             if (tile == FFT_TILE_NARROW && TN != TD) return run(std::integral_constant<int, TN>{}, T256{});
+        }
+        if constexpr (TILES == TILES_ALL) {
+            if (tile == FFT_TILE_WIDE && TW != TD) return run(std::integral_constant<int, TW>{}, T256{});
             if (tile == FFT_TILE_NARROW_T512 && TN != TD && NW != kFftThreads)
                 return run(std::integral_constant<int, TN>{}, std::integral_constant<int, NW>{});
         }
