@@ -438,6 +438,7 @@ struct LatArgs {
     int nx, ny, nz, npairs, nr;
     int p0;                       // first pair of this chunk
     int width;                    // threads, and pairs, of a group
+    int cols, skip;               // cells of blockIdx.x: rows of cols, those with i, j < skip left out
     int folded;                   // G holds blocks [Nx+1][Ny+1], else [2Nx][2Ny]
     double dx, dy;
     const double2 *segA, *segB;   // [seg][comp][pair]
@@ -571,14 +572,15 @@ __device__ __forceinline__ double2 wab(const double (&w)[WN], int c, double2 q, 
 // 128 x 128 x 32, 256 pairs a group: 0.73 ms for both sets; 3.6 ms with every thread working out the edges'
 // geometry for its own pair, 1.16 ms with the geometry shared but one pass over the segments per edge.
 // 32 x 32 x 8 (64 and 36 pairs), 4 groups of 64: 38 us a set instead of 101 with one.
-constexpr int kCellSegs = 32;
+constexpr int kCellSegs = 32, kNearCells = 8;
 
 template <int ASYM, bool GROUPS>
 __global__ __launch_bounds__(256) void lateral_kernel(LatArgs a)
 {
     __shared__ CellWeights<kCellSegs> cw;
     const int64_t cell = blockIdx.x;
-    const int i = (int)(cell / a.ny), j = (int)(cell % a.ny);
+    const int i = (int)(cell / a.cols), j = (int)(cell % a.cols);
+    if (i < a.skip && j < a.skip) return;
     const int grp = GROUPS ? threadIdx.x / a.width : 0, tp = threadIdx.x - grp * a.width;
     const int groups = GROUPS ? blockDim.x / a.width : 1;
     const int p = blockIdx.y * a.width + tp, np = a.npairs;
@@ -975,10 +977,28 @@ void build_green_atoa(const GreenInput &in, GreenScratch &work, double2 *G, bool
                 while (la.width > 16 && (la.width / 2 >= np || cells * ceil_div(np, la.width) < 4 * device_cus())) la.width /= 2;
                 wgs = (int)ceil_div(np, la.width);
             }
-            const dim3 grid((unsigned)cells, wgs), nt((unsigned)threads);
-            auto run = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, nt, 0, s, la); };
-            if (threads > la.width) asym ? run(lateral_kernel<1, true>) : run(lateral_kernel<0, true>);
-            else asym ? run(lateral_kernel<1, false>) : run(lateral_kernel<0, false>);
+            auto run = [&](int64_t n, int y, int nt) {
+                const dim3 grid((unsigned)n, (unsigned)y), block((unsigned)nt);
+                auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, block, 0, s, la); };
+                if (nt > la.width) asym ? go(lateral_kernel<1, true>) : go(lateral_kernel<0, true>);
+                else asym ? go(lateral_kernel<1, false>) : go(lateral_kernel<0, false>);
+            };
+            la.cols = g.ny;
+            la.skip = 0;
+            // The cells next to the source, with up to 200 segments, by groups in a launch of their own, unless the
+            // others take longer than their chain (140 us) anyway (16384 workgroups, about 0.1 ms) or all go by
+            // groups. 48 x 48 x 32: 39 + 58 and 58 + 73 us a set where one launch took 165 and 190, the whole call
+            // 1157 -> 1117 us; 96 x 48 x 17 605 -> 577 us.
+            if (threads == la.width && cells * wgs < 64 * device_cus()) {
+                const int wide = la.width;
+                la.width = 64;
+                la.cols = std::min(kNearCells, g.ny);
+                run((int64_t)std::min(kNearCells, g.nx) * la.cols, (int)ceil_div(np, 64), 256);
+                la.width = wide;
+                la.cols = g.ny;
+                la.skip = kNearCells;
+            }
+            run(cells, wgs, threads);
             XTR_LAUNCH_CHECK("lateral_kernel");
         }
     }

@@ -44,3 +44,14 @@ def test_level_tensor_near_and_far(oracle, torch_cuda, shape, shift, electric):
     op.calculate_green_atoo(0.0, electric, x_shift=sx, y_shift=sy)
     _close(op.green_atoo(electric), oracle.green_atoo_level(m, w, 0.0, electric, x_shift=sx, y_shift=sy),
            f"{shape} {shift} {'E' if electric else 'H'}")
+
+
+@pytest.mark.parametrize("shape", [(32, 32, 12), (4, 256, 12), (64, 20, 17)])
+def test_cells_near_the_source_apart_from_the_others(oracle, torch_cuda, shape):
+    """Enough cells and pairs that the cells within 8 of the source take a launch of their own."""
+    m = cm.small_model(*shape, seed=sum(shape))
+    w = cm.omega_of(m.frequencies[0])
+    op = X.ConvolutionOperator(m, w)
+    op.calculate_green_tensor()
+    ref = oracle.green_atoa(m, w)
+    _close(op.green_tensor(), ref, f"{shape}")
