@@ -14,7 +14,7 @@
  *
  * Thread model: one host thread drives one handle at a time; host-pointer calls return after
  * the handle's stream has finished the work. xtr_fgmres_solve_batch runs several right-hand
- * sides on their own host threads and streams internally.
+ * sides in lockstep on the calling thread, each on a stack of its own.
  */
 #ifndef XTREME_HIP_H
 #define XTREME_HIP_H
