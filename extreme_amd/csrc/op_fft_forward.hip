@@ -58,6 +58,18 @@ struct IoFwdY {
 
 // Last inverse pass along y, fused with ExtractData and PerformLastStep
 // even lengths 2^a m, m in {1, 3, 5, 15, 25, 75}, up to 512 (Nx, Ny <= 256)
+int fft_tile_row_bytes(int p, int precision, int tile)
+{
+    const int e = precision ? 8 : 16, d = p * 16 * e <= 32768 ? 16 : 8;
+    int cols = d;
+    if (p >= 64) {
+        if (tile == FFT_TILE_WIDE) cols = 2 * d;
+        if (tile == FFT_TILE_NARROW || tile == FFT_TILE_NARROW_T512) cols = d / 2;
+        if (tile == FFT_TILE_REG_ALT) cols = p * 2 * d * e <= 65536 ? 2 * d : d / 2;
+    }
+    return cols * e;
+}
+
 int fft_tile_options(int p, int precision, int *tiles)
 {
     int n = 0;

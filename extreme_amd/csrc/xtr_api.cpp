@@ -274,6 +274,14 @@ struct xtr_op {
                         XTR_CHECK(hipEventElapsedTime(&ms, e0, e1));
                         if (r > 0) total += ms;
                     }
+                    // Rows shorter than a cache line of 128 bytes cost more on a first pass over large spectra, which
+                    // are not in the Infinity Cache then as they are here: at 128 x 128 x 32 (201 MB) the 4-column
+                    // tile of the forward x pass takes 50 us repeated and 80 on new buffers, the 16-column one 52
+                    // both times. There they have to gain a tenth; at 64 x 64 x 32 in complex64 (25 MB) an apply takes
+                    // 95 us with them and 98 without, and a first pass 175 us either way.
+                    if (xtr::fft_tile_row_bytes(P[k], a.precision, t) < 128 &&
+                        (size_t)a.nrhs * g.M() * (a.precision ? 8 : 16) > ((size_t)64 << 20))
+                        total *= 1.1f;
                     if (o == 0 || total < best_ms) {
                         best_ms = total;
                         best[k] = t;

@@ -119,6 +119,8 @@ enum {
 };
 // the column tiles a pencil length offers in this precision (FFT_TILE_*), into tiles[8]; returns how many
 int fft_tile_options(int p, int precision, int *tiles);
+// bytes of a tile's rows, its contiguous runs in memory
+int fft_tile_row_bytes(int p, int precision, int tile);
 
 // Stage launchers (used separately for per-stage timing).
 void launch_fwd_y(const ApplyArgs &a, hipStream_t s);
