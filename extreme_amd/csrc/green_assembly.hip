@@ -435,7 +435,7 @@ __device__ inline Factors factors(double s, double u, double rs, double ru, doub
 }
 
 struct LatArgs {
-    int nx, ny, nz, npairs, nr;
+    int nx, ny, nz, npairs;
     int p0;                       // first pair of this chunk
     int width;                    // threads, and pairs, of a group
     int cols, skip;               // cells of blockIdx.x: rows of cols, those with i, j < skip left out
@@ -443,6 +443,7 @@ struct LatArgs {
     double dx, dy;
     const double2 *segA, *segB;   // [seg][comp][pair]
     const double *radii;
+    const Knot *knots;            // of cell i ny + j
     double2 *G;
     int64_t gblk;
     int64_t off[4];               // component offsets in the per-wavenumber block, q-order
@@ -488,6 +489,22 @@ __device__ inline bool stretch_ends(int e, double x1, double x2, double y1, doub
     return true;
 }
 
+// The two ends of a cell's eight stretches among the radii: thread (cell, stretch, side), cells (i, j), i from i0,
+// j from j0, ncy a row. A binary search is a chain of a dozen loads, which every workgroup of a cell went through
+// before it could start: at 128 x 128 x 32 9 us here, lateral_kernel 0.73 -> 0.60 ms and atoo_lateral_kernel 60
+// and 50 -> 44 and 36 us.
+__global__ __launch_bounds__(256) void knots_kernel(const double *radii, int nr, double dx, double dy, double xs, double ys,
+                                                    int i0, int j0, int ncy, int cells, Knot *knots)
+{
+    const int t = blockIdx.x * blockDim.x + threadIdx.x, cell = t >> 4, e = (t >> 1) & 7;
+    if (cell >= cells) return;
+    const int i = i0 + cell / ncy, j = j0 + cell % ncy;
+    StretchEnds st;
+    stretch_ends(e, dx * (i - 0.5) - xs, dx * (i + 0.5) - xs, dy * (j - 0.5) - ys, dy * (j + 0.5) - ys, st);
+    const double c = t & 1 ? st.r : st.l;
+    knots[t] = e < 4 ? make_knot(radii, nr, c, st.v) : make_knot(radii, nr, st.v, c);
+}
+
 // The four edge integrals of one cell (x1, x2) x (y1, y2) as weights on the segments I_c(rho) = A_c rho + B_c they
 // cross. A component's value is sum over segments of w . (A, B); w holds, for the edges along x and along y, the
 // signed factors d1, d2, d3 (each for A and B) summed over the edge pair: sign -1 for the nearer edge, +1 for the
@@ -504,15 +521,15 @@ struct CellWeights {
     int is[8];
     double f[SEGS][8][WN];
     double w[SEGS][2][WN];        // [edges along x, along y]
-    // the cell's stretches; returns through lo, hi the segments they cross (after the team's next sync)
-    __device__ void ends(int tid, const double *radii, int nr, double x1, double x2, double y1, double y2)
+    // the cell's stretches, their ends from knots_kernel; range returns the segments they cross (after the team's
+    // next sync)
+    __device__ void ends(int tid, const Knot *knots, double x1, double x2, double y1, double y2)
     {
         if (tid >= 16) return;
         const int e = tid >> 1, side = tid & 1;
+        const Knot k = knots[tid];
         StretchEnds t;
         const bool there = stretch_ends(e, x1, x2, y1, y2, t);
-        const double c = side ? t.r : t.l;
-        const Knot k = e < 4 ? make_knot(radii, nr, c, t.v) : make_knot(radii, nr, t.v, c);
         if (side) {
             st[e].right = k;
         } else {
@@ -569,9 +586,9 @@ __device__ __forceinline__ double2 wab(const double (&w)[WN], int c, double2 q, 
 // One workgroup per cell and a share of the pairs; groups of `width` threads share the segments between them, and
 // their sums meet in LDS. Bound by the L2 reads of the segments' coefficients (96 bytes a pair and segment) on a
 // large grid, and on a small one by the chain of the cells next to the source, which cross up to 200 segments. At
-// 128 x 128 x 32, 256 pairs a group: 0.73 ms for both sets; 3.6 ms with every thread working out the edges'
+// 128 x 128 x 32, 256 pairs a group: 0.60 ms for both sets; 3.6 ms with every thread working out the edges'
 // geometry for its own pair, 1.16 ms with the geometry shared but one pass over the segments per edge.
-// 32 x 32 x 8 (64 and 36 pairs), 4 groups of 64: 38 us a set instead of 101 with one.
+// 32 x 32 x 8 (64 and 36 pairs), 4 groups of 64 against one: 38 and 101 us a set, each with its searches.
 constexpr int kCellSegs = 32, kNearCells = 8;
 
 template <int ASYM, bool GROUPS>
@@ -584,7 +601,8 @@ __global__ __launch_bounds__(256) void lateral_kernel(LatArgs a)
     const int grp = GROUPS ? threadIdx.x / a.width : 0, tp = threadIdx.x - grp * a.width;
     const int groups = GROUPS ? blockDim.x / a.width : 1;
     const int p = blockIdx.y * a.width + tp, np = a.npairs;
-    cw.ends(threadIdx.x, a.radii, a.nr, a.dx * (i - 0.5), a.dx * (i + 0.5), a.dy * (j - 0.5), a.dy * (j + 0.5));
+    cw.ends(threadIdx.x, a.knots + (i * a.ny + j) * 16, a.dx * (i - 0.5), a.dx * (i + 0.5), a.dy * (j - 0.5),
+            a.dy * (j + 0.5));
     __syncthreads();
     int lo, hi;
     cw.range(lo, hi);
@@ -653,6 +671,14 @@ __global__ __launch_bounds__(256) void lateral_kernel(LatArgs a)
         if (j >= 1) a.G[((int64_t)i * ny2 + (ny2 - j)) * a.gblk + o] = (double)a.ys[t] * g;
         if (i >= 1 && j >= 1) a.G[((nx2 - i) * ny2 + (ny2 - j)) * a.gblk + o] = (double)(a.xs[t] * a.ys[t]) * g;
     }
+}
+
+void launch_knots(const double *radii, int nr, double dx, double dy, double xs, double ys, int i0, int j0, int ncy,
+                  int64_t cells, Knot *knots, hipStream_t s)
+{
+    hipLaunchKernelGGL(knots_kernel, dim3((unsigned)ceil_div(16 * cells, 256)), dim3(256), 0, s, radii, nr, dx, dy, xs, ys, i0,
+                       j0, ncy, (int)cells, knots);
+    XTR_LAUNCH_CHECK("knots_kernel");
 }
 
 // ---- host: plans ------------------------------------------------------------------------------
@@ -919,13 +945,16 @@ void build_green_atoa(const GreenInput &in, GreenScratch &work, double2 *G, bool
         need[1] = std::max(need[1], (size_t)chunk[asym] * ncomp * ph.nmerged);
         need[2] = need[3] = need[1];
     }
-    size_t bytes = ph.device_bytes();
+    const int64_t cells = (int64_t)g.nx * g.ny;
+    size_t bytes = ph.device_bytes() + GreenScratch::padded(16 * cells * sizeof(Knot));
     for (size_t n : need) bytes += GreenScratch::padded(n * sizeof(double2));
     work.reserve(bytes);
     unsigned char *base;
     const PlanDev d = ph.upload(work, base, s);
     double2 *U = work.take<double2>(need[0]), *I = work.take<double2>(need[1]), *segA = work.take<double2>(need[2]),
             *segB = work.take<double2>(need[3]);
+    Knot *knots = work.take<Knot>(16 * cells);
+    launch_knots(d.radii, ph.nmerged, in.dx, in.dy, 0.0, 0.0, 0, 0, g.ny, cells, knots, s);
     if (!folded) XTR_CHECK(hipMemsetAsync(G, 0, (size_t)g.L() * g.gblk() * sizeof(double2), s));
 
     const int nitems = ph.nitems, nlam_max = ph.nlam_max, nmerged = ph.nmerged;
@@ -948,12 +977,12 @@ void build_green_atoa(const GreenInput &in, GreenScratch &work, double2 *G, bool
             la.npairs = np;
             la.p0 = p0;
             la.folded = folded ? 1 : 0;
-            la.nr = nmerged;
             la.dx = in.dx;
             la.dy = in.dy;
             la.segA = segA;
             la.segB = segB;
             la.radii = d.radii;
+            la.knots = knots;
             la.G = G;
             la.gblk = g.gblk();
             const int64_t S = g.S(), A = (int64_t)nz * nz;
@@ -966,7 +995,6 @@ void build_green_atoa(const GreenInput &in, GreenScratch &work, double2 *G, bool
                 for (int t = 0; t < 3; ++t) { la.xs[t] = 1; la.ys[t] = 1; }
                 la.xs[3] = -1; la.ys[3] = -1;
             }
-            const int64_t cells = (int64_t)g.nx * g.ny;
             int wgs = (int)ceil_div(np, 256);                        // of a cell, with equal shares of the pairs
             la.width = (int)(ceil_div(ceil_div(np, wgs), 64) * 64);
             int threads = la.width;
@@ -987,8 +1015,8 @@ void build_green_atoa(const GreenInput &in, GreenScratch &work, double2 *G, bool
             la.skip = 0;
             // The cells next to the source, with up to 200 segments, by groups in a launch of their own, unless the
             // others take longer than their chain (140 us) anyway (16384 workgroups, about 0.1 ms) or all go by
-            // groups. 48 x 48 x 32: 39 + 58 and 58 + 73 us a set where one launch took 165 and 190, the whole call
-            // 1157 -> 1117 us; 96 x 48 x 17 605 -> 577 us.
+            // groups. 48 x 48 x 32: 39 + 58 and 58 + 73 us a set where one launch took 165 and 190 (all with their
+            // searches), the whole call 1157 -> 1117 us; 96 x 48 x 17 605 -> 577 us.
             if (threads == la.width && cells * wgs < 64 * device_cus()) {
                 const int wide = la.width;
                 la.width = 64;
@@ -1146,11 +1174,12 @@ __global__ void zero_rho_kernel(int nz, int ncomp, int k1, int k2, double alpha2
 }
 
 struct AoArgs {
-    int nx, ny, nz, nr;
+    int nx, ny, nz;
     double dx, dy;
     double xs, ys;                // minus the level's shift (AtoOLevelGreenTensorCalculator.cs:119-125)
     const double2 *segA, *segB;   // [seg][comp][tr]
     const double *radii;
+    const Knot *knots;            // of the offsets in order
     double2 *G;                   // [2Nx][2Ny][components][nz], components as in atoo_components
     int folded;                   // [Nx+1][Ny+1][components][nz], offsets i, j >= 0 only
     int width;                    // lanes of a group: a power of 2, the layers or 64
@@ -1164,8 +1193,9 @@ struct AoArgs {
 // segments in groups of `width` lanes, lane = transmitter layer, each group its own segments.
 // Bound by the chain over the segments of the offsets next to the receiver, up to 200 of some 1500 where one 8 cells
 // away crosses 22: those within kAoNear cells are shared by the 4 waves of a workgroup, which come first; the others
-// take a wave each. 128 x 128 x 32, folded: 60 (electric) and 50 us; 120 and 114 with a wave for every offset, and
-// there 0.64 ms each over all offsets with every thread working out the geometry, 0.26 and 0.22 with weights.
+// take a wave each. 128 x 128 x 32, folded: 44 (electric) and 36 us; 60 and 50 with the searches for the knots in it,
+// 120 and 114 with a wave for every offset as well; over all offsets 0.26 and 0.22 ms then, and 0.64 ms each with
+// every thread working out the geometry.
 constexpr int kAoWaves = 4, kAoSegs = 8, kAoNear = 8;
 
 // Sums of one offset for the layers tr0 .. tr0 + width - 1, complete in the first `width` lanes of the team's first wave
@@ -1249,8 +1279,9 @@ __device__ __forceinline__ void ao_offset(const AoArgs &a, CellWeights<kAoSegs *
                                           const Sync &sync)
 {
     constexpr int no = ELECTRIC ? 8 : 7;
-    cw.ends(tid, a.radii, a.nr, a.dx * (i - 0.5) - a.xs, a.dx * (i + 0.5) - a.xs, a.dy * (j - 0.5) - a.ys,
-            a.dy * (j + 0.5) - a.ys);
+    const int first_i = a.folded ? 0 : 1 - a.nx, first_j = a.folded ? 0 : 1 - a.ny, ncy = a.folded ? a.ny : 2 * a.ny - 1;
+    cw.ends(tid, a.knots + ((i - first_i) * ncy + j - first_j) * 16, a.dx * (i - 0.5) - a.xs, a.dx * (i + 0.5) - a.xs,
+            a.dy * (j - 0.5) - a.ys, a.dy * (j + 0.5) - a.ys);
     sync();
     int lo, hi;
     cw.range(lo, hi);
@@ -1336,13 +1367,17 @@ void build_green_atoo_level(const GreenInput &in, GreenScratch &work, double lev
     const size_t pts_at = ph.pack.add(pts);
     const size_t need[4] = {(size_t)nz * nitems * ncomp * nlam_max, (size_t)ncomp * nz * nmerged,
                             (size_t)nseg * ncomp * nz, (size_t)nseg * ncomp * nz};
-    size_t bytes = ph.device_bytes();
+    const int ncx = folded ? g.nx : 2 * g.nx - 1, ncy = folded ? g.ny : 2 * g.ny - 1, cells = ncx * ncy;
+    size_t bytes = ph.device_bytes() + GreenScratch::padded(16 * cells * sizeof(Knot));
     for (size_t n : need) bytes += GreenScratch::padded(n * sizeof(double2));
     work.reserve(bytes);
     unsigned char *base;
     const PlanDev d = ph.upload(work, base, s);
     double2 *U = work.take<double2>(need[0]), *I = work.take<double2>(need[1]), *segA = work.take<double2>(need[2]),
             *segB = work.take<double2>(need[3]);
+    Knot *knots = work.take<Knot>((size_t)16 * cells);
+    launch_knots(d.radii, nmerged, in.dx, in.dy, -shift_x, -shift_y, folded ? 0 : 1 - g.nx, folded ? 0 : 1 - g.ny, ncy, cells,
+                 knots, s);
     hipLaunchKernelGGL(point_u_kernel, dim3((unsigned)ceil_div(nlam_max, 64), nitems, nz), dim3(64), 0, s, d.lm, nz,
                        (const PointInfo *)(base + pts_at), electric, nitems, nlam_max, d.nlam, d.lam, d.eta, d.ex, d.p1,
                        d.q1, d.ps, d.qs, U);
@@ -1373,7 +1408,6 @@ void build_green_atoo_level(const GreenInput &in, GreenScratch &work, double lev
     a.nx = g.nx;
     a.ny = g.ny;
     a.nz = nz;
-    a.nr = nmerged;
     a.dx = in.dx;
     a.dy = in.dy;
     a.xs = -shift_x;
@@ -1381,10 +1415,10 @@ void build_green_atoo_level(const GreenInput &in, GreenScratch &work, double lev
     a.segA = segA;
     a.segB = segB;
     a.radii = d.radii;
+    a.knots = knots;
     a.G = G;
     a.folded = folded ? 1 : 0;
     if (!folded) XTR_CHECK(hipMemsetAsync(G, 0, (size_t)g.L() * ntc * nz * sizeof(double2), s));
-    const int cells = folded ? g.nx * g.ny : (2 * g.nx - 1) * (2 * g.ny - 1);
     for (a.width = 8; a.width < nz && a.width < 64;) a.width *= 2;
     // within kAoNear cells of the receiver, as far as the offsets go (i1 = i0 where none is)
     auto window = [&](double shift, double d, int n, int &from, int &to) {
