@@ -27,6 +27,7 @@
 #include "xtr_mfma.h"
 
 #include <algorithm>
+#include <complex>
 #include <cmath>
 #include <cstdio>
 #include <cstring>
@@ -160,20 +161,27 @@ __global__ __launch_bounds__(64) void layer_aux_kernel(const LayerModel *lmp, in
 struct PairInfo {
     int r, s, t, b, kase;     // background layers of rc/tr, min/max; 0 match, 1 rc below, 2 rc above
     double r1, r2, s1, s2, dt, db1;
+    double2 iz;               // 1 / (2 zeta_rc), times zeta_rc / zeta_tr where rc is the lower layer
 };
 
-// A[rc][tr] (CalculateA :160-200; CalculateASigma :138-158 for sigma = 1)
-__device__ inline double2 ann_at(const LayerModel &lm, const double2 *E, const double2 *X, const double2 *P,
-                                 const double2 *Q, int rc, int tr, int sigma)
+// A[rc][tr] (CalculateA :160-200; CalculateASigma :138-158 for sigma = 1), A of the lower triangle with the ratio
+// zeta_rc / zeta_tr for sigma = 1; ann_over: without that ratio and over den
+__device__ inline double2 ann_over(const LayerModel &lm, const double2 *E, const double2 *X, const double2 *P,
+                                   const double2 *Q, int rc, int tr, double2 den)
 {
     const int smax = rc > tr ? rc : tr, rmin = rc < tr ? rc : tr;
-    double2 prev = c_(1) / (E[smax] * (c_(1) - P[smax] * Q[smax] * X[smax]));
+    double2 prev = c_(1) / (E[smax] * (c_(1) - P[smax] * Q[smax] * X[smax]) * den);
     for (int k = smax - 1; k >= rmin; --k) {
         const double2 q = ((c_(1) + P[k + 1]) / (c_(1) + P[k] * X[k])) * cexp_d(lm.depth[k + 1] * (E[k + 1] - E[k]));
         prev = q * prev;
     }
-    if (sigma && rc > tr) return (lm.zeta[rc] / lm.zeta[tr]) * prev;
     return prev;
+}
+__device__ inline double2 ann_at(const LayerModel &lm, const double2 *E, const double2 *X, const double2 *P,
+                                 const double2 *Q, int rc, int tr, int sigma)
+{
+    const double2 a = ann_over(lm, E, X, P, Q, rc, tr, c_(1));
+    return sigma && rc > tr ? (lm.zeta[rc] / lm.zeta[tr]) * a : a;
 }
 
 // The layer model lies in memory: indexed by a pair's layer, an argument would go through scratch.
@@ -214,15 +222,16 @@ __global__ __launch_bounds__(64) void pair_u_kernel(const LayerModel *lmp, int n
         C = cexp_d(-pi.r1 * er + pi.s2 * es) * faces;
         D = cexp_d(F - pi.s1 * es + pi.r2 * er) * faces;
     }
-    const double2 zrc2 = 2.0 * lm.zeta[pi.r];
     const int ncomp = asym ? 1 : 3;
     double2 *out = U + (((int64_t)p * nitems + it) * ncomp) * nlam_max + m;
-    const double2 fac = c_(1) / (er * es);
+    // A complex division is some 60 instructions, and there were five or six a thread: the ones by zeta are per pair
+    // (iz, with ann's ratio of zetas), those by eta go into ann's: 0.42 -> 0.35 ms.
+    const double2 ee = asym ? es : er * es;
     for (int set = asym ? 1 : 0; set < 2; ++set) {
         const double2 *P = (set ? ps : p1) + base;
         const double2 *Q = (set ? qs : q1) + base;
         const double2 Pt = P[pi.t], Qb = Q[pi.b];
-        const double2 ann = ann_at(lm, E, X, P, Q, pi.r, pi.s, set);
+        const double2 annfac = ann_over(lm, E, X, P, Q, pi.r, pi.s, ee);
         double2 psi1, psi3;
         if (pi.kase == 0) {
             const int n = pi.r;
@@ -244,19 +253,19 @@ __global__ __launch_bounds__(64) void pair_u_kernel(const LayerModel *lmp, int n
         }
         if (set == 0) {
             // U1 (:144-159), normalised by i omega Mu0 / 2
-            const double2 u1 = ann * fac * (Pt * T + Qb * Rv + psi1);
+            const double2 u1 = annfac * (Pt * T + Qb * Rv + psi1);
             out[0] = u1 * (c_(0, lm.omega * kMu0) * c_(0.5));
             continue;
         }
         if (asym) {
             // U3 (:195-210), normalised by lambda / (2 zeta_rc)
-            const double2 u3 = ann * (c_(1) / es) * (-1.0 * (Pt * T) + Qb * Rv + psi3);
-            out[0] = u3 * (c_(l) / zrc2);
+            const double2 u3 = annfac * (-1.0 * (Pt * T) + Qb * Rv + psi3);
+            out[0] = u3 * (l * pi.iz);
             return;
         }
         // U2 (:183-193), normalised by 1 / (2 zeta_rc)
-        const double2 u2 = ann * (Pt * T + Qb * Rv - psi1);
-        out[(int64_t)1 * nlam_max] = u2 / zrc2;
+        const double2 u2 = annfac * ee * (Pt * T + Qb * Rv - psi1);
+        out[(int64_t)1 * nlam_max] = u2 * pi.iz;
         // U5 (:161-181, 290-311), normalised by lambda^2 / (2 zeta_rc)
         double2 u5;
         if (pi.kase == 0) {
@@ -268,13 +277,13 @@ __global__ __launch_bounds__(64) void pair_u_kernel(const LayerModel *lmp, int n
             const double2 PQ = P[n] * Q[n];
             const double2 part1 = -(c_(1) - xr);
             const double2 part2 = PQ * (cexp_d(-(2 * ln - tau) * en) - cexp_d(-2 * ln * en));
-            const double2 part3 = (kk / c_(l * l)) * (c_(1) - PQ * cexp_d(-2 * ln * en)) * (tau * en);
+            const double2 part3 = ((1 / (l * l)) * kk) * (c_(1) - PQ * cexp_d(-2 * ln * en)) * (tau * en);
             const double2 psi5 = 2.0 * (part1 + part2 + part3);
-            u5 = (ann * fac) * (Pt * T + Qb * Rv + psi5);
+            u5 = annfac * (Pt * T + Qb * Rv + psi5);
         } else {
-            u5 = ann * fac * (Pt * T + Qb * Rv + psi1);
+            u5 = annfac * (Pt * T + Qb * Rv + psi1);
         }
-        out[(int64_t)2 * nlam_max] = u5 * (c_(l * l) / zrc2);
+        out[(int64_t)2 * nlam_max] = u5 * (l * l * pi.iz);
     }
 }
 
@@ -924,6 +933,9 @@ void build_green_atoa(const GreenInput &in, GreenScratch &work, double2 *G, bool
         pi.b = std::max(pi.r, pi.s);
         pi.dt = lm.depth[pi.t];
         pi.db1 = lm.depth[pi.b + 1];
+        const std::complex<double> zr(lm.zeta[pi.r].x, lm.zeta[pi.r].y), zs(lm.zeta[pi.s].x, lm.zeta[pi.s].y);
+        const std::complex<double> iz = 0.5 / (pi.r > pi.s ? zs : zr);
+        pi.iz = make_double2(iz.real(), iz.imag());
         const double zw = pi.r1 + (pi.r2 - pi.r1) / 2;
         pi.kase = (zw > pi.s1 && zw < pi.s2) ? 0 : (zw >= pi.s2 ? 1 : 2);
         pairs[asym].push_back(pi);
