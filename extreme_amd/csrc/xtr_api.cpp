@@ -401,9 +401,9 @@ struct StepReq {
     const void *V = nullptr, *u = nullptr;   // apply: V = x; as in xtr::StepRhs otherwise
     void *w = nullptr, *next = nullptr;      // apply: w = y
     int cnt = 0, mul = 0;
+    bool now = false;                        // norm: its result is needed before the next request
     const std::function<void()> *call = nullptr;
-    // norm's result is only needed after the next request that waits
-    bool has_result() const { return op == StepOp::cgs || op == StepOp::residual; }
+    bool has_result() const { return op == StepOp::cgs || op == StepOp::residual || now; }
 };
 
 // Small results of kernels in host memory that the host polls: begin(n) marks n values as missing, and a value
@@ -711,12 +711,13 @@ struct Gmres {
         ctx->matvecs++;
     }
 
-    // asks for |v|; its value is there after the next residual
-    void norm(const VT *v)
+    // asks for |v|; its value is there at once (now) or after the next residual
+    void norm(const VT *v, bool now)
     {
         StepReq r;
         r.op = StepOp::norm;
         r.w = (void *)v;
+        r.now = now;
         ctx->run(r);
         ctx->dots++;
     }
@@ -888,15 +889,23 @@ struct Gmres {
     void solve(const VT *rhs, const VT *x0, VT *result, double &bea_out, double &be_out, int &conv)
     {
         iter_counter = 0;
-        norm(rhs);                                      // read together with the residual's
-        matvec(x0, r0);
-        double beta = residual(rhs, r0, col(V, 0));
-        const double bn = ctx->norm(ctx->b_host, n);
-        // NaN or Inf would end the iteration as if converged (bea > tol is false): refuse instead
-        if (!std::isfinite(bn)) throw std::runtime_error("the right-hand side holds NaN or Inf");
+        // The caller's right-hand side may be zero or not finite, which ends the solve without an apply: its norm is
+        // waited for, once a solve. The inner solver's is a basis vector of norm 1: that norm is read together with
+        // the residual's.
+        norm(rhs, flexible);
+        auto rhs_norm = [&] {
+            const double v = ctx->norm(ctx->b_host, n);
+            // NaN or Inf would end the iteration as if converged (bea > tol is false): refuse instead
+            if (!std::isfinite(v)) throw std::runtime_error("the right-hand side holds NaN or Inf");
+            return v;
+        };
+        double bn = flexible ? rhs_norm() : -1, beta = -1;
+        if (bn != 0) {
+            matvec(x0, r0);
+            beta = residual(rhs, r0, col(V, 0));
+            if (!flexible) bn = rhs_norm();
+        }
         if (bn == 0) {
-            ctx->matvecs--;                             // of a residual that is not used
-            ctx->dots--;
             bea_out = 0; be_out = 0; conv = 1;
             return;
         }
@@ -983,10 +992,10 @@ void run_fgmres(xtr_op *op, const xtr_gmres_params &p, Slot &sl, const VT *b, VT
 
 // Solves of several right-hand sides side by side, in step, on one host thread and the operator's stream. Each is a
 // fiber (its own stack, switched by ucontext) that runs until it asks for something of the GPU. When all have, what
-// they ask for is launched together: first whatever has no result to wait for, then the Gram-Schmidt passes and
-// residuals, whose results the host waits for once, and the apply when every solve that is still running asks for it, so that
-// the Green tensor is streamed once for all of them. Each right-hand side follows exactly the iteration of its own
-// solve. Fibers make no HIP call and no callback: those run on the caller's stack (StepOp::call).
+// they ask for is launched together: first calls and norms, then the Gram-Schmidt passes and residuals, whose results
+// the host waits for once, and the apply when every solve that is still running asks for it, so that the Green tensor
+// is streamed once for all of them. Each right-hand side follows exactly the iteration of its own solve. Fibers make no
+// HIP call and no callback: those run on the caller's stack (StepOp::call).
 template <typename VT>
 class Lockstep {
 public:
@@ -1021,6 +1030,8 @@ public:
             if (!calls.empty() || !norms.empty()) {
                 for (int r : calls) attempt({r}, [&] { (*fib_[r].req->call)(); });
                 if (!norms.empty()) attempt(norms, [&] { launch(StepOp::norm, norms, ctx, R); });
+                for (int r : norms)
+                    if (fib_[r].req->now && !fib_[r].fault) attempt({r}, [&] { ctx[r]->wait(); });
                 for (int r : calls) resume(r);
                 for (int r : norms) resume(r);
                 continue;
