@@ -56,29 +56,14 @@ struct IoFwdY {
     }
 };
 
-// Last inverse pass along y, fused with ExtractData and PerformLastStep
-// even lengths 2^a m, m in {1, 3, 5, 15, 25, 75}, up to 512 (Nx, Ny <= 256)
-int fft_tile_row_bytes(int p, int precision, int tile)
-{
-    const int e = precision ? 8 : 16, d = p * 16 * e <= 32768 ? 16 : 8;
-    int cols = d;
-    if (p >= 64) {
-        if (tile == FFT_TILE_WIDE) cols = 2 * d;
-        if (tile == FFT_TILE_NARROW || tile == FFT_TILE_NARROW_T512) cols = d / 2;
-        if (tile == FFT_TILE_REG_ALT) cols = p * 2 * d * e <= 65536 ? 2 * d : d / 2;
-    }
-    return cols * e;
-}
-
 int fft_tile_options(int p, int precision, int *tiles)
 {
     int n = 0;
     tiles[n++] = FFT_TILE_DEFAULT;
     if (p < 64) return n;
     const int e = precision ? 8 : 16;
-    const int d = (p * 16 * e <= 32768) ? 16 : 8;
-    tiles[n++] = FFT_TILE_NARROW;                    // d / 2 >= 4 always
-    if (p * 2 * d * e <= 131072) tiles[n++] = FFT_TILE_WIDE;
+    tiles[n++] = FFT_TILE_NARROW;
+    if (fft_tile_cols(p, e, FFT_TILE_WIDE) > fft_tile_cols(p, e, FFT_TILE_DEFAULT)) tiles[n++] = FFT_TILE_WIDE;
     if (p >= 128) tiles[n++] = FFT_TILE_NARROW_T512;
     if (p == 64 || p == 128 || p == 256 || p == 512) {
         tiles[n++] = FFT_TILE_REG;
@@ -87,6 +72,7 @@ int fft_tile_options(int p, int precision, int *tiles)
     return n;
 }
 
+// even lengths 2^a m, m in {1, 3, 5, 15, 25, 75}, up to 512 (Nx, Ny <= 256)
 bool fft_length_supported(int p)
 {
     switch (p) {

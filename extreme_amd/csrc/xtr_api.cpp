@@ -221,11 +221,11 @@ struct xtr_op {
     // x; x and y never overlap, which apply_raw checks).
     std::array<int, 4> fft_tiles(xtr::ApplyArgs &a, hipStream_t s)
     {
-        const int P[4] = {2 * g.ny, 2 * g.nx, 2 * g.nx, 2 * g.ny};
-        if (const char *e = std::getenv("XTR_FFT_TILES")) {
+        const int P[4] = {2 * g.ny, 2 * g.nx, 2 * g.nx, 2 * g.ny}, e = a.precision ? 8 : 16;
+        if (const char *fixed = std::getenv("XTR_FFT_TILES")) {
             std::array<int, 4> t{};
             for (int k = 0; k < 4; ++k) {
-                const char c = e[0] && std::strlen(e) == 4 ? e[k] : 'd';
+                const char c = std::strlen(fixed) == 4 ? fixed[k] : 'd';
                 t[k] = c == 'w'   ? xtr::FFT_TILE_WIDE
                        : c == 'n' ? xtr::FFT_TILE_NARROW
                        : c == 'm' ? xtr::FFT_TILE_NARROW_T512
@@ -274,14 +274,7 @@ struct xtr_op {
                         XTR_CHECK(hipEventElapsedTime(&ms, e0, e1));
                         if (r > 0) total += ms;
                     }
-                    // Rows shorter than a cache line of 128 bytes cost more on a first pass over large spectra, which
-                    // are not in the Infinity Cache then as they are here: at 128 x 128 x 32 (201 MB) the 4-column
-                    // tile of the forward x pass takes 50 us repeated and 80 on new buffers, the 16-column one 52
-                    // both times. There they have to gain a tenth; at 64 x 64 x 32 in complex64 (25 MB) an apply takes
-                    // 95 us with them and 98 without, and a first pass 175 us either way.
-                    if (xtr::fft_tile_row_bytes(P[k], a.precision, t) < 128 &&
-                        (size_t)a.nrhs * g.M() * (a.precision ? 8 : 16) > ((size_t)64 << 20))
-                        total *= 1.1f;
+                    total *= (float)xtr::fft_tile_weight(g.M() * e, P[k], e, t);
                     if (o == 0 || total < best_ms) {
                         best_ms = total;
                         best[k] = t;

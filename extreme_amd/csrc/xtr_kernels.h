@@ -6,6 +6,8 @@
 
 #include <cstdint>
 
+#include "xtr_tiles.h"
+
 namespace xtr {
 
 constexpr int kMaxRhs = 8;
@@ -109,18 +111,8 @@ struct ApplyArgs {
     RhsPtrs v;
 };
 
-enum {
-    FFT_TILE_DEFAULT = 0,
-    FFT_TILE_NARROW = 1,
-    FFT_TILE_WIDE = 2,
-    FFT_TILE_NARROW_T512 = 3,
-    FFT_TILE_REG = 4,        // register-resident stages (lengths 64..512), the default column count
-    FFT_TILE_REG_ALT = 5,    // the same with twice the columns (half where that exceeds 64 KB of LDS)
-};
 // the column tiles a pencil length offers in this precision (FFT_TILE_*), into tiles[8]; returns how many
 int fft_tile_options(int p, int precision, int *tiles);
-// bytes of a tile's rows, its contiguous runs in memory
-int fft_tile_row_bytes(int p, int precision, int tile);
 
 // Stage launchers (used separately for per-stage timing).
 void launch_fwd_y(const ApplyArgs &a, hipStream_t s);

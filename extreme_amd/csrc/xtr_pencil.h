@@ -329,39 +329,19 @@ __global__ __launch_bounds__(NT) void pencil_fft_reg_kernel(IO io, const cplx<T>
     reg_stage<T, P, TC, DIR, P, 1, NT>(io, rhs, c0, s, tw, tid, a);
 }
 
-// Column tiles per pencil length. The default tile has 16 columns while P x 16 stays within 32 KB,
-// else 8. For lengths from 64 there are two more: the narrow tile (half the columns, more workgroups
-// per CU) and the wide one (twice the columns, longer contiguous runs per row, within 128 KB); from
-// 128, the narrow tile also runs with 512 threads (twice the waves per CU for the same LDS). Which
+// Column tiles per pencil length (fft_tile_cols): the default, for lengths from 64 a narrow and a wide one, and
+// from 128 the narrow tile also with 512 threads (twice the waves per CU for the same LDS). Which
 // one a pass uses is measured on the device (the operator's tile tuning); the choice does not change
 // the arithmetic, only how the columns are grouped and how many threads share a tile.
 template <typename T, int P>
-constexpr int tile_cols()
-{
-    return (P * 16 * (int)sizeof(cplx<T>) <= 32768) ? 16 : 8;
-}
-template <typename T, int P>
 constexpr int tile_cols_of(int tile)
 {
-    constexpr int d = tile_cols<T, P>();
-    if (P < 64) return d;
-    if (tile == FFT_TILE_WIDE) return P * 2 * d * (int)sizeof(cplx<T>) <= 131072 ? 2 * d : d;
-    if (tile == FFT_TILE_NARROW || tile == FFT_TILE_NARROW_T512) return d / 2 >= 4 ? d / 2 : d;
-    return d;
+    return fft_tile_cols(P, (int)sizeof(cplx<T>), tile);
 }
 template <int P>
 constexpr int tile_threads_of(int tile)
 {
     return tile == FFT_TILE_NARROW_T512 && P >= 128 ? 512 : kFftThreads;
-}
-// register pencils: the default column count, or the alternative (twice that within 64 KB of LDS,
-// else half)
-template <typename T, int P>
-constexpr int reg_cols_of(int tile)
-{
-    constexpr int d = tile_cols<T, P>();
-    if (tile != FFT_TILE_REG_ALT) return d;
-    return P * 2 * d * (int)sizeof(cplx<T>) <= 65536 ? 2 * d : d / 2;
 }
 
 // TILES_ALL: every tile (the apply's passes, which measure them); otherwise the default, the register pencil of the
@@ -392,11 +372,11 @@ void launch_pencil(int P, const IO &io, int64_t ncols, int nrhs, const void *tw,
                 };
                 if constexpr (TILES == TILES_ALL) {
                     if (tile == FFT_TILE_REG_ALT) {
-                        reg(std::integral_constant<int, reg_cols_of<T, PP>(FFT_TILE_REG_ALT)>{});
+                        reg(std::integral_constant<int, tile_cols_of<T, PP>(FFT_TILE_REG_ALT)>{});
                         return;
                     }
                 }
-                reg(std::integral_constant<int, reg_cols_of<T, PP>(FFT_TILE_REG)>{});
+                reg(std::integral_constant<int, tile_cols_of<T, PP>(FFT_TILE_REG)>{});
                 return;
             }
         }
