@@ -48,17 +48,8 @@ METRIC = "FGMRES solve time per freq (2 pol) to 1e-8 residual; op-apply HBM GB/s
 # Keyed by (workload, nz, right-hand sides per launch, Green layout); no entry reports null.
 MEASURED_TRAFFIC = {("C2", 32, 2, "folded"): 1.5120e9,   # contract_block_kernel<double, 32, 2>
                     ("C5", 64, 2, "folded"): 2.0671e10,  # contract_fold64_kernel<double>
-                    ("C2", 32, 2, "full"): 4.7647e9,     # contract_stream_kernel<double, 2>
+                    ("C2", 32, 2, "full"): 4.7647e9,     # contract_stream_kernel<double>
                     ("C5", 64, 2, "full"): 7.2476e10}    # contract_stream64_kernel<double, 2>
-
-
-def contract_kernel_name(nz, layout):
-    """The FP64 contraction kernel a two-right-hand-side apply launches at this nz and Green layout."""
-    if layout == "folded":
-        return "contract_fold64_kernel<double>" if nz == 64 else (
-            f"contract_block_kernel<double, {nz}, 2>" if nz <= 47 else "contract_rows_kernel<double, 1>")
-    return {32: "contract_stream_kernel<double, 2>", 64: "contract_stream64_kernel<double, 2>"}.get(
-        nz, "contract_kernel<double>")
 
 
 def log(msg):
@@ -164,7 +155,7 @@ def sweep(model, args):
     rounds = rhs_applies = rounds2 = 0
     contract_bytes = apply_bytes = 0.0
     contract2_ms = 0.0                 # contraction launches with two right-hand sides
-    layout = None
+    layout = kernel2 = None            # kernel2: the contraction kernel of those launches
     cpu = None
     green_s = []
     mixed_rows = {}
@@ -191,6 +182,7 @@ def sweep(model, args):
         st, cnt = p.op.stage_times()
         st2, cnt2 = p.op.stage_times(2)
         p.op.set_profiling(False)
+        kernel2 = p.op.contract_kernel(2)
         contract2_ms += st2["contract"]
         rounds2 += cnt2
         layout, nblk = p.op.green_layout()
@@ -299,7 +291,7 @@ def sweep(model, args):
         "apply_gpu_share_of_solve": apply_ms * 1e-3 / total,
         "stage_ms_per_apply": {k: v / max(rounds, 1) for k, v in stage_ms.items()},
         "green_seconds_per_freq": float(np.mean(green_s)),
-        "roofline": {"kernel": contract_kernel_name(nz, layout), "bound": "hbm", "achieved": achieved,
+        "roofline": {"kernel": kernel2, "bound": "hbm", "achieved": achieved,
                      "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": achieved / HBM_PEAK_GBS,
                      "traffic": MEASURED_TRAFFIC.get((m.name, nz, 2, layout)),
                      "avg_launch_ms": launch2_ms, "launches": rounds2, "green_layout": layout,

@@ -386,6 +386,7 @@ void launch_block(const ApplyArgs &a, hipStream_t s)
     const unsigned grid = (unsigned)std::min<int64_t>(p.Lq, ceil_div((int64_t)resident * device_cus(), groups));
     hipLaunchKernelGGL((contract_block_kernel<T, NZ, NR>), dim3(grid, groups), dim3(64 * K::W), 0, s, p);
     XTR_LAUNCH_CHECK("contract_block_kernel");
+    note_contract(a, "contract_block_kernel", NZ, NR);
 }
 
 // Depths LO..HI; false for another depth or one whose block does not fit. One right-hand side or two by

@@ -125,6 +125,7 @@ void launch_direct(const ApplyArgs &a, hipStream_t s)
     else if (a.nrhs <= 4) hipLaunchKernelGGL((contract_direct_kernel<T, NZ, 2>), grid, nt, 0, s, p);
     else hipLaunchKernelGGL((contract_direct_kernel<T, NZ, 4>), grid, nt, 0, s, p);
     XTR_LAUNCH_CHECK("contract_direct_kernel");
+    note_contract(a, "contract_direct_kernel", NZ, a.nrhs <= 2 ? 1 : a.nrhs <= 4 ? 2 : 4);
 }
 
 template <typename T, int NZ = 1>
@@ -234,6 +235,7 @@ void launch_rows(const ApplyArgs &a, hipStream_t s)
     const size_t lds = (size_t)8 * CT * (4 * steps + 2) * sizeof(cplx<T>);
     hipLaunchKernelGGL((contract_rows_kernel<T, CT>), grid, nt, lds, s, p, a.g.nz, asym_swizzle_mask(a.g.nz));
     XTR_LAUNCH_CHECK("contract_rows_kernel");
+    note_contract(a, "contract_rows_kernel", 0, CT);
 }
 
 }  // namespace

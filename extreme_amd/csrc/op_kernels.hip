@@ -572,6 +572,7 @@ static bool contract_stream64(const ApplyArgs &a, hipStream_t s)
     if (a.precision == 0) launch_stream64<double>(a, grid, s);
     else launch_stream64<float>(a, grid, s);
     XTR_LAUNCH_CHECK("contract_stream64_kernel");
+    note_contract(a, "contract_stream64_kernel", 0, a.nrhs);
     return true;
 }
 
@@ -585,6 +586,7 @@ static bool contract_stream(const ApplyArgs &a, hipStream_t s)
     hipLaunchKernelGGL((contract_stream_kernel<T>), dim3(grid), dim3(256), 0, s, (const cplx<T> *)a.G,
                        (cplx<T> *)a.buf, L, a.g.M(), a.nrhs);
     XTR_LAUNCH_CHECK("contract_stream_kernel");
+    note_contract(a, "contract_stream_kernel");
     return true;
 }
 
@@ -974,6 +976,7 @@ static bool contract_fold64(const ApplyArgs &a, hipStream_t s)
                                (float2 *)a.buf + h0 * a.g.M(), Lq, a.g.M(), nh, a.g.nx, a.g.ny);
         XTR_LAUNCH_CHECK("contract_fold64_kernel");
     }
+    note_contract(a, "contract_fold64_kernel");
     return true;
 }
 
@@ -1017,6 +1020,7 @@ static void contract(const ApplyArgs &a, hipStream_t s)
     hipLaunchKernelGGL(contract_kernel<T>, grid, dim3(threads), lds, s, (const cplx<T> *)a.G, (cplx<T> *)a.buf, L,
                        nz, a.nrhs, W, a.g.M(), a.packed_rc, a.folded ? a.g.nx : 0, a.g.ny);
     XTR_LAUNCH_CHECK("contract_kernel");
+    note_contract(a, "contract_kernel");
 }
 
 void launch_contract(const ApplyArgs &a, hipStream_t s) { a.precision ? contract<float>(a, s) : contract<double>(a, s); }

@@ -184,6 +184,7 @@ struct xtr_op {
     // Per-stage timing: one set of six events per apply while profiling is on, summed on demand.
     bool profiling = false;
     std::array<int, 4> last_tiles{{-1, -1, -1, -1}};   // FFT column tiles of the latest apply
+    std::array<xtr::ContractKernel, xtr::kMaxRhs + 1> ran;   // by right-hand sides, of the latest apply of so many
     std::vector<std::array<hipEvent_t, 6>> ev_sets;
     std::vector<int> ev_nrhs;                        // right-hand sides of the apply each set timed
     size_t ev_used = 0;
@@ -328,6 +329,7 @@ struct xtr_op {
         a.tw_y = p == XTR_FP64 ? (const void *)tw64_y.p : (const void *)tw32_y.p;
         a.vec32 = vec32 ? 1 : 0;
         a.v = v;
+        a.ran = &ran[nrhs];
         last_tiles = fft_tiles(a, s);
         for (int k = 0; k < 4; ++k) a.fft_tile[k] = last_tiles[k];
         hipEvent_t *ev = profiling ? next_events(nrhs) : nullptr;
@@ -1555,6 +1557,25 @@ int xtr_op_fft_tiles(xtr_op *op, int *tiles4)
         require(op && tiles4, "null argument");
         std::lock_guard<std::mutex> lk(op->apply_mu);
         for (int k = 0; k < 4; ++k) tiles4[k] = op->last_tiles[k];
+    });
+}
+
+int xtr_op_contract_kernel(xtr_op *op, int nrhs, char *name, int len)
+{
+    return guarded([&] {
+        require(op && name && len > 0, "null argument");
+        require(nrhs >= 1 && nrhs <= op->max_rhs, "nrhs out of range");
+        std::lock_guard<std::mutex> lk(op->apply_mu);
+        const xtr::ContractKernel &k = op->ran[nrhs];
+        std::string s;
+        if (k.name) {
+            s = std::string(k.name) + (k.precision ? "<float" : "<double");
+            for (int arg : {k.depth, k.group})
+                if (arg) s += ", " + std::to_string(arg);
+            s += ">";
+        }
+        require((int)s.size() < len, "the name does not fit");
+        std::memcpy(name, s.c_str(), s.size() + 1);
     });
 }
 

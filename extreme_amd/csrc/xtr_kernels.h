@@ -89,6 +89,12 @@ struct RhsPtrs {
     const double2 *R[kMaxRhs];
 };
 
+// The kernel that a contraction launched: its name and, after the element type, its template arguments (0: none).
+struct ContractKernel {
+    const char *name = nullptr;
+    int precision = 0, depth = 0, group = 0;
+};
+
 // ---- operator apply (op_kernels.hip) -------------------------------------------------------
 // Twiddle tables exp(-2 pi i k / P), k < P, in the apply precision.
 // precision: 0 = FP64 (double2 buffers / Green), 1 = FP32 (float2).
@@ -109,10 +115,16 @@ struct ApplyArgs {
     int fft_tile[4];          // column tile of fwd_y, fwd_x, inv_x, inv_y (FFT_TILE_*)
     int vec32;                // v.x and v.y point to complex64 vectors (float2; precision FP32 only)
     RhsPtrs v;
+    ContractKernel *ran;      // where launch_contract notes its kernel, or null
 };
 
 // the column tiles a pencil length offers in this precision (FFT_TILE_*), into tiles[8]; returns how many
 int fft_tile_options(int p, int precision, int *tiles);
+
+inline void note_contract(const ApplyArgs &a, const char *name, int depth = 0, int group = 0)
+{
+    if (a.ran) *a.ran = ContractKernel{name, a.precision, depth, group};
+}
 
 // Stage launchers (used separately for per-stage timing).
 void launch_fwd_y(const ApplyArgs &a, hipStream_t s);

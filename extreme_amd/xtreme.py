@@ -112,6 +112,7 @@ def lib():
         L.xtr_op_stage_times.argtypes = [C.c_void_p, C.POINTER(C.c_double), C.POINTER(C.c_int64)]
         L.xtr_op_stage_times_rhs.argtypes = [C.c_void_p, C.c_int, C.POINTER(C.c_double), C.POINTER(C.c_int64)]
         L.xtr_op_fft_tiles.argtypes = [C.c_void_p, C.POINTER(C.c_int)]
+        L.xtr_op_contract_kernel.argtypes = [C.c_void_p, C.c_int, C.c_char_p, C.c_int]
         L.xtr_op_sizes.argtypes = [C.c_void_p, C.POINTER(C.c_int64), C.POINTER(C.c_int64), C.POINTER(C.c_int64)]
         L.xtr_op_green_layout.argtypes = [C.c_void_p, C.POINTER(C.c_int), C.POINTER(C.c_int64)]
         L.xtr_op_green_mirror_check.argtypes = [C.c_void_p, C.POINTER(C.c_double)]
@@ -462,6 +463,12 @@ class ConvolutionOperator:
         _check(lib().xtr_op_fft_tiles(self._h, out))
         return None if out[0] < 0 else dict(zip(("fwd_y", "fwd_x", "inv_x", "inv_y"),
                                                 (self.FFT_TILES[t] for t in out)))
+
+    def contract_kernel(self, nrhs: int):
+        """Name of the contraction kernel that the latest apply of nrhs right-hand sides launched; None before one."""
+        name = C.create_string_buffer(96)
+        _check(lib().xtr_op_contract_kernel(self._h, int(nrhs), name, len(name)))
+        return name.value.decode() or None
 
     def sizes(self):
         n, gb, bb = C.c_int64(), C.c_int64(), C.c_int64()

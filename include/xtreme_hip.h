@@ -235,6 +235,12 @@ int xtr_op_stage_times_rhs(xtr_op *op, int nrhs, double *out5, int64_t *applies)
  * change the radix plan, so results move by rounding only. */
 int xtr_op_fft_tiles(xtr_op *op, int *tiles4);
 
+/* No counterpart in the reference: the contraction kernel that the latest apply of nrhs right-hand
+ * sides launched, as in a kernel trace without its namespace ("contract_block_kernel<double, 32, 2>"),
+ * zero-terminated into name[len]; empty before the first such apply. Which kernel runs depends on the
+ * grid, the layers, the precision, the right-hand sides and how the Green tensor is kept. */
+int xtr_op_contract_kernel(xtr_op *op, int nrhs, char *name, int len);
+
 /* ---- observation level (AtoO) ----------------------------------------------------------------- */
 
 /* Replaces: AtoOCalculator.CalculateGreenTensorAtoOLevelElectric / ...Magnetic
