@@ -64,6 +64,11 @@ struct BlockCfg {
     static constexpr int STORES = 4 * CT;
     // B fragments and accumulators have to leave the waves of a workgroup in the register file
     static constexpr bool ok = LDS <= 160 * 1024 && 3 * KC * CT * (int)sizeof(T) / 4 <= 100 && C >= NR;
+    // B fragments, accumulators, LDS offsets and copy sources, in registers; what the waves of a workgroup leave of
+    // the register file holds 16 more at the most without spills (complex64 in groups of 4: 152 at 47 layers fit in
+    // 168, 154 at 58 and 60 spill 2 and 3 values, 188 at 63 spill 37).
+    static constexpr int REGS = (3 * KC + 8) * CT * (int)sizeof(T) / 4 + 2 * KC + most(N1) + most(N2) + 4 * most(NU);
+    static constexpr bool spills = REGS + 16 > 512 / ((W + 3) / 4) / 8 * 8;
 };
 
 template <typename T>
@@ -405,8 +410,13 @@ bool contract_block_range(const ApplyArgs &a, hipStream_t s)
             // to 3, by registers and LDS): 8 right-hand sides at 64 x 64, groups of 2 and of 4: nz = 16 77 and
             // 82 us, 20: 130 and 155, 24: 166 and 188; outside these depths 12: 60 and 54, 32: 287 and 266.
             constexpr int most = BlockCfg<T, LO, 4>::ok && (LO < 16 || LO > 25) ? 4 : BlockCfg<T, LO, 2>::ok ? 2 : 1;
+            // Where a group of 4 spills, 3 and 4 go in two groups of 2: complex64, 40 x 40 x 63 114 and 118 us instead
+            // of 139 and 144, x 57 103 and 107 instead of 124 and 129, x 60 108 and 111 instead of 109 and 110; 16 x 20
+            // x 63 32 instead of 43. More than 4 stay in two groups of 4: a third group reads the tensor once more
+            // (5 at 40 x 40 x 63: 263 us, in groups of 2 300).
+            constexpr int two = BlockCfg<T, LO, 2>::ok ? 2 : 1;
             if (a.nrhs == 1) launch_block<T, LO, 1>(a, s);
-            else if (a.nrhs == 2 && BlockCfg<T, LO, 2>::ok) launch_block<T, LO, BlockCfg<T, LO, 2>::ok ? 2 : 1>(a, s);
+            else if (a.nrhs == 2 || (a.nrhs <= 4 && most == 4 && BlockCfg<T, LO, 4>::spills)) launch_block<T, LO, two>(a, s);
             else launch_block<T, LO, most>(a, s);
             return true;
         }

@@ -4,13 +4,33 @@ against the generic per-wavenumber kernel and the oracle on either side of the l
 Tolerances: a result sums 3 nz <= 258 products, so two orders of summation differ by at most about 258 eps of the sum
 of magnitudes, a few times that of the result for random data: 1e-13 (complex128), and 1e-12 against the oracle, whose
 transforms differ too; with the transforms in float32 as well 2e-6 (complex64)."""
+import os
+import re
+import struct
+import subprocess
+
 import numpy as np
 import pytest
 
+from extreme_amd import cartesian_model as cm
+from extreme_amd import xtreme as X
 from tests.conftest import rel
-from tests.test_gpu_block_contraction import _op
+from tests.test_gpu_folded import _mirror_symmetric_green
 
 pytestmark = pytest.mark.gpu
+
+
+def _op(oracle, shape, nrhs, precision, seed):
+    """An operator with a random tensor, scaled (by the resistivity times the layer thickness) so that the convolution
+    is of the size of its input and a wrong block shows as its share of the result."""
+    m = cm.small_model(*shape, seed=seed)
+    w = cm.omega_of(m.frequencies[0])
+    G = {c: g * (1e4 / np.sqrt(3 * m.nz)) for c, g in _mirror_symmetric_green(oracle, m, seed).items()}
+    op = X.ConvolutionOperator(m, w, precision=precision, max_rhs=nrhs)
+    op.set_green_tensor(G)
+    assert op.green_layout()[0] == "folded"
+    op.prepare_operator("A")
+    return m, w, G, op
 
 
 def _x(m, nrhs, seed):
@@ -53,8 +73,6 @@ def test_few_layers_on_either_side(oracle, torch_cuda, monkeypatch, grid, nz, nr
 def test_kernel_by_depth_and_layout(oracle, torch_cuda, monkeypatch, nz, nrhs, precision, layout, kernel):
     if layout:
         monkeypatch.setenv("XTR_GREEN_LAYOUT", layout)
-    from extreme_amd import cartesian_model as cm
-    from extreme_amd import xtreme as X
     m = cm.small_model(4, 5, nz, seed=nz)
     op = X.ConvolutionOperator(m, cm.omega_of(m.frequencies[0]), precision=precision, max_rhs=nrhs)
     op.calculate_green_tensor()
@@ -65,3 +83,45 @@ def test_kernel_by_depth_and_layout(oracle, torch_cuda, monkeypatch, nz, nrhs, p
         assert op.contract_kernel(1) is None
     with pytest.raises(X.XtrError, match="nrhs"):
         op.contract_kernel(nrhs + 1)
+
+
+def _spills(tmp_path):
+    """{mangled kernel name: spilled vector registers} from the metadata of the library's device code."""
+    data, magic, out = open(X.LIB_PATH, "rb").read(), b"__CLANG_OFFLOAD_BUNDLE__", {}
+    for at in (m.start() for m in re.finditer(magic, data)):
+        count, pos = struct.unpack_from("<Q", data, at + len(magic))[0], at + len(magic) + 8
+        for _ in range(count):
+            offset, size, length = struct.unpack_from("<QQQ", data, pos)
+            triple = data[pos + 24:pos + 24 + length]
+            pos += 24 + length
+            if not triple.endswith(b"gfx950"):
+                continue
+            (tmp_path / "code").write_bytes(data[at + offset:at + offset + size])
+            notes = subprocess.run([os.path.join(os.environ.get("ROCM_PATH", "/opt/rocm"), "llvm", "bin", "llvm-readelf"), "--notes",
+                                    str(tmp_path / "code")], check=True, capture_output=True, text=True).stdout
+            for kernel in re.split(r"\n\s*- \.agpr_count", notes)[1:]:
+                name, spilled = re.search(r"\.name:\s*(\S+)", kernel), re.search(r"\.vgpr_spill_count:\s*(\d+)", kernel)
+                out[name.group(1)] = int(spilled.group(1))
+    return out
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+def test_up_to_four_right_hand_sides_do_not_spill(torch_cuda, tmp_path, precision):
+    """A kernel that spills runs its copies in step with its scratch accesses: the dispatch of up to four right-hand
+    sides chooses none. From 26 layers on, where groups of four begin (below them no kernel comes near its registers)."""
+    spills, seen = _spills(tmp_path), set()
+    letter = {"double": "d", "float": "f"}
+    for nz in range(26, 64):
+        m = cm.small_model(4, 5, nz, seed=nz)
+        op = X.ConvolutionOperator(m, cm.omega_of(m.frequencies[0]), precision=precision, max_rhs=4)
+        op.calculate_green_tensor()
+        op.prepare_operator("A")
+        for nrhs in range(1, 5):
+            op.apply(_x(m, nrhs, nz))
+            name = op.contract_kernel(nrhs)
+            t, *args = re.search(r"<(.*)>", name).group(1).split(", ")
+            mangled = name.split("<")[0] + "I" + letter[t] + "".join(f"Li{a}E" for a in args) + "E"
+            found = [v for k, v in spills.items() if mangled in k]
+            assert found and max(found) == 0, (nz, nrhs, name, found)
+            seen.add(name)
+    assert len(seen) > 38
