@@ -125,3 +125,23 @@ def test_up_to_four_right_hand_sides_do_not_spill(torch_cuda, tmp_path, precisio
             assert found and max(found) == 0, (nz, nrhs, name, found)
             seen.add(name)
     assert len(seen) > 38
+
+
+@pytest.mark.parametrize("precision,tol", [("fp64", 1e-13), ("fp32", 2e-6)])
+@pytest.mark.parametrize("nrhs", [1, 2, 3, 4, 8])
+def test_every_depth_where_the_convolution_weighs(oracle, torch_cuda, monkeypatch, nrhs, precision, tol):
+    worst = (0.0, None)
+    for nz in range(1, 86):
+        if 3 * nz * nrhs > 1024:
+            continue
+        m, _, _, op = _op(oracle, (4, 5, nz), nrhs, precision, nz + nrhs)
+        xs = _x(m, nrhs, nz)
+        y = op.apply(xs)
+        kernel = op.contract_kernel(nrhs)
+        monkeypatch.setenv("XTR_CONTRACT_KERNEL", "generic")
+        g = op.apply(xs)
+        monkeypatch.delenv("XTR_CONTRACT_KERNEL")
+        e = max(rel(y[r], g[r]) for r in range(nrhs))
+        worst = max(worst, (e, kernel))
+        assert e < tol, (kernel, e)
+    print(f"nrhs {nrhs} {precision}: worst {worst[0]:.1e}, {worst[1]}", flush=True)
