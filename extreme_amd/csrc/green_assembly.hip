@@ -12,15 +12,17 @@
 //         [HankelCoefficients.cs:103-118, ScalarMathUtils.cs:189-241, InnerResultsCombiner.cs:19-62]
 //   K4    piecewise-linear segments I(rho) = A rho + B  [ScalarSegments.cs:86-128]
 //   K5    lateral integration of every cell of the positive quadrant by line integrals along
-//         its four edges, written straight into the device layout (a full tensor with its mirror
-//         images; a folded one gets them from the parities in the FFT's loads)
+//         its four edges (the knots of all cells' edges first, knots_kernel; then per cell the segments'
+//         weights, in LDS, and their sums with the pairs' coefficients), written straight into the
+//         device layout (a full tensor with its mirror images; a folded one gets them from the parities
+//         in the FFT's loads)
 //         [GreenTensorCalculator.cs:166-552, IntegralFactors.cs:17-30, QSign.cs:64-67,
 //          GreenTensorFftPopulator.cs:37-148]
 //   FFT   forward 2-D pencil FFT of every column  [AtoAGreenTensorCalculatorComponent.cs:197-279]
 //
-// Threads of K5 own one transceiver pair each and share the cell, so the edge geometry, the
-// knot search and the segment walk are uniform across a wavefront while the per-pair segment
-// coefficients are read coalesced.
+// A workgroup of K5 takes one cell: its threads form the weights of 32 segments at a time together, and each then
+// sums them for a transceiver pair of its own, whose segment coefficients are read coalesced. Where pairs are few,
+// groups of threads share a pair's segments.
 #include "xtr_common.h"
 #include "xtr_green.h"
 #include "xtr_kernels.h"
@@ -520,9 +522,9 @@ __global__ __launch_bounds__(256) void knots_kernel(const double *radii, int nr,
 // farther. What FillResultAlongX/Y (:413-437) multiply by the QSigns tables (QSign.cs:31-38, 64-67) is a sign of
 // the component and, for d3 only, the opposite sign on a stretch mirrored about the axis (rows AlongXSymm,
 // AlongYSymm); the latter is in the weights here, the former with the components' sums.
-// The weights are the same for every pair of layers, so a team of threads forms them once in LDS: knots by binary
-// search, then a logarithm and two square roots for each (segment, stretch), then the sums. Each coefficient is
-// then read once per cell and segment instead of once per edge and segment.
+// The weights are the same for every pair of layers, so a team of threads forms them once in LDS, from the knots
+// that knots_kernel found: a logarithm and two square roots for each (segment, stretch), then the sums. Each
+// coefficient is then read once per cell and segment instead of once per edge and segment.
 enum { W1A, W1B, W2A, W2B, W3A, W3B, WN };
 template <int SEGS>
 struct CellWeights {

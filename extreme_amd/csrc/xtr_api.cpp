@@ -87,8 +87,8 @@ struct DevBuf {
     DevBuf &operator=(const DevBuf &) = delete;
 };
 
-// Pinned host memory that kernels write directly (mapped into the device address space,
-// fine-grained coherent): small results the host reads after the stream has passed the writer.
+// Pinned host memory that kernels write directly (mapped into the device address space, fine-grained coherent):
+// small results that the host polls value by value (Polled) while the kernels that store them may still run.
 template <typename T>
 struct MappedBuf {
     T *p = nullptr;     // host address

@@ -1,4 +1,5 @@
-// Device helpers of the folded contractions (op_kernels.hip, contract_block.hip): waits on copies in
+// Device helpers of the folded contractions (op_kernels.hip, contract_block.h,
+// contract_direct.hip) and of the Hankel filter (green_assembly.hip): waits on copies in
 // flight, the 16x16x4 MFMAs and their lane layout, LDS reads by byte offset.
 #pragma once
 
